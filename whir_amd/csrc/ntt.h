@@ -32,6 +32,8 @@ struct RsArgs {
   const uint64_t* const* msg_tab = nullptr;
   uint64_t* const* out_tab = nullptr;
   uint64_t mpi = 1;
+  // First message of this call: message j of M is message j0 + j of the arrays above.
+  uint64_t j0 = 0;
 };
 
 // Powers of w_n, the order-n root of unity of the reference's NTT (n = 2^logn), as two

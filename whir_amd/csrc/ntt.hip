@@ -25,6 +25,7 @@
 #include "common.h"
 #include "gl.h"
 #include "ntt.h"
+#include "ntt_mx.h"
 
 #include <algorithm>
 #include <cstdio>
@@ -670,8 +671,10 @@ static int variant_bits(int D) { return (((ntt_variant().pad >> D) & 1) << 1) | 
 
 // One encode's schedule: the four-step split and, per pass, the in-LDS variant
 // (bit 1: padding, bit 0: radix 16) and the LDS tile size in u64 words (which sets
-// how many columns / rows / sequences a block transforms).
+// how many columns / rows / sequences a block transforms).  mx: the matrix-core kernels
+// of ntt_mx.hip instead, which have a schedule of their own.
 struct NttSched {
+  bool mx = false;
   int logC1 = 0;
   int v1 = 0, v2 = 0;
   int tw1 = 4096, tw2 = 4096;
@@ -685,6 +688,10 @@ static NttSched default_sched(int D, int logC) {
   // passes at 2^26 outputs on MI355X, as measured by the autotuner); pass 2 is not.
   if (D == 1 && !getenv("WHIR_NTT_VARIANT") && logC > MAX_PASS_LOG) s.v1 = 2;
   s.tw1 = s.tw2 = tile_words();
+  // The matrix-core kernels wherever they transform this size: no shape between one message
+  // of 2^8 Fp elements and 16 of 2^18 measured slower (1.0-1.9x faster, MI355X).
+  int c1 = 0;
+  s.mx = mx_split(D, logC, &c1);
   return s;
 }
 
@@ -770,6 +777,24 @@ static void pass2(RsArgs a, uint64_t* scratch, int logC1, int v, int tw, hipStre
   }
 }
 
+static MxTables mx_tables(int logN, int logC, int logC1, hipStream_t st) {
+  MxTables t;
+  if (logC1) {
+    t.row = shape_table(2, logN, logC, logC1, st);
+    t.post = shape_table(1, logN, logC, logC1, st);
+  } else {
+    t.pre = shape_table(0, logN, logC, 0, st);
+  }
+  return t;
+}
+
+template <int D>
+static void run_mx(const RsArgs& a, uint64_t* scratch, hipStream_t st) {
+  int logC1 = 0;
+  (void)mx_split(D, a.logC, &logC1);
+  mx_encode(D, a, mx_tables(log2_exact(a.N), a.logC, logC1, st), scratch, st);
+}
+
 // ------------------------------------------------------------------ autotuner
 // With tuning on (whir_ntt_autotune(1) or WHIR_NTT_AUTOTUNE=1), the first encode of
 // each shape (degree, log N, log C, messages) times every candidate schedule on the
@@ -845,9 +870,10 @@ static double time_on(hipStream_t st, F fn) {
 static constexpr double kTuneMargin = 0.97;
 
 template <int D>
-static SchedEntry tune(RsArgs a, uint64_t* scratch, hipStream_t st) {
+static SchedEntry tune_butterflies(RsArgs a, uint64_t* scratch, hipStream_t st) {
   const int logN = log2_exact(a.N), logC = a.logC;
-  const NttSched def = default_sched(D, logC);
+  NttSched def = default_sched(D, logC);
+  def.mx = false;
   const std::vector<int> tws = tile_candidates();
   SchedEntry best;
   best.s = def;
@@ -930,6 +956,10 @@ static SchedEntry tune(RsArgs a, uint64_t* scratch, hipStream_t st) {
 
 template <int D>
 static void run_sched(RsArgs a, uint64_t* scratch, const NttSched& s, hipStream_t st) {
+  if (s.mx) {
+    run_mx<D>(a, scratch, st);
+    return;
+  }
   if (a.logC <= MAX_PASS_LOG) {
     single<D>(a, s.v1, s.tw1, st);
     return;
@@ -939,6 +969,24 @@ static void run_sched(RsArgs a, uint64_t* scratch, const NttSched& s, hipStream_
   const uint64_t* post = shape_table(1, logN, a.logC, s.logC1, st);
   pass1<D, pass1_ept<D>()>(a, post, scratch, logN, s.logC1, s.v1, s.tw1, st);
   pass2<D>(a, scratch, s.logC1, s.v2, s.tw2, st);
+}
+
+// Sizes the matrix-core kernels take keep them unless a schedule of the butterfly kernels
+// is clearly faster.
+template <int D>
+static SchedEntry tune(RsArgs a, uint64_t* scratch, hipStream_t st) {
+  SchedEntry best = tune_butterflies<D>(a, scratch, st);
+  if (!default_sched(D, a.logC).mx) return best;
+  best.ms_default = time_on(st, [&] { run_mx<D>(a, scratch, st); });
+  best.candidates++;
+  if (best.ms1 + best.ms2 < kTuneMargin * best.ms_default) {
+    run_sched<D>(a, scratch, best.s, st);
+  } else {
+    best.s.mx = true;
+    best.ms1 = best.ms_default;
+    best.ms2 = 0;
+  }
+  return best;
 }
 
 // The schedule recorded for a shape, else the built-in one.
@@ -999,6 +1047,13 @@ void rs_prepare(int D, uint64_t N, int logC, uint64_t M, hipStream_t st) {
   const int logN = log2_exact(N);
   WHIR_REQUIRE(logN >= 0 && logC <= logN, "rs_prepare: bad shape");
   const NttSched s = sched_for(D, N, logC, M);
+  if (s.mx) {
+    int logC1 = 0;
+    (void)mx_split(D, logC, &logC1);
+    (void)mx_tables(logN, logC, logC1, st);
+    mx_prepare();
+    return;
+  }
   if (logC <= MAX_PASS_LOG) {
     (void)shape_table(0, logN, logC, 0, st);
     (void)flat_twiddles(logC);
@@ -1046,7 +1101,7 @@ void ntt_set_schedule(int D, int logN, int logC, uint64_t M, int logC1, int v1, 
     WHIR_REQUIRE(logC1 >= logC - MAX_PASS_LOG && logC1 <= MAX_PASS_LOG, "ntt schedule: split out of range");
   }
   SchedEntry e;
-  e.s = NttSched{logC1, v1, v2, tw1, tw2};
+  e.s = NttSched{false, logC1, v1, v2, tw1, tw2};
   std::lock_guard<std::mutex> g(g_sched_mu);
   g_sched[SchedKey{D, logN, logC, M}] = e;
 }
@@ -1068,9 +1123,9 @@ std::string ntt_schedules_json() {
              "%s{\"degree\":%d,\"log_n\":%d,\"log_c\":%d,\"messages\":%llu,\"log_c1\":%d,"
              "\"pass1\":{\"pad\":%d,\"radix16\":%d,\"tile_words\":%d},"
              "\"pass2\":{\"pad\":%d,\"radix16\":%d,\"tile_words\":%d},"
-             "\"tuned_ms\":%.4f,\"default_ms\":%.4f,\"candidates\":%d}",
+             "\"matrix_cores\":%s,\"tuned_ms\":%.4f,\"default_ms\":%.4f,\"candidates\":%d}",
              first ? "" : ",", k.D, k.logN, k.logC, (unsigned long long)k.M, e.s.logC1, (e.s.v1 >> 1) & 1, e.s.v1 & 1,
-             e.s.tw1, (e.s.v2 >> 1) & 1, e.s.v2 & 1, e.s.tw2, e.ms1 + e.ms2, e.ms_default, e.candidates);
+             e.s.tw1, (e.s.v2 >> 1) & 1, e.s.v2 & 1, e.s.tw2, e.s.mx ? "true" : "false", e.ms1 + e.ms2, e.ms_default, e.candidates);
     out += buf;
     first = false;
   }
