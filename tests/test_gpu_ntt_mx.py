@@ -1,6 +1,6 @@
 """The matrix-core Reed-Solomon kernels (whir_amd/csrc/ntt_mx.hip) against the oracle's
-encoder (cooley_tukey.rs:411-477 restated): every radix combination (one pass 2^8..2^10,
-two passes 2^16..2^20), each degree, cosets in full and ragged, masks, odd message counts
+encoder (cooley_tukey.rs:411-477 restated): every radix combination (one pass 2^4..2^10,
+a column step and rows 2^11..2^15, two passes 2^16..2^20), each degree, cosets in full and ragged, masks, odd message counts
 and the values at which a carry or a borrow is taken.  Exact arithmetic: no tolerance."""
 import numpy as np
 import pytest
@@ -17,6 +17,16 @@ EDGES = np.array([0, 1, P - 1, P - 2, 0xFFFFFFFF, 0x100000000, 0xFFFFFFFE0000000
 
 # D, messages, message length, codeword length, mask length
 CASES = [
+    (1, 1, 1 << 4, 1 << 4, 0), (1, 3, 1 << 4, 1 << 6, 0), (2, 5, 1 << 4, 1 << 9, 0), (3, 3, 1 << 4, 1 << 7, 0),
+    (1, 2, 1 << 5, 1 << 5, 0), (2, 3, 1 << 5, 1 << 8, 0), (3, 17, 1 << 5, 1 << 6, 0), (1, 3, 21, 1 << 7, 2),
+    (1, 1, 1 << 6, 1 << 6, 0), (1, 37, 1 << 6, 1 << 8, 0), (2, 3, 1 << 6, 1 << 10, 0), (3, 5, 1 << 6, 1 << 7, 0),
+    (1, 3, 1 << 7, 1 << 7, 0), (2, 33, 1 << 7, 1 << 8, 0), (3, 3, 1 << 7, 1 << 10, 0), (1, 600, 40, 1 << 6, 0),
+    (1, 3, 1 << 11, 1 << 11, 0), (2, 2, 1 << 11, 1 << 13, 0), (3, 3, 1 << 11, 1 << 12, 0), (2, 3, 1500, 1 << 11, 9),
+    (1, 1, 1 << 12, 1 << 12, 0), (2, 3, 1 << 12, 1 << 14, 0), (3, 2, 1 << 12, 1 << 13, 0), (1, 3, 4000, 1 << 13, 3),
+    (1, 5, 1 << 12, 1 << 20, 0), (2, 9, 1 << 12, 1 << 20, 0), (1, 33, 2500, 1 << 17, 1),
+    (1, 2, 1 << 13, 1 << 15, 0), (2, 2, 1 << 13, 1 << 13, 0), (3, 2, 1 << 13, 1 << 14, 0),
+    (1, 3, 1 << 14, 1 << 15, 0), (2, 1, 1 << 14, 1 << 16, 0), (3, 2, 10000, 1 << 14, 0),
+    (1, 1, 1 << 15, 1 << 16, 0), (2, 3, 1 << 15, 1 << 15, 0), (3, 1, 20000, 1 << 16, 10),
     (1, 1, 1 << 8, 1 << 8, 0), (1, 5, 1 << 8, 1 << 10, 0), (2, 3, 1 << 8, 1 << 11, 0), (3, 7, 1 << 8, 1 << 9, 0),
     (1, 3, 1 << 9, 1 << 10, 0), (2, 5, 1 << 9, 1 << 9, 0), (3, 3, 1 << 9, 1 << 12, 0),
     (1, 9, 1 << 10, 1 << 11, 0), (2, 3, 1 << 10, 1 << 12, 0), (3, 5, 1 << 10, 1 << 10, 0),

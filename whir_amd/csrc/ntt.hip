@@ -680,7 +680,7 @@ struct NttSched {
   int tw1 = 4096, tw2 = 4096;
 };
 
-static NttSched default_sched(int D, int logC) {
+static NttSched default_sched(int D, int logC, uint64_t words) {
   NttSched s;
   s.logC1 = logC <= MAX_PASS_LOG ? 0 : (logC + 1) / 2;
   s.v1 = s.v2 = variant_bits(D);
@@ -689,9 +689,12 @@ static NttSched default_sched(int D, int logC) {
   if (D == 1 && !getenv("WHIR_NTT_VARIANT") && logC > MAX_PASS_LOG) s.v1 = 2;
   s.tw1 = s.tw2 = tile_words();
   // The matrix-core kernels wherever they transform this size: no shape between one message
-  // of 2^8 Fp elements and 16 of 2^18 measured slower (1.0-1.9x faster, MI355X).
+  // of 2^4 Fp elements and 16 of 2^18 Fp3 ones measured slower (1.0-2.6x faster, MI355X),
+  // but for extension codewords of 2^22 words and more over 2^11 elements: there the one
+  // butterfly pass beats a column step and rows (Fp2 2^22 words 38.6 against 40.1 us, 2^24
+  // 118.8 against 132; at 2^19 15.8 against 12.0).
   int c1 = 0;
-  s.mx = mx_split(D, logC, &c1);
+  s.mx = mx_split(logC, &c1) && !(logC == 11 && D > 1 && words >= (1ull << 22));
   return s;
 }
 
@@ -791,7 +794,7 @@ static MxTables mx_tables(int logN, int logC, int logC1, hipStream_t st) {
 template <int D>
 static void run_mx(const RsArgs& a, uint64_t* scratch, hipStream_t st) {
   int logC1 = 0;
-  (void)mx_split(D, a.logC, &logC1);
+  (void)mx_split(a.logC, &logC1);
   mx_encode(D, a, mx_tables(log2_exact(a.N), a.logC, logC1, st), scratch, st);
 }
 
@@ -872,7 +875,7 @@ static constexpr double kTuneMargin = 0.97;
 template <int D>
 static SchedEntry tune_butterflies(RsArgs a, uint64_t* scratch, hipStream_t st) {
   const int logN = log2_exact(a.N), logC = a.logC;
-  NttSched def = default_sched(D, logC);
+  NttSched def = default_sched(D, logC, a.M * a.N * D);
   def.mx = false;
   const std::vector<int> tws = tile_candidates();
   SchedEntry best;
@@ -976,7 +979,7 @@ static void run_sched(RsArgs a, uint64_t* scratch, const NttSched& s, hipStream_
 template <int D>
 static SchedEntry tune(RsArgs a, uint64_t* scratch, hipStream_t st) {
   SchedEntry best = tune_butterflies<D>(a, scratch, st);
-  if (!default_sched(D, a.logC).mx) return best;
+  if (!default_sched(D, a.logC, a.M * a.N * D).mx) return best;
   best.ms_default = time_on(st, [&] { run_mx<D>(a, scratch, st); });
   best.candidates++;
   if (best.ms1 + best.ms2 < kTuneMargin * best.ms_default) {
@@ -995,7 +998,7 @@ static NttSched sched_for(int D, uint64_t N, int logC, uint64_t M, bool* found =
   std::lock_guard<std::mutex> g(g_sched_mu);
   auto it = g_sched.find(key);
   if (found) *found = it != g_sched.end();
-  return it != g_sched.end() ? it->second.s : default_sched(D, logC);
+  return it != g_sched.end() ? it->second.s : default_sched(D, logC, M * N * D);
 }
 
 // Messages of one coefficient and no mask: the polynomial is a constant, so every
@@ -1032,7 +1035,7 @@ static void launch(RsArgs a, uint64_t* scratch, hipStream_t st) {
     return;
   }
   if (!autotune_on()) {
-    run_sched<D>(a, scratch, default_sched(D, a.logC), st);
+    run_sched<D>(a, scratch, s, st);
     return;
   }
   SchedEntry e = tune<D>(a, scratch, st);  // also leaves the output behind
@@ -1049,7 +1052,7 @@ void rs_prepare(int D, uint64_t N, int logC, uint64_t M, hipStream_t st) {
   const NttSched s = sched_for(D, N, logC, M);
   if (s.mx) {
     int logC1 = 0;
-    (void)mx_split(D, logC, &logC1);
+    (void)mx_split(logC, &logC1);
     (void)mx_tables(logN, logC, logC1, st);
     mx_prepare();
     return;
@@ -1067,7 +1070,8 @@ void rs_prepare(int D, uint64_t N, int logC, uint64_t M, hipStream_t st) {
 
 size_t rs_scratch_words(int D, uint64_t M, uint64_t N, uint64_t C) {
   int logC = log2_exact(C);
-  return logC > MAX_PASS_LOG ? (size_t)M * N * D : 0;
+  // a matrix-core encode of 2^11 elements is a column step and rows, too
+  return logC >= MAX_PASS_LOG ? (size_t)M * N * D : 0;
 }
 
 void rs_encode_cols(int D, RsArgs a, uint64_t* scratch, hipStream_t st) {

@@ -19,7 +19,7 @@ struct MxTables {
 
 // Whether the matrix-core kernels transform cosets of 2^logC elements, and how: the
 // four-step split's log C1 (0: one pass).
-bool mx_split(int D, int logC, int* logC1);
+bool mx_split(int logC, int* logC1);
 void mx_prepare();  // builds the constant tables (not during a stream capture)
 void mx_encode(int D, const RsArgs& a, const MxTables& t, uint64_t* scratch, hipStream_t st);
 

@@ -1,8 +1,8 @@
 // Reed-Solomon expansion on the matrix cores (CDNA4 int8 MFMA).
 //
-// The transforms of ntt.hip again (same layout, same values), for cosets of 2^8 .. 2^10
-// (one pass) and 2^16 .. 2^20 elements (two passes), with the DFTs as integer matrix
-// products.  A Goldilocks element is eight signed base-256 digits, x = sum_b s_b 2^(8b),
+// The transforms of ntt.hip again (same layout, same values), for cosets of 2^4 .. 2^10
+// elements (one pass) and 2^11 .. 2^20 (two passes, 2^12 also one), with the DFTs as integer
+// matrix products.  A Goldilocks element is eight signed base-256 digits, x = sum_b s_b 2^(8b),
 // -128 <= s_b < 128, and multiplying by a constant w is linear in the digits:
 //     w x = sum_b s_b (w 2^(8b) mod p),
 // with the constants' own eight digits as the rows of an int8 matrix.  A whole small DFT
@@ -24,7 +24,9 @@
 // a 2^10-point one.  Measured on MI355X, 16 messages, two passes, before -> after:
 //     Fp  2^20 -> 2^22: 603 + 432 -> 351 + 314 us    Fp  2^18 -> 2^22: 548 + 366 -> 295 + 254 us
 //     Fp2 2^16 -> 2^21: 393 + 289 -> 280 + 247 us    Fp3 2^18 -> 2^21: 834 + 619 -> 470 + 505 us
+//     Fp2 2^12 -> 2^20: 284 -> 204 us                Fp3 2^14 -> 2^17: 79 -> 59 us
 //     one pass, Fp2 2^8 -> 2^19: 98 -> 62 us         Fp3 2^10 -> 2^19: 264 -> 112 us
+//     small, Fp 2^10 -> 2^11: 15.5 -> 7.3 us         Fp2 2^12 -> 2^13: 21.2 -> 12.8 us
 // Pass 2 of 2^8 and 2^9 points moves 1.07 GB in 240-250 us, 4.4 TB/s where a large copy
 // reaches 4.7: it is at the memory's rate.  Pass 1 and the 2^10-point pass 2 are bound by
 // VALU issue with four waves per SIMD; 128 registers a lane, 64 of them the matrix, allow
@@ -153,7 +155,7 @@ DEV uint64_t recombine(v4i L, v4i H, const Opaque& k) {
   return fix_carry((uint32_t)T, hi, c);
 }
 
-// A radix-R step (R = 16, 32) of 16 columns by one wave.  Lane (n, g), n = lane % 16 and
+// A radix-R step (R = 8, 16, 32) of 16 columns by one wave.  Lane (n, g), n = lane % 16 and
 // g = lane / 16, loads R/4 elements of column n, element i of index g + in_u(i), and ends
 // with R/4 outputs, output i of index out_g g + out_u(i).
 //   FULL (R = 16): the 16-point transform is one product with the 128 x 128 digit matrix;
@@ -164,11 +166,11 @@ DEV uint64_t recombine(v4i L, v4i H, const Opaque& k) {
 template <int LR, bool FULL>
 struct Step {
   static constexpr int N = 1 << (LR - 2);
-  static constexpr int out_g = FULL ? 1 : LR == 4 ? 2 : 4;
-  static DEV constexpr int in_u(int i) { return FULL ? 4 * i : 4 * (i & 1) + (i >> 1) * 8; }
+  static constexpr int out_g = FULL || LR == 3 ? 1 : LR == 4 ? 2 : 4;
+  static DEV constexpr int in_u(int i) { return FULL || LR == 3 ? 4 * i : 4 * (i & 1) + (i >> 1) * 8; }
   // which of its elements index j is, for the lane group j % 4 that loads it
   static DEV constexpr int in_i(int j) { return FULL ? j >> 2 : (j >> 2 & 1) + (j >> 3) * 2; }
-  static DEV constexpr int out_u(int i) { return FULL ? 4 * i : LR == 4 ? 8 * (i >> 1) + (i & 1) : 16 * (i >> 2) + (i & 3); }
+  static DEV constexpr int out_u(int i) { return FULL || LR == 3 ? 4 * i : LR == 4 ? 8 * (i >> 1) + (i & 1) : 16 * (i >> 2) + (i & 3); }
 };
 
 struct Mats {
@@ -215,6 +217,8 @@ DEV void dft(const Mats& A, const uint64_t (&x)[1 << (LR - 2)], F emit) {
       emit(u, recombine(L0, H0, A.k));
       emit(u + 1, recombine(L1, H1, A.k));
     }
+  } else if constexpr (LR == 3) {
+    dft8(A, 0, biased(x[0]), biased(x[1]), 0, 1, emit);
   } else if constexpr (LR == 4) {
     const uint64_t b0 = biased(x[0]), b1 = biased(x[1]);
     dft8(A, 0, addl(b0, x[2]), addl(b1, x[3]), 0, 2, emit);
@@ -276,6 +280,10 @@ constexpr int row_threads() { return D == 3 && LA == 5 ? 768 : 512; }
 // Rows of length S that a block of pass 2 transforms.
 template <int D>
 constexpr int row_block(int S) { return (D == 1 ? 8 : D == 2 ? 4 : 2) * (1024 / S); }
+
+// Most sequences of length S that a block of the single pass transforms.
+template <int D>
+constexpr int sequences(int S) { return row_block<D>(S); }
 
 // ------------------------------------------------------------------ pass 1: columns
 template <int D, int LA, int LB, bool NEXT16>
@@ -361,11 +369,11 @@ __global__ __launch_bounds__(512, 4) void k_mx_pass1(RsArgs a, const v4i* mat, c
 }
 
 // ------------------------------------------------------------------ pass 2: rows
-template <int D, int LA, int LB>
+template <int D, int LA, int LB, int B>
 __global__ __launch_bounds__((row_threads<D, LA>()), 4) void k_mx_pass2(RsArgs a, const v4i* mat, const uint64_t* tw, const uint64_t* Y,
                                                         int logC1) {
   constexpr int TH = row_threads<D, LA>(), RA = 1 << LA, RB = 1 << LB, S = RA * RB;
-  constexpr int B = row_block<D>(S), BY = B < 16 ? B : 16, BD = B * D;
+  constexpr int BY = B < 16 ? B : 16, BD = B * D;
   constexpr bool F16 = LA == 4 && LB == 4;
   using SA = Step<LA, F16>;
   using SB = Step<LB, F16>;
@@ -418,59 +426,222 @@ __global__ __launch_bounds__((row_threads<D, LA>()), 4) void k_mx_pass2(RsArgs a
 
 // ------------------------------------------------------------------ single pass
 template <int D, int LA, int LB>
-__global__ __launch_bounds__(512, 4) void k_mx_single(RsArgs a, const v4i* mat, const uint64_t* tw, const uint64_t* pre) {
+__global__ __launch_bounds__(512, 4) void k_mx_single(RsArgs a, const v4i* mat, const uint64_t* tw, const uint64_t* pre,
+                                                    int G) {
   constexpr int TH = 512, RA = 1 << LA, RB = 1 << LB, S = RA * RB;
-  constexpr int G = (D == 1 ? 8 : D == 2 ? 4 : 2) * (1024 / S);
   constexpr bool F16 = LA == 4 && LB == 4;
   using SA = Step<LA, F16>;
   using SB = Step<LB, F16>;
   constexpr int NA = RA / 4, NB = RB / 4, KS = RB * D + D;
-  __shared__ uint64_t s[G * RA * KS];
+  __shared__ uint64_t s[sequences<D>(S) * RA * KS];
   __shared__ uint64_t t1[S];
   const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const size_t nseq = (size_t)a.M * a.Q;
+  const uint32_t nseq = (uint32_t)(a.M * a.Q), Q = (uint32_t)a.Q;
+  const int logQ = __builtin_ctz(Q);  // a power of two, as the codeword and coset lengths are
   for (int k = threadIdx.x; k < S; k += TH) t1[k] = tw[k];
   Mats A;
   load_mats(A, mat + (F16 ? MAT16 : 0));
   const size_t Lw = a.L * D, mw = a.mask_len * D;
   __syncthreads();
-  for (size_t seq0 = (size_t)blockIdx.x * G; seq0 < nseq; seq0 += (size_t)gridDim.x * G) {
+  for (uint32_t seq0 = blockIdx.x * G; seq0 < nseq; seq0 += gridDim.x * G) {
 #pragma unroll 1
     for (int t = wave; t < G * RB * D / 16; t += TH / 64) {
-      const uint32_t sq = t / (RB * D / 16), wl = (t % (RB * D / 16)) * 16 + n, lo = wl / D;
-      const size_t seq = seq0 + sq;
-      if (seq >= nseq) break;  // uniform: later sequences are past the end too
-      const size_t j = seq / a.Q, c = seq % a.Q;
+      // group: 16 words (lo, d), of one sequence unless a sequence has fewer or 24 of them
+      constexpr bool ONE = RB * D % 16 == 0;
+      const uint32_t q = t * 16 + n, sq = ONE ? t / (RB * D / 16) : q / (RB * D), wl = q - sq * (RB * D), lo = wl / D;
+      if (seq0 + (t * 16) / (RB * D) >= nseq) break;  // uniform: later sequences are past the end too
+      const uint32_t seq = min(seq0 + sq, nseq - 1), j = seq >> logQ, c = seq & (Q - 1);
       const uint64_t* msg = msg_ptr<D>(a, j);
       const uint64_t* mask = a.masks ? a.masks + (a.j0 + j) * mw : nullptr;
-      uint64_t x[NA];
+      uint64_t x[NA], p[NA];
 #pragma unroll
-      for (int i = 0; i < NA; i++) x[i] = word_at<D>(msg, Lw, mask, mw, (SA::in_u(i) + g) * (RB * D) + wl);
+      for (int e = 0; e < NA; e++) {
+        x[e] = word_at<D>(msg, Lw, mask, mw, (SA::in_u(e) + g) * (RB * D) + wl);
+        p[e] = ld(pre + (size_t)c * S + SA::in_u(e) * RB, (g * RB + lo) * 8);
+      }
 #pragma unroll
-      for (int i = 0; i < NA; i++)
-        x[i] = mulw<F16>(x[i], ld(pre + c * S + SA::in_u(i) * RB, (g * RB + lo) * 8), A.k);
+      for (int e = 0; e < NA; e++) x[e] = mulw<F16>(x[e], p[e], A.k);
       SCHED_FENCE();
       const uint64_t* w = t1 + lo * RA + SA::out_g * g;
       uint64_t* d = s + (sq * RA + SA::out_g * g) * KS + wl;
-      dft<LA, F16>(A, x, [&](int i, uint64_t o) { d[SA::out_u(i) * KS] = mulw<F16>(o, w[SA::out_u(i)], A.k); });
+      dft<LA, F16>(A, x, [&](int e, uint64_t o) { d[SA::out_u(e) * KS] = mulw<F16>(o, w[SA::out_u(e)], A.k); });
     }
     __syncthreads();
 #pragma unroll 1
     for (int t = wave; t < G * RA * D / 16; t += TH / 64) {
-      const uint32_t sq = t / (RA * D / 16), kw = (t % (RA * D / 16)) * 16 + n, k1 = kw / D;
-      const size_t seq = seq0 + sq;
-      if (seq >= nseq) break;
-      const size_t j = seq / a.Q, c = seq % a.Q;
+      constexpr bool ONE = RA * D % 16 == 0;
+      const uint32_t q = t * 16 + n, sq = ONE ? t / (RA * D / 16) : q / (RA * D), kw = q - sq * (RA * D), k1 = kw / D;
+      if (seq0 + (t * 16) / (RA * D) >= nseq) break;
+      const uint32_t seq = min(seq0 + sq, nseq - 1), j = seq >> logQ, c = seq & (Q - 1);
       uint64_t x[NB];
       const uint64_t* src = s + (sq * RA + k1) * KS + g * D + kw % D;
 #pragma unroll
-      for (int i = 0; i < NB; i++) x[i] = src[SB::in_u(i) * D];
-      uint64_t* out = out_ptr<D>(a, j) + c * S * D;
+      for (int e = 0; e < NB; e++) x[e] = src[SB::in_u(e) * D];
+      uint64_t* out = out_ptr<D>(a, j) + (size_t)c * S * D;
       const uint32_t vo = (RA * D * SB::out_g * g + kw) * 8;
-      dft<LB, F16>(A, x, [&](int i, uint64_t o) { st(out + RA * D * SB::out_u(i), vo, canon(o)); });
+      dft<LB, F16>(A, x, [&](int e, uint64_t o) {
+        if (ONE || seq0 + sq < nseq) st(out + RA * D * SB::out_u(e), vo, canon(o));
+      });
     }
     __syncthreads();
+  }
+}
+
+// ------------------------------------------------------------------ pass 1 of one step
+// Columns of C2 = 8, 16 or 32 elements: a wave takes 16 word columns of one (message, coset)
+// straight from memory to memory, no LDS and no barrier.
+template <int D, int LA, bool NEXT16>
+__global__ __launch_bounds__(512, 4) void k_mx_column(RsArgs a, const v4i* mat, const uint64_t* row, const uint64_t* post,
+                                                     uint64_t* Y, int logC1, int logBY) {
+  constexpr int RA = 1 << LA, NA = RA / 4;
+  constexpr bool F16 = LA == 4;
+  using SA = Step<LA, F16>;
+  const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t C1w = (uint32_t)D << logC1, ntile = C1w / 16, nwt = C1w / 8;
+  const size_t C = (size_t)1 << a.logC;
+  const size_t Lw = a.L * D, mw = a.mask_len * D;
+  const bool full = a.L == C;
+  Mats A;
+  load_mats(A, mat + (F16 ? MAT16 : 0));
+  // column groups: tiles fastest, then cosets (the same message words), then messages
+  const uint32_t units = ntile * (uint32_t)a.Q * (uint32_t)a.M;
+  const uint32_t per = (units + 7) / 8, u1 = min(units, (blockIdx.x % 8 + 1) * per);
+  for (uint32_t u = (blockIdx.x % 8) * per + (blockIdx.x / 8) * 8 + wave; u < u1; u += gridDim.x) {
+    const uint32_t wc = (u % ntile) * 16 + n, jc = u / ntile;
+    const uint32_t c = jc % (uint32_t)a.Q, j = jc / (uint32_t)a.Q;
+    const uint64_t* msg = msg_ptr<D>(a, j);
+    const uint64_t* mask = a.masks ? a.masks + (a.j0 + j) * mw : nullptr;
+    const uint32_t i1 = wc / D, t2 = SA::out_g * g;
+    const uint32_t v0 = (g * C1w + wc) * 8, vp = ((t2 << logC1) + i1) * 8;
+    uint64_t x[NA], r[NA], w[NA];
+#pragma unroll
+    for (int e = 0; e < NA; e++) {
+      x[e] = full ? ld(msg + (size_t)SA::in_u(e) * C1w, v0)
+                  : word_at<D>(msg, Lw, mask, mw, (size_t)SA::in_u(e) * C1w + (v0 >> 3));
+      r[e] = ld(row + (size_t)c * RA + SA::in_u(e), g * 8);
+      w[e] = ld(post + c * C + ((size_t)SA::out_u(e) << logC1), vp);
+    }
+    if (c) {
+#pragma unroll
+      for (int e = 0; e < NA; e++) x[e] = mulw<F16>(x[e], r[e], A.k);
+    } else if constexpr (F16) {
+#pragma unroll
+      for (int e = 0; e < NA; e++) x[e] = biased(x[e]);
+    }
+    uint64_t* yj = Y + ((size_t)j * a.N + c * C) * D;
+    dft<LA, F16>(A, x, [&](int e, uint64_t o) {
+      const uint32_t t = t2 + SA::out_u(e);
+      const uint32_t vy = (((((t >> logBY) * nwt + (wc >> 3)) << logBY) + (t & ((1u << logBY) - 1))) * 8 + (wc & 7)) * 8;
+      st(yj, vy, mulw<NEXT16>(o, w[e], A.k));
+    });
+  }
+}
+
+// ------------------------------------------------------------------ single pass, three steps
+// C = 2^12 = 16 * 16 * 16, each step in place in LDS.  The first step's output factor
+// w_N^(lo (c + Q k1)) is the four-step post factor of the split 16 * 256.
+template <int D>
+__global__ __launch_bounds__(512, 4) void k_mx_cube(RsArgs a, const v4i* mat, const uint64_t* tw256, const uint64_t* row,
+                                                   const uint64_t* post) {
+  constexpr int S = 4096, G = D == 1 ? 2 : 1, KS = 256 * D + D;
+  using SA = Step<4, true>;
+  __shared__ uint64_t s[G * 16 * KS];
+  __shared__ uint64_t t2[256];
+  const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t nseq = (uint32_t)(a.M * a.Q), Q = (uint32_t)a.Q;
+  const int logQ = __builtin_ctz(Q);
+  const size_t Lw = a.L * D, mw = a.mask_len * D;
+  Mats A;
+  load_mats(A, mat + MAT16);
+  if (threadIdx.x < 256) t2[threadIdx.x] = tw256[threadIdx.x];
+  __syncthreads();
+  for (uint32_t seq0 = blockIdx.x * G; seq0 < nseq; seq0 += gridDim.x * G) {
+#pragma unroll 1
+    for (int t = wave; t < G * 16 * D; t += 8) {
+      const uint32_t sq = t / (16 * D), wl = (t % (16 * D)) * 16 + n, lo = wl / D;
+      const uint32_t seq = seq0 + sq;
+      if (seq >= nseq) break;  // uniform: later sequences are past the end too
+      const uint32_t j = seq >> logQ, c = seq & (Q - 1);
+      const uint64_t* msg = msg_ptr<D>(a, j);
+      const uint64_t* mask = a.masks ? a.masks + (a.j0 + j) * mw : nullptr;
+      uint64_t x[4], r[4], w[4];
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        x[e] = word_at<D>(msg, Lw, mask, mw, (SA::in_u(e) + g) * (256 * D) + wl);
+        r[e] = ld(row + (size_t)c * 16 + SA::in_u(e), g * 8);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; e++) w[e] = ld(post + (size_t)c * S + SA::out_u(e) * 256, (g * 256 + lo) * 8);
+#pragma unroll
+      for (int e = 0; e < 4; e++) x[e] = mulw<true>(x[e], r[e], A.k);
+      SCHED_FENCE();
+      uint64_t* d = s + (sq * 16 + g) * KS + wl;
+      dft<4, true>(A, x, [&](int e, uint64_t o) { d[SA::out_u(e) * KS] = mulw<true>(o, w[e], A.k); });
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (int t = wave; t < G * 16 * D; t += 8) {  // group: 16 words (lo2, d) of one k1
+      const uint32_t kq = t / D, wl = (t % D) * 16 + n, lo2 = wl / D;
+      uint64_t* p = s + kq * KS + wl + g * (16 * D);
+      uint64_t x[4];
+#pragma unroll
+      for (int e = 0; e < 4; e++) x[e] = p[SA::in_u(e) * 16 * D];
+      const uint64_t* w = t2 + lo2 * 16 + g;
+      dft<4, true>(A, x, [&](int e, uint64_t o) { p[SA::out_u(e) * 16 * D] = mulw<true>(o, w[SA::out_u(e)], A.k); });
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (int t = wave; t < G * 16 * D; t += 8) {  // group: 16 words (k1, d) of one k2
+      const uint32_t sq = t / (16 * D), r = t % (16 * D), k2 = r / D, kw = (r % D) * 16 + n, k1 = kw / D, d = kw % D;
+      const uint32_t seq = seq0 + sq;
+      if (seq >= nseq) break;
+      const uint32_t j = seq >> logQ, c = seq & (Q - 1);
+      uint64_t x[4];
+      const uint64_t* p = s + (sq * 16 + k1) * KS + (k2 * 16 + g) * D + d;
+#pragma unroll
+      for (int e = 0; e < 4; e++) x[e] = p[SA::in_u(e) * D];
+      uint64_t* out = out_ptr<D>(a, j) + ((size_t)c * S + k2 * 16) * D;
+      const uint32_t vo = (256 * D * g + kw) * 8;
+      dft<4, true>(A, x, [&](int e, uint64_t o) { st(out + 256 * D * SA::out_u(e), vo, canon(o)); });
+    }
+    __syncthreads();
+  }
+}
+
+// ------------------------------------------------------------------ single pass, one step
+// C = 16 or 32: 16 columns of a wave are 16 (coset, d) words of one message, which all read
+// the same coefficients.
+template <int D, int LA>
+__global__ __launch_bounds__(512, 4) void k_mx_short(RsArgs a, const v4i* mat, const uint64_t* pre) {
+  constexpr int RA = 1 << LA, NA = RA / 4;
+  constexpr bool F16 = LA == 4;
+  using SA = Step<LA, F16>;
+  const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const size_t Lw = a.L * D, mw = a.mask_len * D;
+  Mats A;
+  load_mats(A, mat + (F16 ? MAT16 : 0));
+  const uint64_t words = a.Q * D, groups = (words + 15) / 16, units = groups * a.M;
+  for (uint64_t u = (uint64_t)blockIdx.x * 8 + wave; u < units; u += (uint64_t)gridDim.x * 8) {
+    const uint64_t j = u / groups, cw = (u % groups) * 16 + n, c = min(cw, words - 1) / D;
+    const uint32_t d = (uint32_t)(min(cw, words - 1) % D);
+    const uint64_t* msg = msg_ptr<D>(a, j);
+    const uint64_t* mask = a.masks ? a.masks + (a.j0 + j) * mw : nullptr;
+    uint64_t x[NA], p[NA];
+#pragma unroll
+    for (int e = 0; e < NA; e++) {
+      x[e] = word_at<D>(msg, Lw, mask, mw, (SA::in_u(e) + g) * D + d);
+      p[e] = pre[c * RA + SA::in_u(e) + g];
+    }
+#pragma unroll
+    for (int e = 0; e < NA; e++) x[e] = mulw<F16>(x[e], p[e], A.k);
+    uint64_t* o = out_ptr<D>(a, j) + (c * RA + SA::out_g * g) * D + d;
+    dft<LA, F16>(A, x, [&](int e, uint64_t v) {
+      if (cw < words) o[SA::out_u(e) * D] = canon(v);
+    });
   }
 }
 
@@ -482,6 +653,9 @@ struct Consts {
 };
 std::mutex g_mu;
 std::map<int, Consts> g_consts;
+
+// log2 of the first radix of a two-step transform of 2^s points: 8*8, 16*8, 16*16, 32*16, 32*32
+constexpr int first_step(int s) { return s == 6 ? 3 : s <= 8 ? 4 : 5; }
 
 // Signed digits of v mod p in base 256.
 void digits(uint64_t v, int8_t out[8]) {
@@ -532,8 +706,8 @@ Consts build_consts() {
   WHIR_HIP(hipMalloc(&p, m.size()));
   WHIR_HIP(hipMemcpy(p, m.data(), m.size(), hipMemcpyHostToDevice));
   c.mat = (const v4i*)p;
-  for (int s = 8; s <= 10; s++) {
-    const int LA = s == 8 ? 4 : 5, RA = 1 << LA, RB = 1 << (s - LA);
+  for (int s = 6; s <= 10; s++) {
+    const int LA = first_step(s), RA = 1 << LA, RB = 1 << (s - LA);
     std::vector<uint64_t> t((size_t)1 << s);
     const uint64_t w = gl::root_of_unity(1ull << s);
     for (int lo = 0; lo < RB; lo++)
@@ -567,34 +741,76 @@ unsigned resident(const Consts& k, uint64_t nlogical) {
   return (unsigned)std::min<uint64_t>((nlogical + 7) / 8 * 8, std::max(8, k.cus * 2 / 8 * 8));
 }
 
+// log2 of the rows that lie together in pass 1's output, for rows of 2^logC1 in cosets of 2^logC.
+template <int D>
+int log_by(int logC1, int logC) {
+  int by = 0;
+  while ((2 << by) <= std::min({16, row_block<D>(1 << logC1), 1 << (logC - logC1)})) by++;
+  return by;
+}
+
 template <int D, int LA, int LB>
 void pass1(const RsArgs& a, const Consts& k, const MxTables& t, uint64_t* scratch, int logC1, hipStream_t st) {
   constexpr int S = 1 << (LA + LB), WB = TILE / S;
   const uint64_t base = ((uint64_t)D << logC1) / WB * a.Q;
   int jn = 1;
   while (jn * 2 <= (int)a.M && base * ((a.M + jn * 2 - 1) / (jn * 2)) >= 512) jn *= 2;
-  int by = 0;
-  while ((2 << by) <= std::min(16, row_block<D>(1 << logC1))) by++;
   ProfScope prof(kernel_name("k_mx_pass1", D, LA + LB), st, 8.0 * D * ((double)a.M * a.L + (double)a.M * a.N));
   auto kernel = logC1 == 8 ? k_mx_pass1<D, LA, LB, true> : k_mx_pass1<D, LA, LB, false>;
   kernel<<<xcd_grid(base * ((a.M + jn - 1) / jn)), 512, 0, st>>>(a, k.mat, k.tw[LA + LB], t.row, t.post, scratch, logC1,
-                                                                     by, jn);
+                                                                     log_by<D>(logC1, a.logC), jn);
   WHIR_HIP(hipGetLastError());
 }
 template <int D, int LA, int LB>
 void pass2(const RsArgs& a, const Consts& k, const uint64_t* scratch, int logC1, hipStream_t st) {
-  constexpr int S = 1 << (LA + LB), B = (D == 1 ? 8 : D == 2 ? 4 : 2) * (1024 / S);
+  constexpr int B = row_block<D>(1 << (LA + LB));
   const uint64_t C2 = 1ull << (a.logC - logC1);
   ProfScope prof(kernel_name("k_mx_pass2", D, LA + LB), st, 16.0 * D * (double)a.M * a.N);
-  k_mx_pass2<D, LA, LB><<<resident(k, C2 / B * a.Q * a.M), row_threads<D, LA>(), 0, st>>>(a, k.mat, k.tw[LA + LB], scratch, logC1);
+  const auto launch = [&](auto kernel, int rows) {
+    kernel<<<resident(k, C2 / rows * a.Q * a.M), row_threads<D, LA>(), 0, st>>>(a, k.mat, k.tw[LA + LB], scratch, logC1);
+  };
+  // the column steps of 2^11 and 2^12 elements leave 8 and 16 rows
+  constexpr int B16 = std::min(B, 16), B8 = std::min(B, 8);
+  if (C2 >= B) launch(k_mx_pass2<D, LA, LB, B>, B);
+  else if (C2 == 16) launch(k_mx_pass2<D, LA, LB, B16>, B16);
+  else launch(k_mx_pass2<D, LA, LB, B8>, B8);
   WHIR_HIP(hipGetLastError());
 }
 template <int D, int LA, int LB>
 void single(const RsArgs& a, const Consts& k, const MxTables& t, hipStream_t st) {
-  constexpr int S = 1 << (LA + LB), G = (D == 1 ? 8 : D == 2 ? 4 : 2) * (1024 / S);
+  constexpr int S = 1 << (LA + LB);
   const uint64_t nseq = a.M * a.Q;
+  WHIR_REQUIRE(nseq < (1ull << 30), "interleaved_encode: too many cosets");
+  // Small encodes spread over the CUs instead of filling their tiles (an even count, so that
+  // groups of 16 words end with a sequence's words): 16 messages 2^10 -> 2^11 13.2 -> 7.3 us.
+  int G = sequences<D>(S);
+  while (G > 2 && nseq <= (uint64_t)k.cus * (G / 2)) G /= 2;
   ProfScope prof(kernel_name("k_mx_single", D, LA + LB), st, 8.0 * D * ((double)a.M * a.L + (double)a.M * a.N));
-  k_mx_single<D, LA, LB><<<resident(k, (nseq + G - 1) / G), 512, 0, st>>>(a, k.mat, k.tw[LA + LB], t.pre);
+  k_mx_single<D, LA, LB><<<resident(k, (nseq + G - 1) / G), 512, 0, st>>>(a, k.mat, k.tw[LA + LB], t.pre, G);
+  WHIR_HIP(hipGetLastError());
+}
+
+template <int D, int LA>
+void column(const RsArgs& a, const Consts& k, const MxTables& t, uint64_t* scratch, int logC1, hipStream_t st) {
+  const uint64_t units = ((uint64_t)D << logC1) / 16 * a.Q * a.M;
+  WHIR_REQUIRE(units < (1ull << 31), "interleaved_encode: too many column groups");
+  ProfScope prof(kernel_name("k_mx_column", D, LA), st, 8.0 * D * ((double)a.M * a.L + (double)a.M * a.N));
+  auto kernel = logC1 == 8 ? k_mx_column<D, LA, true> : k_mx_column<D, LA, false>;
+  kernel<<<resident(k, (units + 7) / 8), 512, 0, st>>>(a, k.mat, t.row, t.post, scratch, logC1, log_by<D>(logC1, a.logC));
+  WHIR_HIP(hipGetLastError());
+}
+template <int D>
+void cube(const RsArgs& a, const Consts& k, const MxTables& t, hipStream_t st) {
+  WHIR_REQUIRE(a.M * a.Q < (1ull << 30), "interleaved_encode: too many cosets");
+  ProfScope prof(kernel_name("k_mx_cube", D), st, 8.0 * D * ((double)a.M * a.L + (double)a.M * a.N));
+  k_mx_cube<D><<<resident(k, (a.M * a.Q + (D == 1)) / (D == 1 ? 2 : 1)), 512, 0, st>>>(a, k.mat, k.tw[8], t.row, t.post);
+  WHIR_HIP(hipGetLastError());
+}
+template <int D, int LA>
+void shortest(const RsArgs& a, const Consts& k, const MxTables& t, hipStream_t st) {
+  const uint64_t units = (a.Q * D + 15) / 16 * a.M;
+  ProfScope prof(kernel_name("k_mx_short", D, LA), st, 8.0 * D * ((double)a.M * a.L + (double)a.M * a.N));
+  k_mx_short<D, LA><<<resident(k, (units + 7) / 8), 512, 0, st>>>(a, k.mat, t.pre);
   WHIR_HIP(hipGetLastError());
 }
 
@@ -602,13 +818,22 @@ template <int D>
 void encode(const RsArgs& a, const MxTables& t, uint64_t* scratch, hipStream_t st) {
   const Consts& k = consts();
   int logC1 = 0;
-  WHIR_REQUIRE(mx_split(D, a.logC, &logC1), "interleaved_encode: no matrix-core transform of this size");
-  if (!logC1) {
-    switch (a.logC) {
-      case 8: return single<D, 4, 4>(a, k, t, st);
-      case 9: return single<D, 5, 4>(a, k, t, st);
-      default: return single<D, 5, 5>(a, k, t, st);
-    }
+  WHIR_REQUIRE(mx_split(a.logC, &logC1), "interleaved_encode: no matrix-core transform of this size");
+  switch (logC1 ? 0 : a.logC) {
+    case 0: break;
+    case 4: return shortest<D, 4>(a, k, t, st);
+    case 5: return shortest<D, 5>(a, k, t, st);
+    case 6: return single<D, 3, 3>(a, k, t, st);
+    case 7: return single<D, 4, 3>(a, k, t, st);
+    case 8: return single<D, 4, 4>(a, k, t, st);
+    case 9: return single<D, 5, 4>(a, k, t, st);
+    default: return single<D, 5, 5>(a, k, t, st);
+  }
+  // 2^12: one kernel instead of a column step and rows once the grid is full (Fp 2^22 words
+  // 35.2 -> 28.4 us, Fp2 2^25 words 239 -> 204; but Fp 2^19 words 11.6 -> 15.9, Fp2 2^20
+  // 16.8 -> 19.9, and Fp2 2^23 words 59.0 and 60.7, the same).
+  if constexpr (D < 3) {
+    if (a.logC == 12 && a.M * a.N * D >= (D == 1 ? 1ull << 22 : 1ull << 24)) return cube<D>(a, k, t, st);
   }
   // Fp3 messages go through both passes in groups whose intermediate is at most 128 MB:
   // pass 2's reads of it (and its partly written lines) then meet in the 256 MB last-level
@@ -621,6 +846,9 @@ void encode(const RsArgs& a, const MxTables& t, uint64_t* scratch, hipStream_t s
     b.j0 = j0;
     b.M = std::min<size_t>(per, a.M - j0);
     switch (a.logC - logC1) {
+      case 3: column<D, 3>(b, k, t, scratch, logC1, st); break;
+      case 4: column<D, 4>(b, k, t, scratch, logC1, st); break;
+      case 5: column<D, 5>(b, k, t, scratch, logC1, st); break;
       case 8: pass1<D, 4, 4>(b, k, t, scratch, logC1, st); break;
       case 9: pass1<D, 5, 4>(b, k, t, scratch, logC1, st); break;
       default: pass1<D, 5, 5>(b, k, t, scratch, logC1, st); break;
@@ -635,9 +863,11 @@ void encode(const RsArgs& a, const MxTables& t, uint64_t* scratch, hipStream_t s
 
 }  // namespace
 
-bool mx_split(int D, int logC, int* logC1) {
-  *logC1 = logC >= 16 ? (logC + 1) / 2 : 0;
-  return (logC >= 8 && logC <= 10) || (logC >= 16 && logC <= 20);
+bool mx_split(int logC, int* logC1) {
+  // one pass up to 2^10; 2^11 .. 2^15 a column step of 8, 16 or 32, then rows; from 2^16
+  // the balanced split
+  *logC1 = logC < 11 ? 0 : logC == 11 ? 8 : logC < 16 ? std::min(logC - 4, 10) : (logC + 1) / 2;
+  return logC >= 4 && logC <= 20;
 }
 
 void mx_prepare() { (void)consts(); }
