@@ -1055,7 +1055,6 @@ static int cov_k(size_t n, int D) {
 // points come as exponents of the domain's root of unity (x = w_N^e), so each of their
 // table entries is one twiddle-table product (exponents multiply mod N); the few OOD
 // points' tables are powers computed in short runs.
-constexpr int GEO_K = 4;        // rows h per block
 constexpr int GEO_RUN = 8;      // consecutive OOD-point table entries per thread
 struct GeoPlan {
   size_t m_e, m_b, H;           // OOD points first, then in-domain points; H = n / 256
@@ -1114,41 +1113,63 @@ __global__ void k_geo_tables(uint64_t* buf, GeoPlan L, const uint64_t* in_dev, C
   }
 }
 
-template <int D>
-__global__ __launch_bounds__(256) void k_geo(uint64_t* acc, size_t n, int accumulate, const uint64_t* buf, GeoPlan L) {
-  const size_t l = threadIdx.x, h0 = (size_t)blockIdx.x * GEO_K;
-  gl::Wide W[GEO_K][D];
+// K rows h per block, the points dealt out to QG groups of 256 lanes (each group sums every
+// QG-th point, then group 0 adds the groups' reduced sums from LDS).  A lane's work is a
+// serial sum over the points, so a short vector needs the groups to fill the chip; the rows
+// a lane shares its LO loads among matter only once it is full.
+template <int D, int K, int QG>
+__global__ __launch_bounds__(256 * QG) void k_geo(uint64_t* acc, size_t n, int accumulate, const uint64_t* buf, GeoPlan L) {
+  __shared__ uint64_t part[QG > 1 ? (QG - 1) * 256 * K * D : 1];
+  const size_t l = threadIdx.x & 255, h0 = (size_t)blockIdx.x * K;
+  const size_t q = QG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
+  gl::Wide W[K][D];
 #pragma unroll
-  for (int k = 0; k < GEO_K; k++)
+  for (int k = 0; k < K; k++)
 #pragma unroll
     for (int d = 0; d < D; d++) W[k][d] = gl::Wide{0, 0, 0};
   const uint64_t* hi = buf + L.hi;
   // in-domain points: HI (extension) x LO (base), D products per row.  The query loops
   // are unrolled so that the loads of several queries share one wait (short vectors run
-  // about one wave per SIMD, with nothing else to hide the latency).
+  // a few waves per SIMD, with little else to hide the latency).
 #pragma unroll 4
-  for (size_t j = 0; j < L.m_b; j++) {
+  for (size_t j = q; j < L.m_b; j += QG) {
     const uint64_t lo = buf[L.lo_b + j * 256 + l];
     const uint64_t* hj = hi + ((L.m_e + j) * L.H + h0) * D;
 #pragma unroll
-    for (int k = 0; k < GEO_K; k++)
+    for (int k = 0; k < K; k++)
 #pragma unroll
       for (int d = 0; d < D; d++) gl::wide_mac(W[k][d], hj[k * D + d], lo);
   }
-  Ext<D> sum[GEO_K];
+  Ext<D> sum[K];
 #pragma unroll
-  for (int k = 0; k < GEO_K; k++)
+  for (int k = 0; k < K; k++)
 #pragma unroll
     for (int d = 0; d < D; d++) sum[k].c[d] = gl::wide_reduce(W[k][d]);
   // OOD points: full extension products
 #pragma unroll 2
-  for (size_t j = 0; j < L.m_e; j++) {
+  for (size_t j = q; j < L.m_e; j += QG) {
     const Ext<D> lo = ld<D>(buf + L.lo_e, j * 256 + l);
 #pragma unroll
-    for (int k = 0; k < GEO_K; k++) sum[k] = gl::eadd<D>(sum[k], gl::emul<D>(ld<D>(hi, j * L.H + h0 + k), lo));
+    for (int k = 0; k < K; k++) sum[k] = gl::eadd<D>(sum[k], gl::emul<D>(ld<D>(hi, j * L.H + h0 + k), lo));
+  }
+  if constexpr (QG > 1) {
+    if (q) {
+#pragma unroll
+      for (int k = 0; k < K; k++)
+#pragma unroll
+        for (int d = 0; d < D; d++) part[(((q - 1) * K + k) * D + d) * 256 + l] = sum[k].c[d];
+    }
+    __syncthreads();
+    if (q) return;
+#pragma unroll
+    for (int g = 0; g < QG - 1; g++)
+#pragma unroll
+      for (int k = 0; k < K; k++)
+#pragma unroll
+        for (int d = 0; d < D; d++) sum[k].c[d] = gl::add(sum[k].c[d], part[((g * K + k) * D + d) * 256 + l]);
   }
 #pragma unroll
-  for (int k = 0; k < GEO_K; k++) {
+  for (int k = 0; k < K; k++) {
     const size_t i = (h0 + k) * 256 + l;
     if (i < n) st<D>(acc, i, accumulate ? gl::eadd<D>(ld<D>(acc, i), sum[k]) : sum[k]);
   }
@@ -1204,7 +1225,13 @@ static void geo_terms_t(uint64_t* acc, size_t n, bool accumulate, const uint64_t
                                                           args, tw);
   WHIR_HIP(hipGetLastError());
   ProfScope prof(kernel_name("k_geo", D), s, 8.0 * D * (accumulate ? 2.0 : 1.0) * (double)n);
-  k_geo<D><<<(unsigned)(L.H / GEO_K), 256, 0, s>>>(acc, n, accumulate ? 1 : 0, buf.as<uint64_t>(), L);
+  const int ac = accumulate ? 1 : 0;
+  const uint64_t* tb = buf.as<uint64_t>();
+  // The shapes measured at n = 2^10, 2^16, 2^18, 2^20 (Fp2, all STIR launches of a proof):
+  // four rows and one group 74 (k_cov), 70, 96, 173 us; four rows and two groups -, -, 71, 167;
+  // one row and four groups 15, 18, 61, 309.
+  if (L.H >= 2048 && L.H % 4 == 0) k_geo<D, 4, 2><<<(unsigned)(L.H / 4), 512, 0, s>>>(acc, n, ac, tb, L);
+  else k_geo<D, 1, 4><<<(unsigned)L.H, 1024, 0, s>>>(acc, n, ac, tb, L);
   WHIR_HIP(hipGetLastError());
 }
 
@@ -1472,7 +1499,7 @@ void covector_stir_dev(int D, uint64_t* acc, size_t n, bool accumulate, const ui
                        const uint64_t* ext_points, size_t m_e, const uint64_t* exps, const uint64_t* points, size_t m_b,
                        int logN, hipStream_t s) {
   const size_t m = m_e + m_b;
-  if (!geo_path_enabled() || m < 8 || n < ((size_t)1 << 14) || n % (256 * GEO_K) || logN > 62) {
+  if (!geo_path_enabled() || m < 8 || !n || n % 256 || logN > 62) {
     // the one-pass kernel, with every point as a field element (in-domain points lifted)
     std::vector<uint64_t> pts(ext_points, ext_points + m_e * D);
     for (size_t j = 0; j < m_b; j++) {
