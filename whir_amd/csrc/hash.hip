@@ -404,15 +404,32 @@ __device__ __forceinline__ uint32_t quad_perm(uint32_t v) {
   return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, false);
 }
 
-// BLAKE3 of the 64-byte message msg[0..15] (LDS, the same for the quad's four lanes),
-// flags CHUNK_START | CHUNK_END | ROOT.  All four lanes of the quad must be active.
-__device__ __forceinline__ void b3q_pair(const uint32_t* msg, const uint32_t (&mo)[28], uint32_t iva, uint32_t ivb,
-                                         uint32_t dinit, uint32_t& lo, uint32_t& hi) {
+// What lane q of a quad keeps: where its message words are, and its column of the initial
+// state (dpar: of a 64-byte message, flags CHUNK_START | CHUNK_END | ROOT).
+struct B3QLane {
+  uint32_t mo[28], iva, ivb, dpar;
+};
+__device__ __forceinline__ B3QLane b3q_lane(uint32_t q) {
+  constexpr B3QSched S = b3q_sched();
+  B3QLane t;
+#pragma unroll
+  for (int j = 0; j < 28; j++) t.mo[j] = (S.p[j] >> (4 * q)) & 15u;
+  t.iva = hd::B3_IV[q];
+  t.ivb = hd::B3_IV[4 + q];
+  t.dpar = q == 2 ? 64u : (q == 3 ? (uint32_t)(hd::B3_CHUNK_START | hd::B3_CHUNK_END | hd::B3_ROOT) : 0u);
+  return t;
+}
+
+// One compression of the 64-byte block msg[0..15] (LDS, the same for the quad's four
+// lanes) from the chaining words (a, b) = (cv[q], cv[4 + q]) with d = dinit in row 3, to
+// lane q's chaining words (lo, hi).  All four lanes of the quad must be active.
+__device__ __forceinline__ void b3q_compress(const uint32_t* msg, const B3QLane& t, uint32_t a, uint32_t b,
+                                             uint32_t dinit, uint32_t& lo, uint32_t& hi) {
   using hd::rotr32;
   uint32_t x[28];
 #pragma unroll
-  for (int j = 0; j < 28; j++) x[j] = msg[mo[j]];
-  uint32_t a = iva, b = ivb, c = iva, d = dinit;
+  for (int j = 0; j < 28; j++) x[j] = msg[t.mo[j]];
+  uint32_t c = t.iva, d = dinit;
 #pragma unroll
   for (int r = 0; r < 7; r++) {
     B3G(a, b, c, d, x[4 * r], x[4 * r + 1]);
@@ -428,83 +445,66 @@ __device__ __forceinline__ void b3q_pair(const uint32_t* msg, const uint32_t (&m
   hi = b ^ d;
 }
 
-// k_merkle_sub for BLAKE3 with a quad per node: quad i takes the place of lane i (the
-// same phases, groups and node indices), four times the threads.
-constexpr int B3Q_THREADS = 4 * MERKLE_THREADS;
+// A parent's message in LDS: pairs of nodes (16 words) lie 20 words apart, so that the 16
+// quads of a wave, which all read the same word of their pairs, meet at most two to a bank
+// (16 or 64 words apart they met eight and sixteen to one).
+constexpr int B3Q_PAIR = 20;
+__device__ __forceinline__ uint32_t b3q_at(uint32_t node) { return (node >> 1) * B3Q_PAIR + (node & 1) * 8; }
 
+// Pairs the 2^L nodes (of a level of `width`, from node `first`) that lie in `src`, level
+// after level, to one node, through `dst` (half as large) and back; quad i makes nodes i, i +
+// quads, ... of each level and stores them to the tree.  Whole block; returns where the last
+// node is.
+constexpr int B3Q_THREADS = 4 * MERKLE_THREADS;
+__device__ __forceinline__ uint32_t* b3q_levels(uint32_t* src, uint32_t* dst, const B3QLane& ql, uint32_t* nodes32,
+                                                size_t W, size_t width, size_t first, int L) {
+  const uint32_t q = threadIdx.x & 3, qi = threadIdx.x >> 2, nq = blockDim.x >> 2;
+  uint32_t cnt = 1u << L;
+  __syncthreads();
+#pragma unroll 1
+  for (int lv = 0; lv < L; lv++) {
+    cnt >>= 1;
+    width >>= 1;
+    first >>= 1;
+    for (uint32_t i = qi; i < cnt; i += nq) {
+      uint32_t lo, hi;
+      b3q_compress(src + i * B3Q_PAIR, ql, ql.iva, ql.ivb, ql.dpar, lo, hi);
+      const size_t node = 2 * W - 2 * width + first + i;
+      nodes32[8 * node + q] = lo;
+      nodes32[8 * node + 4 + q] = hi;
+      dst[b3q_at(i) + q] = lo;
+      dst[b3q_at(i) + 4 + q] = hi;
+    }
+    __syncthreads();
+    uint32_t* t = src;
+    src = dst;
+    dst = t;
+  }
+  return src;
+}
+
+// k_merkle_sub for BLAKE3 with a quad per node (pairs only: G1 = 1), four times the threads.
+// A level of 2^10 nodes goes to the root in one launch, its first level in two rounds.
+constexpr int B3Q_MAX_L = 10;
 __global__ __launch_bounds__(B3Q_THREADS) void k_merkle_sub_b3q(uint8_t* __restrict__ nodes, size_t W, size_t w,
-                                                                 int L, int G1, uint32_t* root_out, BatchTab tab,
+                                                                 int L, uint32_t* root_out, BatchTab tab,
                                                                  MailboxSig sig) {
-  __shared__ uint32_t buf[2][MERKLE_THREADS][8];
-  __shared__ uint32_t grp[MERKLE_THREADS][8][8];
+  __shared__ __attribute__((aligned(16))) uint32_t src[(1 << B3Q_MAX_L) / 2 * B3Q_PAIR], dst[(1 << B3Q_MAX_L) / 4 * B3Q_PAIR];
   size_t blk = blockIdx.x;
   if (tab.nodes) {
     nodes = tab.nodes[blk / tab.per];
     if (root_out) root_out = (uint32_t*)(tab.roots + 32 * (blk / tab.per));
     blk %= tab.per;
   }
-  uint32_t* nodes32 = (uint32_t*)nodes;
   const uint32_t q = threadIdx.x & 3, qi = threadIdx.x >> 2;
-  constexpr B3QSched S = b3q_sched();
-  uint32_t mo[28];
-#pragma unroll
-  for (int j = 0; j < 28; j++) mo[j] = (S.p[j] >> (4 * q)) & 15u;
-  const uint32_t iva = hd::B3_IV[q], ivb = hd::B3_IV[4 + q];
-  const uint32_t dinit = q == 2 ? 64u : (q == 3 ? (uint32_t)(hd::B3_CHUNK_START | hd::B3_CHUNK_END | hd::B3_ROOT) : 0u);
-  size_t width = w;
-  size_t first = blk << L;
-  size_t cnt = (size_t)1 << L;
-  int left = L, cur = 0;
-  bool from_global = true;
-  while (left > 0) {
-    const int G = from_global ? (left < G1 ? left : G1) : 1;
-    const size_t quads = cnt >> G;
-    if (qi < quads) {
-      const size_t f = first + ((size_t)qi << G);
-      uint32_t lo = 0, hi = 0;
-      if (from_global) {
-        for (int k = (int)q; k < (1 << G); k += 4) {
-          const uint4* src = (const uint4*)(nodes + 32 * (2 * W - 2 * width + f + k));
-          uint4* dst = (uint4*)&grp[qi][k][0];
-          dst[0] = src[0];
-          dst[1] = src[1];
-        }
-        __builtin_amdgcn_wave_barrier();
-        size_t wd = width, fl = f;
-        for (int lv = 0; lv < G; lv++) {
-          wd >>= 1;
-          fl >>= 1;
-          const size_t base = 2 * W - 2 * wd + fl;
-          for (int k = 0; k < (1 << (G - 1 - lv)); k++) {
-            b3q_pair(&grp[qi][2 * k][0], mo, iva, ivb, dinit, lo, hi);
-            __builtin_amdgcn_wave_barrier();
-            grp[qi][k][q] = lo;
-            grp[qi][k][4 + q] = hi;
-            nodes32[8 * (base + k) + q] = lo;
-            nodes32[8 * (base + k) + 4 + q] = hi;
-            __builtin_amdgcn_wave_barrier();
-          }
-        }
-      } else {
-        b3q_pair(&buf[cur][2 * qi][0], mo, iva, ivb, dinit, lo, hi);
-        const size_t base = 2 * W - 2 * (width >> 1) + (f >> 1);
-        nodes32[8 * base + q] = lo;
-        nodes32[8 * base + 4 + q] = hi;
-      }
-      buf[cur ^ 1][qi][q] = lo;
-      buf[cur ^ 1][qi][4 + q] = hi;
-    }
-    __syncthreads();
-    cur ^= 1;
-    from_global = false;
-    width >>= G;
-    first >>= G;
-    cnt = quads;
-    left -= G;
-  }
+  const B3QLane ql = b3q_lane(q);
+  const size_t first = blk << L;
+  for (uint32_t i = qi; i < (1u << L) / 2; i += blockDim.x >> 2)  // a pair is 64 contiguous bytes
+    *(uint4*)&src[i * B3Q_PAIR + 4 * q] = ((const uint4*)(nodes + 32 * (2 * W - 2 * w + first)))[4 * i + q];
+  const uint32_t* last = b3q_levels(src, dst, ql, (uint32_t*)nodes, W, w, first, L);
   if (root_out && threadIdx.x == 0) {
 #pragma unroll
-    for (int i = 0; i < 8; i++) root_out[i] = buf[cur][0][i];
+    for (int i = 0; i < 8; i++) root_out[i] = last[i];
     mailbox_raise(sig);
   }
 }
@@ -585,12 +585,13 @@ static size_t merkle_from(int engine, uint8_t* nodes, size_t W, size_t w, hipStr
     // Wide levels: eight nodes per lane first (2^11 per block); otherwise pairs
     // (2^9 per block), which has the shortest chain of dependent hashes.
     const int G1 = w >= ((size_t)MERKLE_THREADS << MERKLE_SPAN_LOG) ? merkle_gmax_rt(engine) : 1;
-    const int maxL = MERKLE_SPAN_LOG - 3 + G1;
+    const bool quads = engine == ENG_BLAKE3 && b3q_enabled() && G1 == 1;
+    const int maxL = quads && w == ((size_t)1 << B3Q_MAX_L) ? B3Q_MAX_L : MERKLE_SPAN_LOG - 3 + G1;
     int L = 0;
     while (L < maxL && ((size_t)2 << L) <= w && (w >> (L + 1)) >= stop) L++;
     const size_t blocks = w >> L;
     const size_t lanes = ((size_t)1 << L) >> std::min(L, G1);  // nodes made by the first phase
-    const bool quad = engine == ENG_BLAKE3 && b3q_enabled() && blocks * count * lanes <= B3Q_MAX_LANES;
+    const bool quad = quads && blocks * count * lanes <= B3Q_MAX_LANES;
     const unsigned threads = quad ? (unsigned)std::max<size_t>(64, std::min<size_t>(B3Q_THREADS, 4 * lanes))
                                   : (unsigned)std::max<size_t>(64, std::min<size_t>(MERKLE_THREADS, lanes));
     ProfScope prof(quad ? "k_merkle_sub_b3q" : "k_merkle_sub", st, 32.0 * (double)(2 * w - (w >> L)) * count);
@@ -599,7 +600,7 @@ static size_t merkle_from(int engine, uint8_t* nodes, size_t W, size_t w, hipStr
     // The launch that makes a single tree's root is the last of the commit.
     const MailboxSig sig = blocks == 1 && !tab.nodes && ro ? mailbox_take(ro) : MailboxSig{};
     if (quad) {
-      k_merkle_sub_b3q<<<(unsigned)(blocks * count), threads, 0, st>>>(nodes, W, w, L, G1, ro, tab, sig);
+      k_merkle_sub_b3q<<<(unsigned)(blocks * count), threads, 0, st>>>(nodes, W, w, L, ro, tab, sig);
     } else {
       engine_switch(engine, [&](auto E) {
         k_merkle_sub<decltype(E)::value><<<(unsigned)(blocks * count), threads, 0, st>>>(nodes, W, w, L, G1, ro,
@@ -786,14 +787,132 @@ __global__ __launch_bounds__(TREE_THREADS) void k_leaves_tree_b3w(const uint64_t
   store_digest(nodes + 32 * (N + N / 2 + R0 / 4 + 16 * (l & 3) + (l >> 2)), gp);
 }
 
+// The same for narrow codewords: a quad per row hashes its blocks (its four lanes load four
+// message words each, a block ahead), then the block's quads pair the digests up to one node
+// per block of 2^L rows.  With few rows the wave-cooperative kernel is a chain of up to 4 nb
+// + 3 dependent compressions on one wave per 256 rows; here it is nb + L shorter ones on 16
+// times the waves.
+template <int D>
+__global__ __launch_bounds__(B3Q_THREADS) void k_leaves_tree_b3q(const uint64_t* __restrict__ cw, size_t N, size_t M,
+                                                                 uint8_t* __restrict__ nodes, int L, uint32_t* root_out,
+                                                                 BatchTab tab, MailboxSig sig) {
+  __shared__ __attribute__((aligned(16))) uint32_t src[MERKLE_THREADS / 2 * B3Q_PAIR], msg[MERKLE_THREADS][B3Q_PAIR];
+  size_t blk = blockIdx.x;
+  if (tab.cw) {
+    cw = tab.cw[blk / tab.per];
+    nodes = tab.nodes[blk / tab.per];
+    if (root_out) root_out = (uint32_t*)(tab.roots + 32 * (blk / tab.per));
+    blk %= tab.per;
+  }
+  uint32_t* nodes32 = (uint32_t*)nodes;
+  const uint32_t q = threadIdx.x & 3, qi = threadIdx.x >> 2;
+  const B3QLane ql = b3q_lane(q);
+  const size_t nb = M * D / 8;
+  const size_t r0 = blk << L;
+  if (qi < (1u << L)) {
+    const size_t r = r0 + qi;
+    const auto load = [&](size_t b) {  // words 4q .. 4q + 3 of block b of row r
+      uint4 v;
+      if constexpr (D == 2) {
+        v = ((const uint4*)cw)[(4 * b + q) * N + r];
+      } else {
+        const size_t w0 = 8 * b + 2 * q, w1 = w0 + 1;
+        const uint64_t x = cw[((w0 / D) * N + r) * D + w0 % D], y = cw[((w1 / D) * N + r) * D + w1 % D];
+        v = make_uint4((uint32_t)x, (uint32_t)(x >> 32), (uint32_t)y, (uint32_t)(y >> 32));
+      }
+      return v;
+    };
+    uint32_t a = ql.iva, b = ql.ivb;
+    uint4 v = load(0);
+#pragma unroll 1
+    for (size_t k = 0; k < nb; k++) {
+      *(uint4*)&msg[qi][4 * q] = v;
+      __builtin_amdgcn_wave_barrier();
+      if (k + 1 < nb) v = load(k + 1);
+      const uint32_t flags =
+          (k == 0 ? hd::B3_CHUNK_START : 0u) | (k + 1 == nb ? (hd::B3_CHUNK_END | hd::B3_ROOT) : 0u);
+      b3q_compress(&msg[qi][0], ql, a, b, q == 2 ? 64u : (q == 3 ? flags : 0u), a, b);
+      __builtin_amdgcn_wave_barrier();
+    }
+    nodes32[8 * r + q] = a;
+    nodes32[8 * r + 4 + q] = b;
+    src[b3q_at(qi) + q] = a;
+    src[b3q_at(qi) + 4 + q] = b;
+  }
+  // (the levels go back and forth between the digests and the room of the rows' blocks)
+  const uint32_t* last = b3q_levels(src, &msg[0][0], ql, nodes32, N, N, r0, L);
+  if (root_out && threadIdx.x == 0) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) root_out[i] = last[i];
+    mailbox_raise(sig);
+  }
+}
+
+// Between the two: one row per lane, then the block's 2^9 digests paired to one by quads.
+constexpr int B3H_LOG = 9;
+template <int D>
+__global__ __launch_bounds__(1 << B3H_LOG) void k_leaves_tree_b3h(const uint64_t* __restrict__ cw, size_t N, size_t M,
+                                                                  uint8_t* __restrict__ nodes, BatchTab tab) {
+  __shared__ __attribute__((aligned(16))) uint32_t src[(1 << B3H_LOG) / 2 * B3Q_PAIR], dst[(1 << B3H_LOG) / 4 * B3Q_PAIR];
+  size_t blk = blockIdx.x;
+  if (tab.cw) {
+    cw = tab.cw[blk / tab.per];
+    nodes = tab.nodes[blk / tab.per];
+    blk %= tab.per;
+  }
+  const size_t nb = M * D / 8, r0 = blk << B3H_LOG, r = r0 + threadIdx.x;
+  {
+    uint32_t cv[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) cv[i] = hd::B3_IV[i];
+#pragma unroll 1
+    for (size_t b = 0; b < nb; b++) {
+      uint32_t m[16];
+      row_block<D>(cw, N, r, b, m);
+      const uint32_t flags =
+          (b == 0 ? hd::B3_CHUNK_START : 0u) | (b + 1 == nb ? (hd::B3_CHUNK_END | hd::B3_ROOT) : 0u);
+      hd::b3_compress(cv, m, 64, 0, flags);
+    }
+    store_digest(nodes + 32 * r, cv);
+    uint4* p = (uint4*)&src[b3q_at(threadIdx.x)];
+    p[0] = make_uint4(cv[0], cv[1], cv[2], cv[3]);
+    p[1] = make_uint4(cv[4], cv[5], cv[6], cv[7]);
+  }
+  (void)b3q_levels(src, dst, b3q_lane(threadIdx.x & 3), (uint32_t*)nodes, N, N, r0, B3H_LOG);
+}
+
 static bool fused_tree_ok(int engine, size_t N, size_t W) {
   return engine == ENG_BLAKE3 && N >= 4 && (N & (N - 1)) == 0 && W % 8 == 0 && W > 0 && W <= 128;
 }
 
+// Leaves and the first levels; returns the width of the last level made, or 0 when the root
+// has gone to root_out.
 template <int D>
-static void commit_cols_t(int engine, const uint64_t* cw, size_t N, size_t M, uint8_t* nodes, hipStream_t st,
-                          BatchTab tab = {}, size_t count = 1) {
+static size_t commit_cols_t(int engine, const uint64_t* cw, size_t N, size_t M, uint8_t* nodes, hipStream_t st,
+                            uint8_t* root_out, BatchTab tab = {}, size_t count = 1) {
   const size_t W = M * D;
+  // Per commit (leaves and tree, 16 Fp2 columns, MI355X), one wave per 256 rows / one lane per
+  // row / a quad per row: 2^12 rows 38 / - / 20 us, 2^16 43 / 30 / 25, 2^17 48 / 32 / 42, 2^18
+  // 52 / 49 / 73, 2^19 77 / 79, 2^20 144 / 137, 2^21 235 / 244; rows of six blocks (Fp3) 2^19
+  // 110 / 106, 2^20 202 / 187, 2^21 339 / 333.
+  if (b3q_enabled() && N * count <= ((size_t)1 << 16)) {
+    int L = 0;
+    while (L < 8 && ((size_t)2 << L) <= N) L++;
+    tab.per = (uint32_t)(N >> L);
+    uint32_t* ro = tab.per == 1 ? (tab.nodes ? (uint32_t*)tab.roots : (uint32_t*)root_out) : nullptr;
+    const MailboxSig sig = tab.per == 1 && !tab.nodes && ro ? mailbox_take(ro) : MailboxSig{};
+    ProfScope prof(kernel_name("k_leaves_tree_b3q", D), st, (8.0 * (double)W * N + 64.0 * N) * count);
+    k_leaves_tree_b3q<D><<<tab.per * (unsigned)count, std::max(64, 4 << L), 0, st>>>(cw, N, M, nodes, L, ro, tab, sig);
+    WHIR_HIP(hipGetLastError());
+    return tab.per == 1 ? 0 : N >> L;
+  }
+  if (b3q_enabled() && N >= (1 << B3H_LOG) && N * count <= ((size_t)1 << (W >= 48 ? 21 : 18))) {
+    tab.per = (uint32_t)(N >> B3H_LOG);
+    ProfScope prof(kernel_name("k_leaves_tree_b3h", D), st, (8.0 * (double)W * N + 64.0 * N) * count);
+    k_leaves_tree_b3h<D><<<tab.per * (unsigned)count, 1 << B3H_LOG, 0, st>>>(cw, N, M, nodes, tab);
+    WHIR_HIP(hipGetLastError());
+    return N >> B3H_LOG;
+  }
   tab.per = blocks_for(N / 4, TREE_THREADS);
   const unsigned grid = tab.per * (unsigned)count;
   const double bytes = (8.0 * (double)W * N + 32.0 * (N + N / 2 + N / 4)) * count;
@@ -805,6 +924,7 @@ static void commit_cols_t(int engine, const uint64_t* cw, size_t N, size_t M, ui
     k_leaves_tree_b3<D><<<grid, TREE_THREADS, 0, st>>>(cw, N, M, nodes, tab);
   }
   WHIR_HIP(hipGetLastError());
+  return N / 4;
 }
 
 void commit_cols_dev(int engine, int D, const uint64_t* cw, size_t N, size_t M, uint8_t* nodes, hipStream_t st,
@@ -816,13 +936,14 @@ void commit_cols_dev(int engine, int D, const uint64_t* cw, size_t N, size_t M, 
     merkle_build_dev(engine, nodes, N, st, root_out);
     return;
   }
+  size_t w = 0;
   switch (D) {
-    case 1: commit_cols_t<1>(engine, cw, N, M, nodes, st); break;
-    case 2: commit_cols_t<2>(engine, cw, N, M, nodes, st); break;
-    case 3: commit_cols_t<3>(engine, cw, N, M, nodes, st); break;
+    case 1: w = commit_cols_t<1>(engine, cw, N, M, nodes, st, root_out); break;
+    case 2: w = commit_cols_t<2>(engine, cw, N, M, nodes, st, root_out); break;
+    case 3: w = commit_cols_t<3>(engine, cw, N, M, nodes, st, root_out); break;
     default: throw Error("leaf hash: extension degree must be 1, 2 or 3");
   }
-  merkle_from(engine, nodes, N, N / 4, st, root_out);
+  if (w) merkle_from(engine, nodes, N, w, st, root_out);
 }
 
 // SHA3-256 / Keccak-256 trees with their top on the host.  The narrow levels of a Keccak
@@ -893,13 +1014,14 @@ void commit_cols_many_dev(int engine, int D, const uint64_t* const* cw_tab, uint
     merkle_from(engine, nullptr, N, N, st, nullptr, tab, count);
     return;
   }
+  size_t w = 0;
   switch (D) {
-    case 1: commit_cols_t<1>(engine, nullptr, N, M, nullptr, st, tab, count); break;
-    case 2: commit_cols_t<2>(engine, nullptr, N, M, nullptr, st, tab, count); break;
-    case 3: commit_cols_t<3>(engine, nullptr, N, M, nullptr, st, tab, count); break;
+    case 1: w = commit_cols_t<1>(engine, nullptr, N, M, nullptr, st, nullptr, tab, count); break;
+    case 2: w = commit_cols_t<2>(engine, nullptr, N, M, nullptr, st, nullptr, tab, count); break;
+    case 3: w = commit_cols_t<3>(engine, nullptr, N, M, nullptr, st, nullptr, tab, count); break;
     default: throw Error("leaf hash: extension degree must be 1, 2 or 3");
   }
-  merkle_from(engine, nullptr, N, N / 4, st, nullptr, tab, count);
+  if (w) merkle_from(engine, nullptr, N, w, st, nullptr, tab, count);
 }
 
 // ------------------------------------------------------------------ constant rows
