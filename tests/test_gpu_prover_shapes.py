@@ -24,3 +24,13 @@ def check(nv, D, engine, k0, k, lir, npts, sec):
                                           (17, 2, 1, 100), (23, 2, 1, 40)])
 def test_stir_terms_over_short_and_long_vectors(nv, D, lir, sec):
     check(nv, D, W.HASH_BLAKE3, 4, 4, lir, 1, sec)
+
+
+# Sumcheck passes that sum two rounds: 2^10 and 2^11 elements are the last that one block
+# and the first that several blocks sum; odd round counts end with a pass of one round's two
+# sums; the initial round runs over tables of 1 to 2^6 blocks.
+@pytest.mark.parametrize("nv,D,k0,k", [(8, 1, 4, 4), (9, 2, 2, 2), (10, 3, 3, 3), (12, 2, 1, 1), (13, 1, 5, 5),
+                                       (13, 2, 3, 5), (14, 3, 4, 4), (14, 2, 2, 5), (15, 1, 3, 3), (15, 2, 4, 4),
+                                       (15, 3, 4, 3), (16, 2, 5, 6), (18, 1, 4, 7), (18, 3, 6, 4)])
+def test_sumcheck_pairs(nv, D, k0, k):
+    check(nv, D, W.HASH_BLAKE3, k0, k, 1, 2, 40 if D == 1 else 80)

@@ -51,104 +51,58 @@ __device__ __forceinline__ void st(uint64_t* p, size_t i, const Ext<D>& v) {
 template <int D>
 __device__ __forceinline__ Ext<D> ld_host(const uint64_t* const* unused, const Ext<D>& v) { return v; }
 
-// Sum NV extension values over the block into thread 0's v (other threads' v are left
-// partial).  Each wave sums its lanes by cross-lane exchanges (no barrier), its first
-// lane puts the wave's sum in LDS, and after one barrier thread 0 adds the waves' sums.
-template <int D, int NV>
-__device__ void block_sum(Ext<D> v[NV]) {
-  __shared__ uint64_t red[RT / 64][NV * D];
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1)
-#pragma unroll
-    for (int k = 0; k < NV; k++) {
-      Ext<D> o;
-#pragma unroll
-      for (int d = 0; d < D; d++) o.c[d] = __shfl_xor(v[k].c[d], off);
-      v[k] = gl::eadd<D>(v[k], o);
-    }
-  const int wave = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 0)
+// Block sums.  The short passes of a proof run these kernels on a wave or a few, where
+// straight-line code is fetched once and used once: at about 0.45 us per KB of cold code
+// on MI355X the fetch, not the arithmetic, was most of their time.  So the exchanges stay
+// a loop over the distance, and the last steps give a word to each thread.
+
+// Sums lane l of every R lanes (R a power of two; lane's role l = lane mod R) over the
+// block: tot[(l NV + k) D + d] for the role's value k, in LDS, for all threads.  At most
+// 1024 threads.
+template <int D, int NV, int R>
+__device__ __forceinline__ void block_role_sum(Ext<D> (&v)[NV], uint64_t* tot) {
+  constexpr int W = R * NV * D;
+  static_assert(W <= 64, "block_role_sum: one wave finishes the words");
+  __shared__ uint64_t red[16][W];
+#pragma unroll 1
+  for (int off = R; off < 64; off <<= 1)
 #pragma unroll
     for (int k = 0; k < NV; k++)
 #pragma unroll
-      for (int d = 0; d < D; d++) red[wave][k * D + d] = v[k].c[d];
+      for (int d = 0; d < D; d++) v[k].c[d] = gl::add(v[k].c[d], (uint64_t)__shfl_xor(v[k].c[d], off));
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  if (lane < R)
+#pragma unroll
+    for (int k = 0; k < NV; k++)
+#pragma unroll
+      for (int d = 0; d < D; d++) red[wave][(lane * NV + k) * D + d] = v[k].c[d];
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (threadIdx.x < W) {
     const int waves = blockDim.x >> 6;
-#pragma unroll
-    for (int k = 0; k < NV; k++) {
-#pragma unroll
-      for (int d = 0; d < D; d++) v[k].c[d] = red[0][k * D + d];
-      for (int w = 1; w < waves; w++) {
-        Ext<D> x;
-#pragma unroll
-        for (int d = 0; d < D; d++) x.c[d] = red[w][k * D + d];
-        v[k] = gl::eadd<D>(v[k], x);
-      }
-    }
+    uint64_t x = red[0][threadIdx.x];
+#pragma unroll 1
+    for (int w = 1; w < waves; w++) x = gl::add(x, red[w][threadIdx.x]);
+    tot[threadIdx.x] = x;
+  }
+  __syncthreads();
+}
+
+// The first W threads (one wave) store a word each; the flag follows when sig asks it to.
+template <int W>
+__device__ __forceinline__ void store_words(uint64_t word, uint64_t* out, const MailboxSig& sig) {
+  if (threadIdx.x < W) out[threadIdx.x] = word;
+  if (sig.flag) {
+    __syncthreads();  // every word is stored before thread 0 raises the flag
+    if (threadIdx.x == 0) mailbox_raise(sig);
   }
 }
 
-// Sum NV extension values over the block; thread 0 writes them to out (and then raises
-// the mailbox flag when sig asks it to).
+// Sum NV extension values over the block and write them to out.
 template <int D, int NV>
-__device__ void block_reduce_store(Ext<D> v[NV], uint64_t* out, MailboxSig sig = {}) {
-  block_sum<D, NV>(v);
-  if (threadIdx.x == 0) {
-#pragma unroll
-    for (int k = 0; k < NV; k++)
-#pragma unroll
-      for (int d = 0; d < D; d++) out[k * D + d] = v[k].c[d];
-    mailbox_raise(sig);
-  }
-}
-
-// Sum NV extension values over a block of RT threads through LDS: each thread stores
-// its values, 16 threads per value add 16 of the stored rows each, and one thread per
-// value adds those 16 partials.  The totals are in tot[0..NV) after the call (all
-// threads).  For single-block reductions of many values, where the cross-lane sum of
-// block_sum is a long chain of exchanges per value.
-template <int D, int NV>
-__device__ void block_sum_lds(const Ext<D> (&v)[NV], Ext<D> (&tot)[NV]) {
-  static_assert(NV * 16 <= RT, "block_sum_lds: at most RT / 16 values");
-  __shared__ uint64_t rows[RT][NV * D];
-  __shared__ uint64_t part[16][NV * D];
-  __shared__ uint64_t sum[NV * D];
-#pragma unroll
-  for (int k = 0; k < NV; k++)
-#pragma unroll
-    for (int d = 0; d < D; d++) rows[threadIdx.x][k * D + d] = v[k].c[d];
-  __syncthreads();
-  if (threadIdx.x < NV * 16) {
-    const int k = threadIdx.x >> 4, p = threadIdx.x & 15;
-    Ext<D> acc = gl::ext_zero<D>();
-    for (int r = p; r < (int)blockDim.x; r += 16) {
-      Ext<D> x;
-#pragma unroll
-      for (int d = 0; d < D; d++) x.c[d] = rows[r][k * D + d];
-      acc = gl::eadd<D>(acc, x);
-    }
-#pragma unroll
-    for (int d = 0; d < D; d++) part[p][k * D + d] = acc.c[d];
-  }
-  __syncthreads();
-  if (threadIdx.x < NV) {
-    Ext<D> acc = gl::ext_zero<D>();
-#pragma unroll
-    for (int p = 0; p < 16; p++) {
-      Ext<D> x;
-#pragma unroll
-      for (int d = 0; d < D; d++) x.c[d] = part[p][threadIdx.x * D + d];
-      acc = gl::eadd<D>(acc, x);
-    }
-#pragma unroll
-    for (int d = 0; d < D; d++) sum[threadIdx.x * D + d] = acc.c[d];
-  }
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < NV; k++)
-#pragma unroll
-    for (int d = 0; d < D; d++) tot[k].c[d] = sum[k * D + d];
+__device__ void block_reduce_store(Ext<D> (&v)[NV], uint64_t* out, MailboxSig sig = {}) {
+  __shared__ uint64_t tot[NV * D];
+  block_role_sum<D, NV, 1>(v, tot);
+  store_words<NV * D>(threadIdx.x < NV * D ? tot[threadIdx.x] : 0, out, sig);
 }
 
 // Final reduction of `nparts` block partials of NV*D words each into `out`
@@ -157,27 +111,23 @@ __device__ void block_sum_lds(const Ext<D> (&v)[NV], Ext<D> (&tot)[NV]) {
 // release that pattern needs writes back the XCD's L2, and the producing kernels
 // have just filled it with their outputs (measured 1.5x slower on MI355X).
 template <int D, int NV>
-__global__ __launch_bounds__(RT) void k_reduce_parts(const uint64_t* parts, size_t nparts, uint64_t* out,
-                                                     MailboxSig sig) {
-  Ext<D> v[NV];
-#pragma unroll
-  for (int k = 0; k < NV; k++) v[k] = gl::ext_zero<D>();
-  for (size_t p = threadIdx.x; p < nparts; p += blockDim.x)
-#pragma unroll
-    for (int k = 0; k < NV; k++) v[k] = gl::eadd<D>(v[k], ld<D>(parts + p * NV * D, k));
-  Ext<D> tot[NV];
-  block_sum_lds<D, NV>(v, tot);
-  if (threadIdx.x == 0) {
-#pragma unroll
-    for (int k = 0; k < NV; k++) st<D>(out, k, tot[k]);
-    mailbox_raise(sig);
-  }
+__global__ __launch_bounds__(1024) void k_reduce_parts(const uint64_t* parts, size_t nparts, uint64_t* out,
+                                                       MailboxSig sig) {
+  __shared__ uint64_t tot[NV * D];
+  Ext<D> v[1] = {gl::ext_zero<D>()};
+  // a value per thread, so that the block reads the partials in order
+  for (size_t e = threadIdx.x; e < nparts * NV; e += blockDim.x) v[0] = gl::eadd<D>(v[0], ld<D>(parts, e));
+  block_role_sum<D, 1, NV>(v, tot);
+  store_words<NV * D>(threadIdx.x < NV * D ? tot[threadIdx.x] : 0, out, sig);
 }
+
+// Threads of a one-block reduction of n values: whole waves, at most 1024.
+static unsigned reduce_threads(size_t n) { return (unsigned)std::min<size_t>(1024, (n + 63) / 64 * 64); }
 
 // last: this launch ends the work a mailbox wait may be armed for.
 template <int D, int NV>
 static void finish_reduce(const uint64_t* parts, unsigned nparts, uint64_t* out, hipStream_t s, bool last = true) {
-  k_reduce_parts<D, NV><<<1, RT, 0, s>>>(parts, nparts, out, last ? mailbox_take(out) : MailboxSig{});
+  k_reduce_parts<D, NV><<<1, reduce_threads(nparts * (size_t)NV), 0, s>>>(parts, nparts, out, last ? mailbox_take(out) : MailboxSig{});
   WHIR_HIP(hipGetLastError());
 }
 
@@ -504,29 +454,46 @@ size_t fold_and_poly_dev(int D, uint64_t* a, uint64_t* b, size_t n, const uint64
 //     U = x_(q+i) - x_i,  V = dx_(q+i) - dx_i:  T0 = sum Ux Uy,  T1 = sum (Ux Vy + Vx Uy),
 //     T2 = sum Vx Vy
 // (the same field values as folding first and summing after, the order of exact
-// additions aside).  Lane i takes positions i, q+i, 2q+i, 3q+i.  With FOLD the vectors
-// are first folded by two pending challenges (r1, then r2) from length 4L, position t
-// from t, L+t, 2L+t, 3L+t of the source, and written (a to a_out, b in place: lane i
-// writes only its own four positions, the only ones below L that it reads).  NS: sums
-// per block, 8 (c0, c2, S0, S1, S2, T0, T1, T2), 2 (c0, c2) or 0.
+// additions aside).  With FOLD the vectors are first folded by two pending challenges
+// (r1, then r2) from length 4L, position t from t, L+t, 2L+t, 3L+t of the source, and
+// written (a to a_out, b in place: a lane writes only its own position, the only one
+// below L that it reads).  NS: sums per block, 8 (c0, c2, S0, S1, S2, T0, T1, T2) or 2
+// (c0, c2).
+//
+// The position folded by r1 then r2 is bilinear in the challenges:
+//   x0 + r1 (x2 - x0) + r2 (x1 - x0) + r1 r2 (x3 - x2 - x1 + x0)
+// so its three products are summed unreduced and reduced once per coefficient.
+template <int D>
+struct Fold4 {
+  Ext<D> r1, r2, r12;
+};
+
 template <int Ds, int D>
-__device__ __forceinline__ Ext<D> fold_twice(const uint64_t* v, size_t t, size_t L, const Ext<D>& r1,
-                                             const Ext<D>& r2) {
-  Ext<D> p, q;
+__device__ __forceinline__ Ext<D> fold_twice(const uint64_t* v, size_t t, size_t L, const Fold4<D>& f) {
+  gl::Wide w[D];
+  gl::wide_zero<D>(w);
+  Ext<D> r;
   if constexpr (Ds == 1 && D > 1) {
-    // base-field source: the first fold scales r1 by a base-field difference
     const uint64_t x0 = v[t], x1 = v[L + t], x2 = v[2 * L + t], x3 = v[3 * L + t];
-    p = gl::escale<D>(r1, gl::sub(x2, x0));
-    p.c[0] = gl::add(p.c[0], x0);
-    q = gl::escale<D>(r1, gl::sub(x3, x1));
-    q.c[0] = gl::add(q.c[0], x1);
+    const uint64_t d1 = gl::sub(x2, x0), d2 = gl::sub(x1, x0), d3 = gl::sub(gl::sub(x3, x2), d2);
+#pragma unroll
+    for (int d = 0; d < D; d++) {
+      gl::wide_mac(w[d], d1, f.r1.c[d]);
+      gl::wide_mac(w[d], d2, f.r2.c[d]);
+      gl::wide_mac(w[d], d3, f.r12.c[d]);
+    }
+    r = gl::ext_reduce<D>(w);
+    r.c[0] = gl::add(r.c[0], x0);
   } else {
     const Ext<D> x0 = ldx<Ds, D>(v, t), x1 = ldx<Ds, D>(v, L + t), x2 = ldx<Ds, D>(v, 2 * L + t),
                  x3 = ldx<Ds, D>(v, 3 * L + t);
-    p = gl::eadd<D>(x0, gl::emul<D>(gl::esub<D>(x2, x0), r1));
-    q = gl::eadd<D>(x1, gl::emul<D>(gl::esub<D>(x3, x1), r1));
+    const Ext<D> d2 = gl::esub<D>(x1, x0);
+    gl::emul_acc<D>(w, gl::esub<D>(x2, x0), f.r1);
+    gl::emul_acc<D>(w, d2, f.r2);
+    gl::emul_acc<D>(w, gl::esub<D>(gl::esub<D>(x3, x2), d2), f.r12);
+    r = gl::eadd<D>(gl::ext_reduce<D>(w), x0);
   }
-  return gl::eadd<D>(p, gl::emul<D>(gl::esub<D>(q, p), r2));
+  return r;
 }
 
 // Element i of a covector view: sum_k hi_k[i >> sh] lo_k[i & (2^sh - 1)].
@@ -539,125 +506,186 @@ __device__ __forceinline__ Ext<D> view_at(const CovView& v, size_t i) {
   return r;
 }
 
-// VIEW: b's values come from the view v (mode 0: y itself; folding modes: y already
-// folded by (r1, r2)) instead of from b, and the folding modes write them into b.
-template <int Ds, int D, bool FOLD, int NS, bool VIEW>
-__global__ __launch_bounds__(RT) void k_sc_pair(const uint64_t* a_in, uint64_t* a_out, uint64_t* b, size_t L,
-                                                Ext<D> r1, Ext<D> r2, uint64_t* parts, MailboxSig sig, CovView v) {
-  constexpr int NA = NS > 0 ? NS : 1;
-  Ext<D> acc[NA];
-#pragma unroll
-  for (int k = 0; k < NA; k++) acc[k] = gl::ext_zero<D>();
-  const size_t q = L >> 2;
-  if constexpr (FOLD && NS == 0) {
-    // the double fold alone: one output position per lane (four times the lanes of the
-    // summing passes, which the short vectors at the end of a sumcheck need)
-    for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < L; t += (size_t)gridDim.x * blockDim.x) {
-      const Ext<D> x = fold_twice<Ds, D>(a_in, t, L, r1, r2);
-      const Ext<D> y = VIEW ? view_at<D>(v, t) : fold_twice<D, D>(b, t, L, r1, r2);
-      st<D>(a_out, t, x);
-      st<D>(b, t, y);
-    }
-    return;
+// The double fold alone, one output position per lane.  VIEW: b's folded values come
+// from the view v instead of from b.
+template <int Ds, int D, bool VIEW>
+__global__ __launch_bounds__(RT) void k_fold4(const uint64_t* a_in, uint64_t* a_out, uint64_t* b, size_t L,
+                                              Fold4<D> f, CovView v) {
+  for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < L; t += (size_t)gridDim.x * blockDim.x) {
+    const Ext<D> x = fold_twice<Ds, D>(a_in, t, L, f);
+    const Ext<D> y = VIEW ? view_at<D>(v, t) : fold_twice<D, D>(b, t, L, f);
+    st<D>(a_out, t, x);
+    st<D>(b, t, y);
   }
-  if constexpr (!FOLD && Ds == 1 && D > 1 && NS == 8) {
-    // x in the base field: every product is base x extension (D multiplies, not an
-    // extension product), and the differences of x are base-field differences.
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < q; i += (size_t)gridDim.x * blockDim.x) {
-      uint64_t x[4];
-      Ext<D> y[4];
-#pragma unroll
-      for (int k = 0; k < 4; k++) {
-        x[k] = a_in[k * q + i];
-        y[k] = VIEW ? view_at<D>(v, k * q + i) : ld<D>(b, k * q + i);
-      }
-      const uint64_t dx0 = gl::sub(x[2], x[0]), dx1 = gl::sub(x[3], x[1]);
-      const Ext<D> dy0 = gl::esub<D>(y[2], y[0]), dy1 = gl::esub<D>(y[3], y[1]);
-      const Ext<D> m0 = gl::escale<D>(y[0], x[0]), d0 = gl::escale<D>(dy0, dx0);
-      acc[0] = gl::eadd<D>(acc[0], gl::eadd<D>(m0, gl::escale<D>(y[1], x[1])));
-      acc[1] = gl::eadd<D>(acc[1], gl::eadd<D>(d0, gl::escale<D>(dy1, dx1)));
-      acc[2] = gl::eadd<D>(acc[2], m0);
-      acc[3] = gl::eadd<D>(acc[3], gl::eadd<D>(gl::escale<D>(dy0, x[0]), gl::escale<D>(y[0], dx0)));
-      acc[4] = gl::eadd<D>(acc[4], d0);
-      const uint64_t ux = gl::sub(x[1], x[0]), vx = gl::sub(dx1, dx0);
-      const Ext<D> uy = gl::esub<D>(y[1], y[0]), vy = gl::esub<D>(dy1, dy0);
-      acc[5] = gl::eadd<D>(acc[5], gl::escale<D>(uy, ux));
-      acc[6] = gl::eadd<D>(acc[6], gl::eadd<D>(gl::escale<D>(vy, ux), gl::escale<D>(uy, vx)));
-      acc[7] = gl::eadd<D>(acc[7], gl::escale<D>(vy, vx));
-    }
-    block_reduce_store<D, NS>(acc, parts + (size_t)blockIdx.x * NS * D, sig);
-    return;
-  }
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < q; i += (size_t)gridDim.x * blockDim.x) {
-    Ext<D> x[4], y[4];
-    static_for<4>([&](auto kc) {  // a constant k keeps x and y in registers for Fp3 too
-      constexpr int k = decltype(kc)::value;
-      const size_t t = k * q + i;
-      if constexpr (FOLD) {
-        x[k] = fold_twice<Ds, D>(a_in, t, L, r1, r2);
-        y[k] = VIEW ? view_at<D>(v, t) : fold_twice<D, D>(b, t, L, r1, r2);
-      } else {
-        x[k] = ldx<Ds, D>(a_in, t);
-        y[k] = VIEW ? view_at<D>(v, t) : ld<D>(b, t);
-      }
-    });
-    if constexpr (FOLD) {
-#pragma unroll
-      for (int k = 0; k < 4; k++) {
-        st<D>(a_out, k * q + i, x[k]);
-        st<D>(b, k * q + i, y[k]);
-      }
-    }
-    if constexpr (NS > 0) {
-      const Ext<D> dx0 = gl::esub<D>(x[2], x[0]), dx1 = gl::esub<D>(x[3], x[1]);
-      const Ext<D> dy0 = gl::esub<D>(y[2], y[0]), dy1 = gl::esub<D>(y[3], y[1]);
-      const Ext<D> m0 = gl::emul<D>(x[0], y[0]), d0 = gl::emul<D>(dx0, dy0);
-      acc[0] = gl::eadd<D>(acc[0], gl::eadd<D>(m0, gl::emul<D>(x[1], y[1])));
-      acc[1] = gl::eadd<D>(acc[1], gl::eadd<D>(d0, gl::emul<D>(dx1, dy1)));
-      if constexpr (NS == 8) {
-        acc[2] = gl::eadd<D>(acc[2], m0);
-        acc[3] = gl::eadd<D>(acc[3], gl::eadd<D>(gl::emul<D>(x[0], dy0), gl::emul<D>(dx0, y[0])));
-        acc[4] = gl::eadd<D>(acc[4], d0);
-        const Ext<D> ux = gl::esub<D>(x[1], x[0]), vx = gl::esub<D>(dx1, dx0);
-        const Ext<D> uy = gl::esub<D>(y[1], y[0]), vy = gl::esub<D>(dy1, dy0);
-        acc[5] = gl::eadd<D>(acc[5], gl::emul<D>(ux, uy));
-        acc[6] = gl::eadd<D>(acc[6], gl::eadd<D>(gl::emul<D>(ux, vy), gl::emul<D>(vx, uy)));
-        acc[7] = gl::eadd<D>(acc[7], gl::emul<D>(vx, vy));
-      }
-    }
-  }
-  if constexpr (NS > 0) block_reduce_store<D, NS>(acc, parts + (size_t)blockIdx.x * NS * D, sig);
 }
 
-template <int Ds, int D, bool FOLD, int NS, bool VIEW>
+// The value of lane CTRL[l] of each quad of lanes (quad_perm: two bits per lane l).
+template <int CTRL>
+__device__ __forceinline__ uint64_t quad_get(uint64_t v) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)v, CTRL, 0xf, 0xf, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(v >> 32), CTRL, 0xf, 0xf, true);
+  return ((uint64_t)hi << 32) | lo;
+}
+template <int CTRL, int D>
+__device__ __forceinline__ Ext<D> quad_get(const Ext<D>& v) {
+  Ext<D> r;
+#pragma unroll
+  for (int d = 0; d < D; d++) r.c[d] = quad_get<CTRL>(v.c[d]);
+  return r;
+}
+constexpr int quad_ctrl(int a, int b, int c, int d) { return a | b << 2 | c << 4 | d << 6; }
+
+// The second factor of a quad's lane: the quarter differences 2 - 0, 3 - 1, 3 - 2, 1 - 0,
+// and for lane 3 in place of its own quarter (3 - 2) - (1 - 0) as the first factor.
+template <int D>
+__device__ __forceinline__ void quad_factors(const Ext<D>& x, Ext<D>& p, Ext<D>& q) {
+  q = gl::esub<D>(quad_get<quad_ctrl(2, 3, 3, 1)>(x), quad_get<quad_ctrl(0, 1, 2, 0)>(x));
+  const Ext<D> w = gl::esub<D>(quad_get<quad_ctrl(2, 2, 2, 2)>(q), q);
+  const bool own = (threadIdx.x & 3) != 3;
+#pragma unroll
+  for (int d = 0; d < D; d++) p.c[d] = own ? x.c[d] : w.c[d];
+}
+// NS == 2: quarters 0 and 1, then the differences 2 - 0 and 3 - 1.
+template <int D>
+__device__ __forceinline__ Ext<D> quad_factor2(const Ext<D>& x) {
+  const Ext<D> w = gl::esub<D>(x, quad_get<quad_ctrl(0, 1, 0, 1)>(x));
+  Ext<D> p;
+#pragma unroll
+  for (int d = 0; d < D; d++) p.c[d] = (threadIdx.x & 2) ? w.c[d] : x.c[d];
+  return p;
+}
+
+// Word e of the pass's sums from the quads' products (NS == 8: prod[(2 l + j) D + d], j = 0
+// the first factors' product of lane l, j = 1 the second's; slot 8 is zero).  With
+// P_l and Q_l for the two: c0 = P0 + P1, c2 = Q0 + Q1, S0 = P0, S1 = P2 - P0 - Q0,
+// S2 = Q0, T0 = Q3, T1 = Q2 - Q3 - P3, T2 = P3.  The hex digits are the slots of each
+// sum's terms, sum 0 in the lowest.
+template <int D>
+__device__ __forceinline__ uint64_t pair_sum_word(const uint64_t* prod, unsigned e) {
+  const unsigned k = e / D, d = e % D;
+  auto at = [&](uint32_t slots) { return prod[((slots >> (4 * k)) & 15) * D + d]; };
+  return gl::sub(gl::sub(gl::add(at(0x65714010u), at(0x88888832u)), at(0x87880888u)), at(0x86881888u));
+}
+
+// Four lanes share the positions i, q+i, 2q+i, 3q+i: lane l folds and holds quarter l of x
+// and y, and the quad forms eight products, two per lane, of which the eight sums are
+// differences.  A lane that takes all four positions itself runs 34 extension products and
+// the sums of eight values in 42 KB of code, against 8 KB here, and that is what the
+// passes of a proof wait for once they are short: Fp2 with the fold on MI355X 20 -> 7.6 us
+// from 2^6 to 2^14 elements, without it 12-19 -> 4-6.6.
+template <int Ds, int D, bool FOLD, int NS>
+__global__ __launch_bounds__(1024) void k_sc_pair(const uint64_t* a_in, uint64_t* a_out, uint64_t* b, size_t L,
+                                                  Fold4<D> f, uint64_t* parts, MailboxSig sig) {
+  constexpr int Dx = FOLD ? D : Ds, NP = NS == 8 ? 2 : 1;
+  gl::Wide w[NP][D];
+#pragma unroll
+  for (int j = 0; j < NP; j++) gl::wide_zero<D>(w[j]);
+  const size_t q = L >> 2, l = threadIdx.x & 3;
+  const size_t step = ((size_t)gridDim.x * blockDim.x) >> 2;
+  auto mac = [&](gl::Wide(&acc)[D], const Ext<Dx>& x, const Ext<D>& y) {
+    if constexpr (Dx == D) {
+      gl::emul_acc<D>(acc, x, y);
+    } else {
+#pragma unroll
+      for (int d = 0; d < D; d++) gl::wide_mac(acc[d], x.c[0], y.c[d]);
+    }
+  };
+#pragma unroll 1
+  for (size_t i = (blockIdx.x * (size_t)blockDim.x + threadIdx.x) >> 2; i < q; i += step) {
+    const size_t t = l * q + i;
+    Ext<Dx> x;
+    Ext<D> y;
+    if constexpr (FOLD) {
+      x = fold_twice<Ds, D>(a_in, t, L, f);
+      y = fold_twice<D, D>(b, t, L, f);
+      st<D>(a_out, t, x);
+      st<D>(b, t, y);
+    } else {
+      x = ld<Dx>(a_in, t);
+      y = ld<D>(b, t);
+    }
+    if constexpr (NS == 8) {
+      Ext<Dx> px, qx;
+      Ext<D> py, qy;
+      quad_factors<Dx>(x, px, qx);
+      quad_factors<D>(y, py, qy);
+      mac(w[0], px, py);
+      mac(w[1], qx, qy);
+    } else {
+      mac(w[0], quad_factor2<Dx>(x), quad_factor2<D>(y));
+    }
+  }
+  Ext<D> v[NP];
+#pragma unroll
+  for (int j = 0; j < NP; j++) v[j] = gl::ext_reduce<D>(w[j]);
+  __shared__ uint64_t prod[9 * D];
+  if (threadIdx.x < D) prod[8 * D + threadIdx.x] = 0;
+  block_role_sum<D, NP, 4>(v, prod);
+  const unsigned e = threadIdx.x;
+  uint64_t word = 0;
+  if (e < NS * D) {
+    if constexpr (NS == 8) word = pair_sum_word<D>(prod, e);
+    else word = gl::add(prod[e / D * 2 * D + e % D], prod[(e / D * 2 + 1) * D + e % D]);
+  }
+  store_words<NS * D>(word, parts + (size_t)blockIdx.x * NS * D, sig);
+}
+
+template <int D>
+static Fold4<D> host_fold4(const uint64_t* r1, const uint64_t* r2) {
+  Fold4<D> f{gl::ext_zero<D>(), gl::ext_zero<D>(), gl::ext_zero<D>()};
+  if (r1 && r2) {
+    f.r1 = host_ext<D>(r1);
+    f.r2 = host_ext<D>(r2);
+    f.r12 = gl::emul<D>(f.r1, f.r2);
+  }
+  return f;
+}
+
+template <int Ds, int D, bool VIEW>
+static void fold4_t(const uint64_t* a_in, uint64_t* a_out, uint64_t* b, size_t L, const uint64_t* r1,
+                    const uint64_t* r2, const CovView& v, hipStream_t s) {
+  ProfScope prof(kernel_name("k_fold4", Ds, D), s, 8.0 * ((Ds + D) * 4.0 * L + 2.0 * D * L));
+  k_fold4<Ds, D, VIEW><<<grid_for(L), RT, 0, s>>>(a_in, a_out, b, L, host_fold4<D>(r1, r2), v);
+  WHIR_HIP(hipGetLastError());
+}
+
+// Up to this many quads a pass runs as one block of up to 1024 threads, which stores its
+// sums itself; above, the second launch (3 us and the gap before it) costs less than the
+// further turns on one CU.  Fp2 on MI355X: 256 quads without a fold 6.6 us in one block,
+// 1024 13 us against 6.5; with the fold 64 quads 5.8 us, 256 10.6 against 7.4 and the launch.
+static constexpr size_t SMALL_PAIRS_SUM = 256, SMALL_PAIRS_FOLD = 64;
+
+template <int Ds, int D, bool FOLD, int NS>
 static void sc_pair_t(const uint64_t* a_in, uint64_t* a_out, uint64_t* b, size_t L, const uint64_t* r1,
-                      const uint64_t* r2, uint64_t* out, const CovView& v, hipStream_t s) {
+                      const uint64_t* r2, uint64_t* out, hipStream_t s) {
   const size_t q = L >> 2;
-  const unsigned g = NS == 0 ? grid_for(L) : (q <= SMALL_PAIRS ? 1u : grid_for(q));
-  DevBuf parts(NS > 0 && g > 1 ? (size_t)g * NS * D * 8 : 0, s);
-  const Ext<D> w1 = r1 ? host_ext<D>(r1) : gl::ext_zero<D>(), w2 = r2 ? host_ext<D>(r2) : gl::ext_zero<D>();
+  const bool one = q <= (FOLD ? SMALL_PAIRS_FOLD : SMALL_PAIRS_SUM);
+  const unsigned g = one ? 1u : grid_for(4 * q);
+  DevBuf parts(one ? 0 : (size_t)g * NS * D * 8, s);
   {
-    ProfScope prof(kernel_name(FOLD ? (NS ? "k_sc_pair_fold" : "k_fold4") : "k_sc_pair", Ds, D), s,
+    ProfScope prof(kernel_name(FOLD ? "k_sc_pair_fold" : "k_sc_pair", Ds, D), s,
                    FOLD ? 8.0 * ((Ds + D) * 4.0 * L + 2.0 * D * L) : 8.0 * (Ds + D) * (double)L);
-    const bool direct = NS > 0 && g == 1;  // one block stores the sums itself
-    k_sc_pair<Ds, D, FOLD, NS, VIEW><<<g, RT, 0, s>>>(a_in, a_out, b, L, w1, w2,
-                                                      direct ? out : parts.as<uint64_t>(),
-                                                      direct ? mailbox_take(out) : MailboxSig{}, v);
+    // one block stores the sums itself
+    k_sc_pair<Ds, D, FOLD, NS><<<g, one ? reduce_threads(4 * q) : RT, 0, s>>>(
+        a_in, a_out, b, L, host_fold4<D>(r1, r2), one ? out : parts.as<uint64_t>(),
+        one ? mailbox_take(out) : MailboxSig{});
     WHIR_HIP(hipGetLastError());
   }
-  if constexpr (NS > 0) {
-    if (g > 1) finish_reduce<D, NS>(parts.as<uint64_t>(), g, out, s);
-  }
+  if (!one) finish_reduce<D, NS>(parts.as<uint64_t>(), g, out, s);
 }
 
 template <int Ds, int D, bool VIEW>
 static void sc_pair_d(int mode, const uint64_t* a_in, uint64_t* a_out, uint64_t* b, size_t L, const uint64_t* r1,
                       const uint64_t* r2, uint64_t* out, const CovView& v, hipStream_t s) {
-  switch (mode) {
-    case 0: sc_pair_t<Ds, D, false, 8, VIEW>(a_in, a_out, b, L, r1, r2, out, v, s); return;
-    case 1: sc_pair_t<Ds, D, true, 8, VIEW>(a_in, a_out, b, L, r1, r2, out, v, s); return;
-    case 2: sc_pair_t<Ds, D, true, 2, VIEW>(a_in, a_out, b, L, r1, r2, out, v, s); return;
-    default: sc_pair_t<Ds, D, true, 0, VIEW>(a_in, a_out, b, L, r1, r2, out, v, s); return;
+  if constexpr (VIEW) {  // the double fold is the only pass that takes a view here
+    fold4_t<Ds, D, true>(a_in, a_out, b, L, r1, r2, v, s);
+  } else {
+    switch (mode) {
+      case 0: sc_pair_t<Ds, D, false, 8>(a_in, a_out, b, L, r1, r2, out, s); return;
+      case 1: sc_pair_t<Ds, D, true, 8>(a_in, a_out, b, L, r1, r2, out, s); return;
+      case 2: sc_pair_t<Ds, D, true, 2>(a_in, a_out, b, L, r1, r2, out, s); return;
+      default: fold4_t<Ds, D, false>(a_in, a_out, b, L, r1, r2, v, s); return;
+    }
   }
 }
 
@@ -696,11 +724,15 @@ void sumcheck_pair_dev(int mode, int Ds, int D, const uint64_t* a_in, uint64_t* 
 constexpr int VIEW_MAX_TERMS = 4;
 
 template <int Ds, int D, bool FOLD, int NT>
-__global__ __launch_bounds__(RT) void k_view_pass(const uint64_t* a_in, uint64_t* a_out, size_t L, Ext<D> r1,
-                                                  Ext<D> r2, CovView v, uint64_t* parts) {
+__global__ __launch_bounds__(RT) void k_view_pass(const uint64_t* a_in, uint64_t* a_out, size_t L, Fold4<D> f,
+                                                  CovView v, uint64_t* parts) {
   const size_t q = L >> 2, B = (size_t)1 << v.sh, Qb = q >> v.sh;
   const size_t a = blockIdx.x / Qb, h = blockIdx.x % Qb;
   const size_t base = a * q + h * B;
+  // thread 4 t + b ends with term t of quarter b: its high-table factor is read here
+  const unsigned et = threadIdx.x >> 2, eb = threadIdx.x & 3;
+  Ext<D> hi = gl::ext_zero<D>();
+  if (et < NT) hi = ld<D>(v.hi, (size_t)et * v.nhi + eb * Qb + h);
   Ext<D> P[NT];
   if constexpr (!FOLD && Ds == 1) {
     gl::Wide W[NT][D];
@@ -737,7 +769,7 @@ __global__ __launch_bounds__(RT) void k_view_pass(const uint64_t* a_in, uint64_t
       for (int t = 0; t < NT; t++) lo[t] = ld<D>(v.lo, ((size_t)t << v.sh) + l);
       Ext<D> x;
       if constexpr (FOLD) {
-        x = fold_twice<Ds, D>(a_in, p, L, r1, r2);
+        x = fold_twice<Ds, D>(a_in, p, L, f);
         st<D>(a_out, p, x);
       } else {
         x = ldx<Ds, D>(a_in, p);
@@ -748,69 +780,53 @@ __global__ __launch_bounds__(RT) void k_view_pass(const uint64_t* a_in, uint64_t
 #pragma unroll
     for (int t = 0; t < NT; t++) P[t] = gl::ext_reduce<D>(W[t]);
   }
-  block_sum<D, NT>(P);
-  if (threadIdx.x == 0) {
+  __shared__ uint64_t tot[NT * D];
+  block_role_sum<D, NT, 1>(P, tot);
+  if (threadIdx.x < 16) {
+    Ext<D> g = gl::ext_zero<D>();
+    if (et < NT) {
+      Ext<D> x;
 #pragma unroll
-    for (int b = 0; b < 4; b++) {
-      Ext<D> g = gl::ext_zero<D>();
-#pragma unroll
-      for (int t = 0; t < NT; t++) g = gl::eadd<D>(g, gl::emul<D>(ld<D>(v.hi, (size_t)t * v.nhi + b * Qb + h), P[t]));
-      st<D>(parts, (size_t)blockIdx.x * 4 + b, g);
+      for (int d = 0; d < D; d++) x.c[d] = tot[et * D + d];
+      g = gl::emul<D>(hi, x);
     }
+    if constexpr (NT > 1)
+#pragma unroll 1
+      for (int off = 4; off < 16; off <<= 1)
+#pragma unroll
+        for (int d = 0; d < D; d++) g.c[d] = gl::add(g.c[d], (uint64_t)__shfl_xor(g.c[d], off));
+    if (threadIdx.x < 4) st<D>(parts, (size_t)blockIdx.x * 4 + eb, g);
   }
 }
 
-// Sums the blocks' G contributions and writes the pass's NS sums, the same values the
-// pairs kernel's accumulators hold (see k_sc_pair: quarters 0..3 of x and y, dx0 = x2 - x0,
-// dx1 = x3 - x1, ux = x1 - x0, vx = dx1 - dx0, likewise for y).
+// Sums the blocks' G contributions and writes the pass's NS sums, through the eight
+// products of the pairs kernel's quads: each is sum_ab c_a c_b G[a][b] for a vector c of
+// 0, 1 and -1 over the quarters.  Thread 16 p + 4 a + b sums G[a][b] over every p-th h.
 template <int D, int NS>
-__global__ __launch_bounds__(RT) void k_view_reduce(const uint64_t* parts, size_t Qb, uint64_t* out, MailboxSig sig) {
-  Ext<D> G[16];
+__global__ __launch_bounds__(1024) void k_view_reduce(const uint64_t* parts, size_t Qb, uint64_t* out,
+                                                      MailboxSig sig) {
+  __shared__ uint64_t G[16 * D], prod[9 * D];
+  const unsigned a = (threadIdx.x >> 2) & 3, b = threadIdx.x & 3, e = threadIdx.x;
+  Ext<D> v[1] = {gl::ext_zero<D>()};
+  for (size_t h = threadIdx.x >> 4; h < Qb; h += blockDim.x >> 4)
+    v[0] = gl::eadd<D>(v[0], ld<D>(parts, (a * Qb + h) * 4 + b));
+  block_role_sum<D, 1, 16>(v, G);
+  // c of products P0, Q0, P1, Q1, P2, Q2, P3, Q3 (slot order): the quarters with +1 and
+  // those with -1, four bits each
+  if (e < 9 * D) {
+    const unsigned slot = e / D, d = e % D, sh = 4 * (slot & 7);
+    const unsigned pos = slot < 8 ? (0x29848241u >> sh) & 15 : 0, neg = slot < 8 ? (0x16402010u >> sh) & 15 : 0;
+    uint64_t r = 0;
 #pragma unroll
-  for (int k = 0; k < 16; k++) G[k] = gl::ext_zero<D>();
-#pragma unroll
-  for (int a = 0; a < 4; a++)
-    for (size_t h = threadIdx.x; h < Qb; h += blockDim.x)
-#pragma unroll
-      for (int b = 0; b < 4; b++) G[a * 4 + b] = gl::eadd<D>(G[a * 4 + b], ld<D>(parts, (a * Qb + h) * 4 + b));
-  Ext<D> T[16];
-  block_sum_lds<D, 16>(G, T);
-  // Thread k < NS forms sum k = B(al1, be1) + B(al2, be2) from the totals, all threads on
-  // one code path: the coefficient of G[a][b] is al1_a be1_b + al2_a be2_b (in -2..2).
-  __shared__ uint64_t res[8 * D];
-  if (threadIdx.x < NS) {
-    // al1, be1, al2, be2 per sum (coefficient vectors over the quarters 0..3)
-    constexpr int V[8][4][4] = {
-        {{1, 0, 0, 0}, {1, 0, 0, 0}, {0, 1, 0, 0}, {0, 1, 0, 0}},          // x0 y0 + x1 y1
-        {{-1, 0, 1, 0}, {-1, 0, 1, 0}, {0, -1, 0, 1}, {0, -1, 0, 1}},      // dx0 dy0 + dx1 dy1
-        {{1, 0, 0, 0}, {1, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}},          // x0 y0
-        {{1, 0, 0, 0}, {-1, 0, 1, 0}, {-1, 0, 1, 0}, {1, 0, 0, 0}},        // x0 dy0 + dx0 y0
-        {{-1, 0, 1, 0}, {-1, 0, 1, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}},        // dx0 dy0
-        {{-1, 1, 0, 0}, {-1, 1, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}},        // ux uy
-        {{-1, 1, 0, 0}, {1, -1, -1, 1}, {1, -1, -1, 1}, {-1, 1, 0, 0}},    // ux vy + vx uy
-        {{1, -1, -1, 1}, {1, -1, -1, 1}, {0, 0, 0, 0}, {0, 0, 0, 0}}};     // vx vy
-    const int k = threadIdx.x;
-    Ext<D> r = gl::ext_zero<D>();
-#pragma unroll
-    for (int a = 0; a < 4; a++)
-#pragma unroll
-      for (int b = 0; b < 4; b++) {
-        const int c = V[k][0][a] * V[k][1][b] + V[k][2][a] * V[k][3][b];
-        const Ext<D>& t = T[a * 4 + b];
-        const Ext<D> z = gl::ext_zero<D>();
-        r = gl::eadd<D>(r, c > 0 ? t : z);
-        r = gl::esub<D>(r, c < 0 ? t : z);
-        r = gl::eadd<D>(r, c > 1 ? t : z);
-        r = gl::esub<D>(r, c < -1 ? t : z);
-      }
-#pragma unroll
-    for (int d = 0; d < D; d++) res[k * D + d] = r.c[d];
+    for (int i = 0; i < 16; i++) {
+      const unsigned pa = pos >> (i >> 2) & 1, na = neg >> (i >> 2) & 1, pb = pos >> (i & 3) & 1, nb = neg >> (i & 3) & 1;
+      const uint64_t x = (pa | na) & (pb | nb) ? G[i * D + d] : 0;
+      r = (pa ^ pb) & 1 ? gl::sub(r, x) : gl::add(r, x);
+    }
+    prod[e] = r;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int k = 0; k < NS * D; k++) out[k] = res[k];
-    mailbox_raise(sig);
-  }
+  store_words<NS * D>(e < NS * D ? pair_sum_word<D>(prod, e) : 0, out, sig);
 }
 
 template <int Ds, int D>
@@ -819,15 +835,15 @@ static void view_pass_t(int mode, const uint64_t* a_in, uint64_t* a_out, size_t 
   const size_t Qb = (L >> 2) >> v.sh;
   const unsigned blocks = (unsigned)(4 * Qb);
   DevBuf parts((size_t)blocks * 4 * D * 8, s);
-  const Ext<D> w1 = r1 ? host_ext<D>(r1) : gl::ext_zero<D>(), w2 = r2 ? host_ext<D>(r2) : gl::ext_zero<D>();
+  const Fold4<D> f = host_fold4<D>(r1, r2);
   {
     ProfScope prof(kernel_name(mode ? "k_view_pass_fold" : "k_view_pass", Ds, D), s,
                    mode ? 8.0 * (Ds * 4.0 * L + D * (double)L) : 8.0 * Ds * (double)L);
     uint64_t* pp = parts.as<uint64_t>();
     auto go = [&](auto nt) {
       constexpr int NT = decltype(nt)::value;
-      if (mode == 0) k_view_pass<Ds, D, false, NT><<<blocks, RT, 0, s>>>(a_in, a_out, L, w1, w2, v, pp);
-      else k_view_pass<Ds, D, true, NT><<<blocks, RT, 0, s>>>(a_in, a_out, L, w1, w2, v, pp);
+      if (mode == 0) k_view_pass<Ds, D, false, NT><<<blocks, RT, 0, s>>>(a_in, a_out, L, f, v, pp);
+      else k_view_pass<Ds, D, true, NT><<<blocks, RT, 0, s>>>(a_in, a_out, L, f, v, pp);
     };
     switch (v.nt) {
       case 1: go(std::integral_constant<int, 1>{}); break;
@@ -837,8 +853,8 @@ static void view_pass_t(int mode, const uint64_t* a_in, uint64_t* a_out, size_t 
     }
     WHIR_HIP(hipGetLastError());
   }
-  if (mode == 2) k_view_reduce<D, 2><<<1, RT, 0, s>>>(parts.as<uint64_t>(), Qb, out, mailbox_take(out));
-  else k_view_reduce<D, 8><<<1, RT, 0, s>>>(parts.as<uint64_t>(), Qb, out, mailbox_take(out));
+  if (mode == 2) k_view_reduce<D, 2><<<1, reduce_threads(16 * Qb), 0, s>>>(parts.as<uint64_t>(), Qb, out, mailbox_take(out));
+  else k_view_reduce<D, 8><<<1, reduce_threads(16 * Qb), 0, s>>>(parts.as<uint64_t>(), Qb, out, mailbox_take(out));
   WHIR_HIP(hipGetLastError());
 }
 
@@ -1451,12 +1467,12 @@ CovView covview_build_dev(int D, uint64_t* buf, size_t nv, const uint64_t* eq_po
 }
 
 template <int D>
-__global__ void k_covview_fold2(const uint64_t* hi, uint64_t* out, size_t nt, size_t nhi, Ext<D> r1, Ext<D> r2) {
+__global__ void k_covview_fold2(const uint64_t* hi, uint64_t* out, size_t nt, size_t nhi, Fold4<D> f) {
   const size_t q = nhi >> 2;
   const size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
   if (e >= nt * q) return;
   const size_t k = e / q, t = e % q;
-  st<D>(out, e, fold_twice<D, D>(hi + k * nhi * D, t, q, r1, r2));
+  st<D>(out, e, fold_twice<D, D>(hi + k * nhi * D, t, q, f));
 }
 
 template <int D>
@@ -1470,9 +1486,9 @@ CovView covview_fold2_dev(int D, const CovView& v, const uint64_t* r1, const uin
   WHIR_REQUIRE(v.nt > 0 && v.nhi >= 4, "covector view: nothing left to fold in the high tables");
   const size_t n = (size_t)v.nt * (v.nhi >> 2);
   switch (D) {
-    case 1: k_covview_fold2<1><<<blocks_for(n, RT), RT, 0, s>>>(v.hi, out_hi, v.nt, v.nhi, host_ext<1>(r1), host_ext<1>(r2)); break;
-    case 2: k_covview_fold2<2><<<blocks_for(n, RT), RT, 0, s>>>(v.hi, out_hi, v.nt, v.nhi, host_ext<2>(r1), host_ext<2>(r2)); break;
-    case 3: k_covview_fold2<3><<<blocks_for(n, RT), RT, 0, s>>>(v.hi, out_hi, v.nt, v.nhi, host_ext<3>(r1), host_ext<3>(r2)); break;
+    case 1: k_covview_fold2<1><<<blocks_for(n, RT), RT, 0, s>>>(v.hi, out_hi, v.nt, v.nhi, host_fold4<1>(r1, r2)); break;
+    case 2: k_covview_fold2<2><<<blocks_for(n, RT), RT, 0, s>>>(v.hi, out_hi, v.nt, v.nhi, host_fold4<2>(r1, r2)); break;
+    case 3: k_covview_fold2<3><<<blocks_for(n, RT), RT, 0, s>>>(v.hi, out_hi, v.nt, v.nhi, host_fold4<3>(r1, r2)); break;
     default: throw Error("covector view: extension degree must be 1, 2 or 3");
   }
   WHIR_HIP(hipGetLastError());
