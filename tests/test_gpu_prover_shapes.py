@@ -4,6 +4,9 @@ import numpy as np
 import pytest
 
 import whir_amd as W
+from oracle import oracle as O
+from test_gpu_batch import case, gpu_batch, oracle_batch
+from test_gpu_kernels import rnd_np
 from test_gpu_prover import gpu_proof, make_case, oracle_proof
 
 pytestmark = pytest.mark.gpu
@@ -34,3 +37,25 @@ def test_stir_terms_over_short_and_long_vectors(nv, D, lir, sec):
                                        (15, 3, 4, 3), (16, 2, 5, 6), (18, 1, 4, 7), (18, 3, 6, 4)])
 def test_sumcheck_pairs(nv, D, k0, k):
     check(nv, D, W.HASH_BLAKE3, k0, k, 1, 2, 40 if D == 1 else 80)
+
+
+# Univariate evaluation: one block of 64 to 1024 threads, several blocks of 1024 elements, and
+# segments of 2048 in several turns; lengths at and beside the edges.
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 255, 256, 257, 1000, 1024, 4095, 4096, 4097, 5121, 2**15 + 1,
+                               2**20, 2**20 + 1, 2**22 + 2049])
+@pytest.mark.parametrize("D,ext", [(1, False), (2, False), (2, True), (3, False), (3, True)])
+def test_univariate_evaluate_lengths(n, D, ext):
+    Ds = D if ext else 1
+    c, x = rnd_np(n + D, n * Ds), rnd_np(n + 12, D)
+    assert np.array_equal(W.mixed_univariate_evaluate(Ds, D, c, x), O.univariate_evaluate(Ds, D, c, x))
+
+
+# Several vectors at several points share launches: one to sixteen vectors (up to four points
+# each), above and below one block per vector, and more points than a launch takes.
+@pytest.mark.parametrize("nv,D,B,NW", [(8, 2, 3, 1), (10, 1, 4, 2), (13, 1, 5, 2), (13, 2, 1, 5), (14, 3, 3, 3),
+                                       (12, 2, 17, 1)])
+def test_out_of_domain_values_of_batches(nv, D, B, NW):
+    vecs, points, params, pid, sid = case(nv, D, W.HASH_BLAKE3, 4, 4, 1, B, NW, 1)
+    _, _, narg, hints, _ = oracle_batch(nv, D, B, NW, vecs, points, params, pid, sid)
+    _, gnarg, ghints, _ = gpu_batch(nv, D, B, NW, vecs, points, params, pid, sid)
+    assert gnarg == narg and ghints == hints

@@ -106,12 +106,11 @@ void covector_stir_dev(int D, uint64_t* acc, size_t n, bool accumulate, const ui
                        const uint64_t* ext_points, size_t m_e, const uint64_t* exps, const uint64_t* points, size_t m_b,
                        int logN, hipStream_t st);
 
-// mixed_univariate_evaluate at m host points x[0..m) in shared passes; results to
-// dev_out[0..m D).
-// padded: dev_out has room for m rounded up to a multiple of 4 values (the kernel
-// then writes its whole groups there directly).
-void univariate_eval_many_dev(int Ds, int D, const uint64_t* coeffs, size_t n, const uint64_t* x, size_t m,
-                              uint64_t* dev_out, hipStream_t st, bool padded = false);
+// mixed_univariate_evaluate of count vectors of n elements (vecs: host array of device
+// pointers) at m host points x[0..m) in shared passes: vector z's value at x_j goes to
+// dev_out[(z m + j) D ..].
+void univariate_eval_many_dev(int Ds, int D, const uint64_t* const* vecs, size_t count, size_t n, const uint64_t* x,
+                              size_t m, uint64_t* dev_out, hipStream_t st);
 
 // mixed_univariate_evaluate of many base-field vectors, each at its own degree-D
 // point, in shared launches: out[e*D .. (e+1)*D) = sum_i jobs[e].coeffs[i] x_e^i.

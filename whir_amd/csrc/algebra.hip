@@ -1543,210 +1543,251 @@ void geometric_accumulate_dev(int D, uint64_t* acc, size_t n, const uint64_t* sc
 }
 
 // ------------------------------------------------------------------ univariate evaluation
-// mixed_univariate_evaluate (src/algebra/mod.rs:105-129) at up to UNI_MP points per
-// pass: f(x_j) = sum_b x_j^(b S) sum_{q < S} c_(b S + q) x_j^q, S = RT UNI_K.  Block
-// b sums its segment against the power table P[j][q] = x_j^q (one base-by-extension
-// or extension product per element and point, no chained step); the final kernel
-// scales block partials by B[j][b] = x_j^(b S) and adds them.
-static constexpr int UNI_K = 16;
-static constexpr int UNI_MP = 4;
+// mixed_univariate_evaluate (src/algebra/mod.rs:105-129) of several vectors at several
+// points.  A block of T <= 256 threads takes G segments of T K elements; thread t holds
+//   a_t = sum_k c_(k T + t) x^(k T)   over all its k, by Horner's rule in x^(T K) over the
+// segments, and within a segment against the powers x^(k T), k < K, which are the same for
+// every thread and come with the launch (through LDS: the arguments are read in one go
+// while the elements are on their way).  A segment's products and the Horner step are
+// summed unreduced and reduced once.  Then one wave forms sum_t a_t x^t: Horner's rule in
+// x^64 over the waves, and a tree of lo + x^(2^i) hi over its lanes, so no thread makes a
+// power of its own; the block's sum times x^(first element) is its part.  A short vector
+// waits for the code as much as for the arithmetic, so the loops stay loops: 4 KB against
+// 27 KB of a lane that steps its own power through sixteen unrolled elements.
+static constexpr int UNI_MP = 4;   // points per launch
+static constexpr int UNI_MV = 16;  // vectors per launch, times points (both rounded up to a power of two)
+static constexpr int UNI_PW = 32;  // squares x^(2^b): vectors of less than 2^32 elements
+static constexpr int UNI_K = 16;   // elements per thread of a segment of k_uni_many
 
-struct UniPlan {
-  size_t m, nb, S;
-  size_t P, B, words, entries;
-  uint64_t x[UNI_MP * 3];  // the points (m x D words), passed with the launch
+// Per point: the squares x^(2^b), then the powers x^(k T).  MP points (at most 3.6 KB, 0.7 to
+// 1.1 KB for the usual single point: the launch copies them).
+template <int D, int K, int MP>
+struct UniArgs {
+  static constexpr int POINT = (UNI_PW + K) * D;
+  const uint64_t* c[UNI_MV];
+  uint64_t w[MP * POINT];
 };
-
-// x_j^(2^b) for b < UNI_PW, computed on the host and passed with the launch: a table
-// entry x_j^e is then the product over the set bits of e, one multiply per set bit
-// instead of a squaring and a multiply per bit (the table launch runs one short wave
-// per SIMD, so its time is its instruction count).
-static constexpr int UNI_PW = 32;
-struct UniPow {
-  uint64_t w[UNI_MP * UNI_PW * 3];
+struct UniGrid {
+  size_t n, G;
+  int lt;      // T = 2^lt threads, 64 <= T <= 256
+  int nv, m;   // slots per vector (points rounded up to a power of two), points
+  int rows;    // slots per block of parts (vectors rounded up, times nv)
 };
 
 template <int D>
-__global__ void k_uni_tables(uint64_t* buf, UniPlan L, UniPow pw) {
-  const size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-  if (e >= L.entries) return;
-  const bool in_p = e < L.m * L.S;
-  const size_t j = in_p ? e / L.S : (e - L.m * L.S) / L.nb;
-  uint64_t ex = in_p ? e % L.S : (uint64_t)((e - L.m * L.S) % L.nb) * L.S;
-  Ext<D> r = gl::ext_base<D>(1);
-  for (int b = 0; ex; b++, ex >>= 1) {
-    if (ex & 1) {
-      Ext<D> p;
+__device__ __forceinline__ Ext<D> uni_arg(const uint64_t* w, int i) {
+  Ext<D> r;
 #pragma unroll
-      for (int d = 0; d < D; d++) p.c[d] = pw.w[(j * UNI_PW + b) * D + d];
-      r = gl::emul<D>(r, p);
-    }
-  }
-  if (in_p) st<D>(buf + L.P, e, r);
-  else st<D>(buf + L.B, e - L.m * L.S, r);
+  for (int d = 0; d < D; d++) r.c[d] = w[i * D + d];
+  return r;
 }
 
-template <int Ds, int D>
-__global__ __launch_bounds__(RT) void k_uni(const uint64_t* c, size_t n, const uint64_t* buf, UniPlan L, int m,
-                                            uint64_t* parts) {
-  const size_t b = blockIdx.x;
-  const size_t i0 = b * L.S + threadIdx.x;
-  Ext<D> acc[UNI_MP];
+// Blocks z take a vector, blocks y a slot.  rows == 0: the block is the only one and stores
+// its points' values to parts in order (sig).
+template <int Ds, int D, int K, int MP>
+__global__ __launch_bounds__(RT) void k_uni(UniArgs<D, K, MP> A, UniGrid U, uint64_t* parts, MailboxSig sig) {
+  constexpr int POINT = (UNI_PW + K) * D;
+  static_assert(K == 4 || K == 8, "k_uni: the step x^(T K) is one of the squares");
+  __shared__ uint64_t arg[POINT], sum[RT * D], first[D];
+  const uint64_t* c = A.c[blockIdx.z];
+  const unsigned T = blockDim.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = T >> 6;
+  const size_t S = (size_t)T * K, base = blockIdx.x * U.G * S;
+  const int step_bit = U.lt + (K == 4 ? 2 : 3);
+#pragma unroll 1
+  for (int j = blockIdx.y; j < U.nv; j += gridDim.y) {
+    Ext<Ds> cv[K];
+    auto load = [&](size_t g) {
+      const size_t i0 = base + g * S + threadIdx.x;
 #pragma unroll
-  for (int j = 0; j < UNI_MP; j++) acc[j] = gl::ext_zero<D>();
-#pragma unroll
-  for (int k = 0; k < UNI_K; k++) {
-    const size_t i = i0 + (size_t)k * RT;
-    if (i >= n) break;
-    const size_t q = (size_t)k * RT + threadIdx.x;
-#pragma unroll
-    for (int j = 0; j < UNI_MP; j++) {
-      if (j < m) {
-        const Ext<D> pw = ld<D>(buf + L.P, j * L.S + q);
-        if constexpr (Ds == 1) acc[j] = gl::eadd<D>(acc[j], gl::escale<D>(pw, c[i]));
-        else acc[j] = gl::eadd<D>(acc[j], gl::emul<D>(pw, ld<D>(c, i)));
+      for (int k = 0; k < K; k++) {
+        const size_t i = i0 + (size_t)k * T;
+        cv[k] = i < U.n ? ld<Ds>(c, i) : gl::ext_zero<Ds>();
       }
+    };
+    load(U.G - 1);
+#pragma unroll 1
+    for (int i = threadIdx.x; i < POINT; i += T) arg[i] = A.w[j * POINT + i];
+    __syncthreads();
+    Ext<D> acc = gl::ext_zero<D>();
+    // many segments: scalar registers hold the factors best (the loop's factors in vector
+    // registers halve the waves per SIMD)
+    const uint64_t* aj = K == 4 ? arg : A.w + j * POINT;
+#pragma unroll 1
+    for (size_t g = U.G;;) {
+      gl::Wide w[D];
+      gl::wide_zero<D>(w);
+#pragma unroll
+      for (int d = 0; d < Ds; d++) w[d].lo = cv[0].c[d];
+      if (g != U.G) gl::emul_acc<D>(w, acc, uni_arg<D>(aj, step_bit));
+#pragma unroll
+      for (int k = 1; k < K; k++) {
+        const Ext<D> p = uni_arg<D>(aj, UNI_PW + k);
+        if constexpr (Ds == D) {
+          gl::emul_acc<D>(w, cv[k], p);
+        } else {
+#pragma unroll
+          for (int d = 0; d < D; d++) gl::wide_mac(w[d], cv[k].c[0], p.c[d]);
+        }
+      }
+      acc = gl::ext_reduce<D>(w);
+      if (--g == 0) break;
+      load(g - 1);
+    }
+    st<D>(sum, threadIdx.x, acc);
+    __syncthreads();
+    // wave 0 sums the threads' values while wave 1 forms x^base (several blocks: T = 256)
+    if (base && wave == 1) {
+      Ext<D> f = gl::ext_base<D>(1);
+#pragma unroll 1
+      for (size_t e = base; e; e &= e - 1) f = gl::emul<D>(f, uni_arg<D>(arg, __builtin_ctzll(e)));
+      if (lane == 0) st<D>(first, 0, f);
+    }
+    Ext<D> v = gl::ext_zero<D>();
+    if (wave == 0) {
+#pragma unroll 1
+      for (int w = waves - 1; w >= 0; w--)
+        v = gl::eadd<D>(ld<D>(sum, w * 64 + lane), gl::emul<D>(v, uni_arg<D>(arg, 6)));
+#pragma unroll 1
+      for (int bit = 5; bit >= 0; bit--) {
+        Ext<D> hi;
+#pragma unroll
+        for (int d = 0; d < D; d++) hi.c[d] = __shfl_xor(v.c[d], 1 << bit);
+        v = gl::eadd<D>(v, gl::emul<D>(hi, uni_arg<D>(arg, bit)));  // right in lanes below 2^bit
+      }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      if (base) v = gl::emul<D>(v, ld<D>(first, 0));
+      if (j >= U.m) v = gl::ext_zero<D>();
+      if (U.rows > 0) st<D>(parts, blockIdx.x * (size_t)U.rows + (size_t)blockIdx.z * U.nv + j, v);
+      else if (j < U.m) st<D>(parts, j, v);
     }
   }
-#pragma unroll
-  for (int j = 0; j < UNI_MP; j++)
-    if (j < m) acc[j] = gl::emul<D>(acc[j], ld<D>(buf + L.B, j * L.nb + b));  // segment offset x_j^(b S)
-  block_reduce_store<D, UNI_MP>(acc, parts + (size_t)blockIdx.x * UNI_MP * D);
+  if (sig.flag && threadIdx.x == 0) mailbox_raise(sig);  // the thread that stored the values
 }
 
-// Vectors of at most UNI_SMALL_BLOCKS blocks skip the table launch: each thread forms
-// x_j^(i0) (its first index) by square-and-multiply from the squares x_j^(2^k) passed
-// with the launch, then steps by x_j^RT; one block stores its sums itself.
-static constexpr size_t UNI_SMALL_BLOCKS = 256;
-
-template <int Ds, int D, int MP>
-__global__ __launch_bounds__(RT) void k_uni_small(const uint64_t* c, size_t n, UniPow pw, uint64_t* parts,
-                                                  MailboxSig sig) {
-  static_assert(RT == 256, "the step x^RT is the square x^(2^8)");
-  const size_t i0 = blockIdx.x * (size_t)RT * UNI_K + threadIdx.x;
-  // Per point: x_j^i0 by square-and-multiply, then the lane's elements in order.  The
-  // elements are loaded a chunk at a time before the chunk's arithmetic (zero past the
-  // end), so a chunk's loads are in flight together rather than one per step of the
-  // power chain; Fp3 takes chunks of four (sixteen unrolled Fp3 steps do not fit the
-  // registers).
-  constexpr int UC = D == 3 ? 4 : UNI_K;
-  Ext<D> acc[UNI_MP];
-#pragma unroll
-  for (int j = 0; j < UNI_MP; j++) acc[j] = gl::ext_zero<D>();
-  if (i0 < n) {
-    static_for<MP>([&](auto jc) {
-      constexpr int j = decltype(jc)::value;
-      Ext<D> p = gl::ext_base<D>(1);
-      for (int bit = 0; (i0 >> bit) != 0; bit++)
-        if ((i0 >> bit) & 1) {
-          Ext<D> sq;
-#pragma unroll
-          for (int d = 0; d < D; d++) sq.c[d] = pw.w[(j * UNI_PW + bit) * D + d];
-          p = gl::emul<D>(p, sq);
-        }
-      Ext<D> step;
-#pragma unroll
-      for (int d = 0; d < D; d++) step.c[d] = pw.w[(j * UNI_PW + 8) * D + d];
-      for (int k0 = 0; k0 < UNI_K; k0 += UC) {
-        Ext<Ds> cv[UC];
-#pragma unroll
-        for (int k = 0; k < UC; k++) {
-          const size_t i = i0 + (size_t)(k0 + k) * RT;
-          cv[k] = i < n ? ldx<Ds, Ds>(c, i) : gl::ext_zero<Ds>();
-        }
-#pragma unroll
-        for (int k = 0; k < UC; k++) {
-          if constexpr (Ds == 1) acc[j] = gl::eadd<D>(acc[j], gl::escale<D>(p, cv[k].c[0]));
-          else acc[j] = gl::eadd<D>(acc[j], gl::emul<D>(p, cv[k]));
-          p = gl::emul<D>(p, step);
-        }
-      }
-    });
+// The vectors' values from the blocks' parts (R slots per block, nv per vector): value j of
+// vector z goes to out[z ms + j].
+template <int D, int R>
+__global__ __launch_bounds__(1024) void k_uni_reduce(const uint64_t* parts, size_t nparts, int nv, int m, int ms,
+                                                     int count, uint64_t* out, MailboxSig sig) {
+  __shared__ uint64_t tot[R * D];
+  Ext<D> v[1] = {gl::ext_zero<D>()};
+  for (size_t e = threadIdx.x; e < nparts * R; e += blockDim.x)
+    if ((int)(e % R) < nv * count) v[0] = gl::eadd<D>(v[0], ld<D>(parts, e));
+  block_role_sum<D, 1, R>(v, tot);
+  const int r = threadIdx.x / D, z = r / nv, j = r % nv;
+  if (threadIdx.x < R * D && z < count && j < m) out[(z * ms + j) * D + threadIdx.x % D] = tot[threadIdx.x];
+  if (sig.flag) {
+    __syncthreads();  // every word is stored before thread 0 raises the flag
+    if (threadIdx.x == 0) mailbox_raise(sig);
   }
-  block_reduce_store<D, UNI_MP>(acc, parts + (size_t)blockIdx.x * UNI_MP * D, sig);
 }
 
-template <int Ds, int D>
-static void uni_t(const uint64_t* c, size_t n, const uint64_t* xs, size_t m, uint64_t* out, hipStream_t s,
-                  bool padded) {
-  for (size_t j0 = 0; j0 < m; j0 += UNI_MP) {
-    const size_t mj = std::min<size_t>(UNI_MP, m - j0);
-    uint64_t* o = out + j0 * D;
-    if (!n) {
-      fill_zero(o, mj * D * 8, s);
-      continue;
+static int next_pow2_int(int n) {
+  int p = 1;
+  while (p < n) p <<= 1;
+  return p;
+}
+
+// One launch (and its reduction): count vectors at m points, values to out[z ms + j].
+template <int Ds, int D, int K, int MP>
+static void uni_launch(const uint64_t* const* c, int count, size_t n, const uint64_t* xs, int m, uint64_t* out,
+                       int ms, bool last, hipStream_t s) {
+  UniArgs<D, K, MP> A{};
+  UniGrid U{};
+  std::copy(c, c + count, A.c);
+  U.n = n;
+  U.m = m;
+  U.nv = next_pow2_int(m);
+  U.lt = 8;
+  if (K == 4)
+    while (U.lt > 6 && n <= ((size_t)K << (U.lt - 1))) U.lt--;
+  const size_t S = (size_t)K << U.lt, segs = (n + S - 1) / S;
+  U.G = (segs + MAX_BLOCKS - 1) / MAX_BLOCKS;
+  const size_t nb = (segs + U.G - 1) / U.G;
+  WHIR_REQUIRE((uint64_t)(nb - 1) * U.G * ((uint64_t)K << U.lt) < ((uint64_t)1 << UNI_PW), "univariate: vector too long");
+  for (int j = 0; j < m; j++) {
+    Ext<D> p, k = gl::ext_base<D>(1);
+    for (int d = 0; d < D; d++) p.c[d] = xs[j * D + d];
+    Ext<D> xt = k;
+    for (int b = 0; b < UNI_PW; b++) {
+      std::copy(p.c, p.c + D, &A.w[j * A.POINT + b * D]);
+      if (b == U.lt) xt = p;
+      p = gl::emul<D>(p, p);
     }
-    UniPlan L{};
-    L.m = mj;
-    L.S = (size_t)RT * UNI_K;
-    L.nb = (n + L.S - 1) / L.S;
-    std::copy(xs + j0 * D, xs + (j0 + mj) * D, L.x);
-    L.P = 0;
-    L.B = L.P + mj * L.S * D;
-    L.words = L.B + mj * L.nb * D;
-    L.entries = mj * (L.S + L.nb);
-    const bool small = L.nb <= UNI_SMALL_BLOCKS;
-    DevBuf buf(small ? 0 : L.words * 8, s), parts(L.nb > 1 ? L.nb * UNI_MP * D * 8 : 0, s),
-        res((mj == UNI_MP || padded) ? 0 : UNI_MP * D * 8, s);
-    WHIR_REQUIRE((uint64_t)(L.nb - 1) * L.S < ((uint64_t)1 << UNI_PW), "univariate: vector too long");
-    UniPow pw;
-    for (size_t j = 0; j < mj; j++) {
-      Ext<D> p;
-      for (int d = 0; d < D; d++) p.c[d] = xs[(j0 + j) * D + d];
-      for (int b = 0; b < UNI_PW; b++) {
-        for (int d = 0; d < D; d++) pw.w[(j * UNI_PW + b) * D + d] = p.c[d];
-        p = gl::emul<D>(p, p);
-      }
-    }
-    // The reduction writes all UNI_MP slots; only the first mj go to the caller
-    // (straight into `out` when it has room for whole groups).
-    uint64_t* dst = (mj == UNI_MP || padded) ? o : res.as<uint64_t>();
-    const bool last = j0 + UNI_MP >= m;
-    if (small) {
-      {
-        ProfScope prof(kernel_name("k_uni_small", Ds, D), s, 8.0 * Ds * (double)n);
-        uint64_t* o_small = L.nb == 1 ? dst : parts.as<uint64_t>();
-        const MailboxSig sig = L.nb == 1 && last ? mailbox_take(dst) : MailboxSig{};
-        auto go = [&](auto mp) {
-          k_uni_small<Ds, D, decltype(mp)::value><<<(unsigned)L.nb, RT, 0, s>>>(c, n, pw, o_small, sig);
-        };
-        switch (mj) {
-          case 1: go(std::integral_constant<int, 1>{}); break;
-          case 2: go(std::integral_constant<int, 2>{}); break;
-          case 3: go(std::integral_constant<int, 3>{}); break;
-          default: go(std::integral_constant<int, 4>{}); break;
-        }
-        WHIR_HIP(hipGetLastError());
-      }
-      if (L.nb > 1) finish_reduce<D, UNI_MP>(parts.as<uint64_t>(), (unsigned)L.nb, dst, s, last);
-      if (dst != o) WHIR_HIP(hipMemcpyAsync(o, dst, mj * D * 8, hipMemcpyDeviceToDevice, s));
-      continue;
-    }
-    k_uni_tables<D><<<blocks_for(L.entries, RT), RT, 0, s>>>(buf.as<uint64_t>(), L, pw);
+    for (int i = 0; i < K; i++, k = gl::emul<D>(k, xt)) std::copy(k.c, k.c + D, &A.w[j * A.POINT + (UNI_PW + i) * D]);
+  }
+  const bool one = nb == 1 && count == 1;
+  U.rows = one ? 0 : next_pow2_int(count) * U.nv;
+  DevBuf parts(one ? 0 : nb * U.rows * D * 8, s);
+  {
+    ProfScope prof(kernel_name("k_uni", Ds, D), s, 8.0 * Ds * (double)n * count);
+    const dim3 grid((unsigned)nb, one ? 1u : (unsigned)U.nv, (unsigned)count);
+    k_uni<Ds, D, K, MP><<<grid, 1u << U.lt, 0, s>>>(A, U, one ? out : parts.as<uint64_t>(),
+                                                   one && last ? mailbox_take(out) : MailboxSig{});
     WHIR_HIP(hipGetLastError());
-    {
-      ProfScope prof(kernel_name("k_uni", Ds, D), s, 8.0 * Ds * (double)n);
-      k_uni<Ds, D><<<(unsigned)L.nb, RT, 0, s>>>(c, n, buf.as<uint64_t>(), L, (int)mj, parts.as<uint64_t>());
-      WHIR_HIP(hipGetLastError());
-    }
-    finish_reduce<D, UNI_MP>(parts.as<uint64_t>(), (unsigned)L.nb, dst, s, last);
-    if (dst != o) WHIR_HIP(hipMemcpyAsync(o, dst, mj * D * 8, hipMemcpyDeviceToDevice, s));
   }
+  if (one) return;
+  const MailboxSig sig = last ? mailbox_take(out) : MailboxSig{};
+  const unsigned th = reduce_threads(nb * U.rows);
+  const uint64_t* pp = parts.as<uint64_t>();
+  switch (U.rows) {
+    case 1: k_uni_reduce<D, 1><<<1, th, 0, s>>>(pp, nb, U.nv, m, ms, count, out, sig); break;
+    case 2: k_uni_reduce<D, 2><<<1, th, 0, s>>>(pp, nb, U.nv, m, ms, count, out, sig); break;
+    case 4: k_uni_reduce<D, 4><<<1, th, 0, s>>>(pp, nb, U.nv, m, ms, count, out, sig); break;
+    case 8: k_uni_reduce<D, 8><<<1, th, 0, s>>>(pp, nb, U.nv, m, ms, count, out, sig); break;
+    default: k_uni_reduce<D, 16><<<1, th, 0, s>>>(pp, nb, U.nv, m, ms, count, out, sig); break;
+  }
+  WHIR_HIP(hipGetLastError());
 }
 
-void univariate_eval_many_dev(int Ds, int D, const uint64_t* c, size_t n, const uint64_t* xs, size_t m,
-                              uint64_t* out, hipStream_t s, bool padded) {
-  if (!m) return;
+// Up to this many elements a segment is 4 per thread, which spreads a short vector over the
+// most CUs; above, 8 per thread halve the Horner steps (2^20 base elements at an Fp2 point on
+// MI355X 13.2 us against 14.1).  2^24 take 42 us (3.2 TB/s; 54 with a table of powers read
+// beside the elements), 2^12 Fp2 7 us (15 with a power chain per lane).
+static constexpr size_t UNI_SHORT = (size_t)1 << 18;
+
+template <int Ds, int D>
+static void uni_t(const uint64_t* const* vecs, size_t count, size_t n, const uint64_t* xs, size_t m, uint64_t* out,
+                  hipStream_t s) {
+  if (!n) {
+    fill_zero(out, count * m * D * 8, s);
+    return;
+  }
+  // Fp3 with K = 8: two points fill the launch's arguments
+  const size_t gm = std::min<size_t>(m, D == 3 && n > UNI_SHORT ? 2 : UNI_MP);
+  const size_t gv = UNI_MV / next_pow2_int((int)gm);
+  for (size_t v = 0; v < count; v += gv)
+    for (size_t j = 0; j < m; j += gm) {
+      const size_t kv = std::min(gv, count - v), kj = std::min(gm, m - j);
+      const bool last = v + kv == count && j + kj == m;
+      uint64_t* o = out + (v * m + j) * D;
+      auto go = [&](auto k, auto mp) {
+        uni_launch<Ds, D, decltype(k)::value, decltype(mp)::value>(vecs + v, (int)kv, n, xs + j * D, (int)kj, o, (int)m,
+                                                                   last, s);
+      };
+      using One = std::integral_constant<int, 1>;
+      using K4 = std::integral_constant<int, 4>;
+      using K8 = std::integral_constant<int, 8>;
+      if (n <= UNI_SHORT) kj == 1 ? go(K4{}, One{}) : go(K4{}, std::integral_constant<int, UNI_MP>{});
+      else kj == 1 ? go(K8{}, One{}) : go(K8{}, std::integral_constant<int, D == 3 ? 2 : UNI_MP>{});
+    }
+}
+
+void univariate_eval_many_dev(int Ds, int D, const uint64_t* const* vecs, size_t count, size_t n, const uint64_t* xs,
+                              size_t m, uint64_t* out, hipStream_t s) {
+  if (!m || !count) return;
   if (Ds == 1) {
     switch (D) {
-      case 1: uni_t<1, 1>(c, n, xs, m, out, s, padded); return;
-      case 2: uni_t<1, 2>(c, n, xs, m, out, s, padded); return;
-      case 3: uni_t<1, 3>(c, n, xs, m, out, s, padded); return;
+      case 1: uni_t<1, 1>(vecs, count, n, xs, m, out, s); return;
+      case 2: uni_t<1, 2>(vecs, count, n, xs, m, out, s); return;
+      case 3: uni_t<1, 3>(vecs, count, n, xs, m, out, s); return;
     }
   } else if (Ds == D) {
     switch (D) {
-      case 2: uni_t<2, 2>(c, n, xs, m, out, s, padded); return;
-      case 3: uni_t<3, 3>(c, n, xs, m, out, s, padded); return;
+      case 2: uni_t<2, 2>(vecs, count, n, xs, m, out, s); return;
+      case 3: uni_t<3, 3>(vecs, count, n, xs, m, out, s); return;
     }
   }
   throw Error("univariate_evaluate: unsupported degrees");
@@ -1898,7 +1939,7 @@ void univariate_eval_batch_dev(int D, const UniJob* jobs, size_t count, uint64_t
 
 void univariate_eval_dev(int Ds, int D, const uint64_t* c, size_t n, const uint64_t* x, uint64_t* out,
                          hipStream_t s) {
-  univariate_eval_many_dev(Ds, D, c, n, x, 1, out, s);
+  univariate_eval_many_dev(Ds, D, &c, 1, n, x, 1, out, s);
 }
 
 // ------------------------------------------------------------------ lift, axpy, dot, gather

@@ -309,20 +309,17 @@ void irs_commit(Transcript& t, const IrsCfg& c, int engine, const uint64_t* cons
       }
     }
   } else if (nood) {
-    // All samples of a vector in shared passes over it, written to the mailbox
-    // (vector b at words [b*pad*D, (b+1)*pad*D)); sent point-major.
+    // All samples of all vectors in shared passes, written to the mailbox (vector b at
+    // words [b*nood*D, (b+1)*nood*D)); sent point-major.
     const size_t pad = (nood + 3) / 4 * 4;
     WHIR_REQUIRE(nvec * pad * D <= RESULT_MAILBOX_WORDS, "too many out-of-domain samples");
-    for (size_t b = 0; b < nvec; b++) {
-      if (b + 1 == nvec) mailbox_arm(s);
-      univariate_eval_many_dev(Ds, D, vecs[b], c.vector_size, w.ood_points.data(), nood, mbox + b * pad * D, s,
-                               true);
-    }
+    mailbox_arm(s);
+    univariate_eval_many_dev(Ds, D, vecs, nvec, c.vector_size, w.ood_points.data(), nood, mbox, s);
     mailbox_wait(s);
     w.ood_values.resize(nood * nvec * D);
     for (size_t i = 0; i < nood; i++)
       for (size_t b = 0; b < nvec; b++) {
-        std::copy(mbox + (b * pad + i) * D, mbox + (b * pad + i + 1) * D, &w.ood_values[(i * nvec + b) * D]);
+        std::copy(mbox + (b * nood + i) * D, mbox + (b * nood + i + 1) * D, &w.ood_values[(i * nvec + b) * D]);
         t.prover_field(D, &w.ood_values[(i * nvec + b) * D], 1);
       }
   }
@@ -1078,13 +1075,10 @@ void prove_impl(const WhirCfg& cfg, Transcript& t, const uint64_t* const* vecs, 
   if (W > 1 && nood) {
     const size_t pad = (nood + 3) / 4 * 4;
     WHIR_REQUIRE(V * pad * D <= RESULT_MAILBOX_WORDS, "too many out-of-domain cross terms");
-    for (size_t j = 0; j < V; j++) {
-      if (j + 1 == V) mailbox_arm(s);
-      univariate_eval_many_dev(1, D, vecs[j], n, opts.data(), nood, mbox + j * pad * D, s, true);
-    }
+    mailbox_arm(s);
+    univariate_eval_many_dev(1, D, vecs, V, n, opts.data(), nood, mbox, s);
     mailbox_wait(s);
-    cross.resize(V * nood * D);
-    for (size_t j = 0; j < V; j++) std::copy(mbox + j * pad * D, mbox + (j * pad + nood) * D, &cross[j * nood * D]);
+    cross.assign(mbox, mbox + V * nood * D);
   }
   std::vector<E<D>> omat;  // nood x V
   for (size_t w = 0, o = 0; w < W; w++) {
