@@ -909,6 +909,8 @@ struct CovPlan {
 // to this many words travel with the launch itself, which saves a staged copy and
 // its launch; larger inputs are copied into the table buffer first.
 static constexpr size_t COV_ARG_WORDS = 320;
+// Larger inputs of short tables (few waves) are read in pinned host memory.
+static constexpr size_t COV_IN_PLACE = (size_t)1 << 16;
 struct CovIn {
   uint64_t w[COV_ARG_WORDS];
 };
@@ -1227,18 +1229,20 @@ static void geo_terms_t(uint64_t* acc, size_t n, bool accumulate, const uint64_t
     for (int k = 0; k < 8; k++) in.insert(in.end(), lo[k].c, lo[k].c + D);
   }
   const bool by_arg = in.size() <= COV_ARG_WORDS;
-  size_t w = by_arg ? 0 : in.size();
+  const size_t entries = m_b * L.H + m_b * 256 + m_e * ((L.H + GEO_RUN - 1) / GEO_RUN) + m_e * (256 / GEO_RUN);
+  const uint64_t* in_place = nullptr;
+  if (!by_arg && entries <= COV_IN_PLACE) in_place = (const uint64_t*)stage_async(in.data(), in.size() * 8, s);
+  size_t w = by_arg || in_place ? 0 : in.size();
   L.hi = w;   w += m * L.H * D;
   L.lo_e = w; w += m_e * 256 * D;
   L.lo_b = w; w += m_b * 256;
   DevBuf buf(w * 8, s);
   CovIn args{};
   if (by_arg) std::copy(in.begin(), in.end(), args.w);
-  else upload_async(buf.ptr, in.data(), in.size() * 8, s);
+  else if (!in_place) upload_async(buf.ptr, in.data(), in.size() * 8, s);
   const TwTable tw = m_b ? twiddles(logN) : TwTable{};
-  const size_t entries = m_b * L.H + m_b * 256 + m_e * ((L.H + GEO_RUN - 1) / GEO_RUN) + m_e * (256 / GEO_RUN);
-  k_geo_tables<D><<<blocks_for(entries, RT), RT, 0, s>>>(buf.as<uint64_t>(), L, by_arg ? nullptr : buf.as<uint64_t>(),
-                                                          args, tw);
+  k_geo_tables<D><<<blocks_for(entries, RT), RT, 0, s>>>(
+      buf.as<uint64_t>(), L, by_arg ? nullptr : in_place ? in_place : buf.as<uint64_t>(), args, tw);
   WHIR_HIP(hipGetLastError());
   ProfScope prof(kernel_name("k_geo", D), s, 8.0 * D * (accumulate ? 2.0 : 1.0) * (double)n);
   const int ac = accumulate ? 1 : 0;
@@ -1320,7 +1324,10 @@ static void covector_t(uint64_t* acc, size_t n, bool accumulate, const uint64_t*
   }
   // Small inputs go with the launch; larger ones are copied to the front of the buffer.
   const bool by_arg = in.size() <= COV_ARG_WORDS;
-  size_t w = by_arg ? 0 : in.size();
+  L.entries = np * (L.nhi + L.nlo) + m * L.nb + L.m_e * (RT + 1) + L.m_b * (RT + 1);
+  const uint64_t* in_place = nullptr;
+  if (!by_arg && L.entries <= COV_IN_PLACE) in_place = (const uint64_t*)stage_async(in.data(), in.size() * 8, s);
+  size_t w = by_arg || in_place ? 0 : in.size();
   L.hi = w;  w += np * L.nhi * D;
   L.lo = w;  w += np * L.nlo * D;
   L.T0 = w;  w += m * L.nb * D;
@@ -1329,13 +1336,12 @@ static void covector_t(uint64_t* acc, size_t n, bool accumulate, const uint64_t*
   L.T1b = w; w += L.m_b * RT;
   L.Xb = w;  w += L.m_b;
   L.words = w;
-  L.entries = np * (L.nhi + L.nlo) + m * L.nb + L.m_e * (RT + 1) + L.m_b * (RT + 1);
   DevBuf buf(L.words * 8, s);
   CovIn args{};
   if (by_arg) std::copy(in.begin(), in.end(), args.w);
-  else upload_async(buf.ptr, in.data(), in.size() * 8, s);
-  k_cov_tables<D><<<blocks_for(L.entries, RT), RT, 0, s>>>(buf.as<uint64_t>(), L, by_arg ? nullptr : buf.as<uint64_t>(),
-                                                            args);
+  else if (!in_place) upload_async(buf.ptr, in.data(), in.size() * 8, s);
+  k_cov_tables<D><<<blocks_for(L.entries, RT), RT, 0, s>>>(
+      buf.as<uint64_t>(), L, by_arg ? nullptr : in_place ? in_place : buf.as<uint64_t>(), args);
   WHIR_HIP(hipGetLastError());
   ProfScope prof(kernel_name("k_cov", D, K), s, 8.0 * D * (accumulate ? 2.0 : 1.0) * (double)n);
   const unsigned g = (unsigned)L.nb;

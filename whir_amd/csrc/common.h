@@ -47,6 +47,18 @@ void release_commit_plans();
 // Enqueue a host->device copy on stream s; `src` may be reused as soon as this
 // returns (small copies go through a pinned per-thread staging area).
 void upload_async(void* dst, const void* src, size_t bytes, hipStream_t s);
+// The same bytes left in the pinned staging area, which a kernel on s can read in place
+// (8-byte aligned): for inputs that few waves read once, where a copy would be a launch of
+// its own (about 8 us between the launches around it on MI355X).  Null when they do not fit.
+const void* stage_async(const void* src, size_t bytes, hipStream_t s);
+// Words copied by one small launch between device and pinned memory (each side either);
+// raise: the launch also raises the flag of an armed mailbox wait on s.
+struct MoveSeg {
+  uint64_t* dst;
+  const uint64_t* src;
+  size_t words;
+};
+void move_words(const MoveSeg* segs, size_t n, hipStream_t s, bool raise);
 // Copy device->host through a pinned per-thread buffer and wait for it.
 void download_sync(void* dst, const void* src, size_t bytes, hipStream_t s);
 

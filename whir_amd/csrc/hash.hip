@@ -980,7 +980,8 @@ void commit_cols_host_top(int engine, int D, const uint64_t* cw, size_t N, size_
   uint8_t* mb = (uint8_t*)result_mailbox(st);
   WHIR_REQUIRE(32 * (2 * w - 1) <= 8 * RESULT_MAILBOX_WORDS, "commit: tree top too wide for the mailbox");
   mailbox_arm(st);
-  WHIR_HIP(hipMemcpyAsync(mb, nodes + 32 * (2 * W - 2 * w), 32 * w, hipMemcpyDefault, st));
+  const MoveSeg in{(uint64_t*)mb, (const uint64_t*)(nodes + 32 * (2 * W - 2 * w)), 4 * w};
+  move_words(&in, 1, st, true);
   mailbox_wait(st);
   const uint8_t pad = engine == ENG_SHA3 ? 0x06 : 0x01;
   const uint8_t* cur = mb;
@@ -992,7 +993,8 @@ void commit_cols_host_top(int engine, int D, const uint64_t* cw, size_t N, size_
   }
   memcpy(root, cur, 32);
   // (ordered before any later launch that writes results to the mailbox)
-  if (w > 1) WHIR_HIP(hipMemcpyAsync(nodes + 32 * (2 * W - w), mb + 32 * w, 32 * (w - 1), hipMemcpyDefault, st));
+  const MoveSeg back{(uint64_t*)(nodes + 32 * (2 * W - w)), (const uint64_t*)(mb + 32 * w), 4 * (w - 1)};
+  if (w > 1) move_words(&back, 1, st, false);
 }
 
 void commit_cols_many_dev(int engine, int D, const uint64_t* const* cw_tab, uint8_t* const* nodes_tab, size_t count,

@@ -287,9 +287,10 @@ void irs_commit(Transcript& t, const IrsCfg& c, int engine, const uint64_t* cons
     // one block would spend ~15 us on.
     const size_t n = c.vector_size;
     uint64_t* stage = host_stage();
+    std::vector<MoveSeg> segs;
+    for (size_t b = 0; b < nvec; b++) segs.push_back(MoveSeg{stage + b * n * Ds, vecs[b], n * Ds});
     mailbox_arm(s);
-    for (size_t b = 0; b < nvec; b++)
-      WHIR_HIP(hipMemcpyAsync(stage + b * n * Ds, vecs[b], n * Ds * 8, hipMemcpyDefault, s));
+    move_words(segs.data(), segs.size(), s, true);
     mailbox_wait(s);
     w.ood_values.resize(nood * nvec * D);
     for (size_t i = 0; i < nood; i++) {
@@ -381,6 +382,10 @@ struct OpenLaunch {
   std::shared_ptr<DevBuf> dout;
 };
 
+// Openings of at most this many values and nodes read their indices and weights in pinned
+// host memory.
+constexpr size_t OPEN_IN_PLACE = 4096;
+
 OpenLaunch open_rows_launch(const DevWitness& w, const std::vector<size_t>& idx, hipStream_t s, int D,
                             const uint64_t* wts, size_t off) {
   OpenLaunch L;
@@ -422,9 +427,16 @@ OpenLaunch open_rows_launch(const DevWitness& w, const std::vector<size_t>& idx,
   // one upload: the row and node indices, then the column weights
   const size_t nidx = idx_sib.size();
   if (D > 0) idx_sib.insert(idx_sib.end(), wts, wts + M * D);
-  DevBuf dis(idx_sib.size() * 8, s);
-  upload_async(dis.ptr, idx_sib.data(), idx_sib.size() * 8, s);
-  const uint64_t* dw = D > 0 ? dis.as<uint64_t>() + nidx : nullptr;
+  // read in place by a few waves; a wide opening would read them over and over
+  const uint64_t* di = nullptr;
+  if (k * M + L.ns <= OPEN_IN_PLACE)
+    di = (const uint64_t*)stage_async(idx_sib.data(), idx_sib.size() * 8, s);
+  DevBuf dis(di ? 0 : idx_sib.size() * 8, s);
+  if (!di) {
+    upload_async(dis.ptr, idx_sib.data(), idx_sib.size() * 8, s);
+    di = dis.as<uint64_t>();
+  }
+  const uint64_t* dw = D > 0 ? di + nidx : nullptr;
   uint64_t* out;
   // WHIR_OPEN_MAILBOX_WORDS lowers the mailbox room openings may use (a test knob that
   // sends them through the device-buffer path).
@@ -437,7 +449,7 @@ OpenLaunch open_rows_launch(const DevWitness& w, const std::vector<size_t>& idx,
     L.dout = std::make_shared<DevBuf>(L.out_words * 8, s);
     out = L.dout->as<uint64_t>();
   }
-  gather_open_dev(w.Ds, w.cw.as<uint64_t>(), N, M, dis.as<uint64_t>(), k, w.nodes.as<uint8_t>(), L.ns, out,
+  gather_open_dev(w.Ds, w.cw.as<uint64_t>(), N, M, di, k, w.nodes.as<uint8_t>(), L.ns, out,
                   (uint8_t*)(out + L.hash_off), s, D, dw, out + L.val_off);
   return L;
 }
@@ -652,22 +664,51 @@ constexpr size_t HOST_SUMCHECK_MAX = 64;
 // memory, extension elements): the same messages, challenges and folds as the device
 // rounds (x'_i = x_i + r (x_(h+i) - x_i), c0 = sum x_i y_i, c2 = sum dx_i dy_i over
 // i < h = n/2).
+//
+// keep: the vectors stay on the host instead (keep->x, keep->y) for a caller whose next
+// step works there, and the device copies are then out of date; vectors that are there
+// already are taken from it.
+template <int D>
+struct HostPair {
+  std::vector<E<D>> x, y;  // empty: the device holds the vectors
+};
+
+// Vectors worked on by the host back to the device.
+template <int D>
+void host_pair_store(const std::vector<E<D>>& x, const std::vector<E<D>>& y, uint64_t* a, uint64_t* b, hipStream_t s) {
+  uint64_t* stage = host_stage();
+  const size_t len = x.size();
+  for (size_t i = 0; i < len; i++) {
+    std::copy(x[i].c, x[i].c + D, stage + i * D);
+    std::copy(y[i].c, y[i].c + D, stage + (len + i) * D);
+  }
+  const MoveSeg segs[2] = {{a, stage, len * D}, {b, stage + len * D, len * D}};
+  move_words(segs, 2, s, false);
+}
+
 template <int D>
 std::vector<E<D>> sumcheck_prove_host(Transcript& t, const SumcheckCfg& sc, int engine, uint64_t* a, uint64_t* b,
-                                      size_t& n, E<D>& sum, hipStream_t s, const std::function<void()>& after_first) {
+                                      size_t& n, E<D>& sum, hipStream_t s, const std::function<void()>& after_first,
+                                      HostPair<D>* keep) {
   const size_t words = n * D;
   WHIR_REQUIRE(n <= HOST_SUMCHECK_MAX && 2 * words <= HOST_STAGE_WORDS, "sumcheck: vectors too long for the host path");
-  uint64_t* stage = host_stage();
-  mailbox_arm(s);
-  WHIR_HIP(hipMemcpyAsync(stage, a, words * 8, hipMemcpyDefault, s));
-  WHIR_HIP(hipMemcpyAsync(stage + words, b, words * 8, hipMemcpyDefault, s));
-  mailbox_wait(s);  // (results queued ahead, e.g. an opening's rows, are in the mailbox)
-  if (after_first) after_first();
-  std::vector<E<D>> x(n), y(n);
-  for (size_t i = 0; i < n; i++) {
-    x[i] = ld<D>(stage + i * D);
-    y[i] = ld<D>(stage + words + i * D);
+  std::vector<E<D>> x, y;
+  if (keep && !keep->x.empty()) {
+    x.swap(keep->x);
+    y.swap(keep->y);
+    if (after_first) mailbox_wait(s);
+  } else {
+    uint64_t* stage = host_stage();
+    const MoveSeg segs[2] = {{stage, a, words}, {stage + words, b, words}};
+    mailbox_arm(s);
+    move_words(segs, 2, s, true);
+    mailbox_wait(s);  // (results queued ahead, e.g. an opening's rows, are in the mailbox)
+    for (size_t i = 0; i < n; i++) {
+      x.push_back(ld<D>(stage + i * D));
+      y.push_back(ld<D>(stage + words + i * D));
+    }
   }
+  if (after_first) after_first();
   std::vector<E<D>> chals;
   size_t len = n;
   for (size_t round = 0; round < sc.num_rounds; round++) {
@@ -690,13 +731,14 @@ std::vector<E<D>> sumcheck_prove_host(Transcript& t, const SumcheckCfg& sc, int 
     }
     len = h;
   }
-  // The folded vectors back to the device.
-  for (size_t i = 0; i < len; i++) {
-    std::copy(x[i].c, x[i].c + D, stage + i * D);
-    std::copy(y[i].c, y[i].c + D, stage + (len + i) * D);
+  x.resize(len);
+  y.resize(len);
+  if (keep) {
+    keep->x.swap(x);
+    keep->y.swap(y);
+  } else {
+    host_pair_store<D>(x, y, a, b, s);
   }
-  WHIR_HIP(hipMemcpyAsync(a, stage, len * D * 8, hipMemcpyDefault, s));
-  WHIR_HIP(hipMemcpyAsync(b, stage + len * D, len * D * 8, hipMemcpyDefault, s));
   n = len;
   return chals;
 }
@@ -704,11 +746,16 @@ std::vector<E<D>> sumcheck_prove_host(Transcript& t, const SumcheckCfg& sc, int 
 template <int D>
 std::vector<E<D>> sumcheck_prove(Transcript& t, const SumcheckCfg& sc, int engine, const uint64_t* a_src, int a_Ds,
                                  uint64_t* a, uint64_t* b, size_t& n, E<D>& sum, hipStream_t s,
-                                 const std::function<void()>& after_first = {}, const CovView* view = nullptr) {
+                                 const std::function<void()>& after_first = {}, const CovView* view = nullptr,
+                                 HostPair<D>* keep = nullptr) {
   WHIR_REQUIRE(n == sc.initial_size, "sumcheck: vector length does not match the configuration");
   if (n <= HOST_SUMCHECK_MAX && n >= 2 && (n & (n - 1)) == 0 && sc.num_rounds >= 1 && !view && a_src == a &&
       a_Ds == D && ((size_t)1 << sc.num_rounds) <= n)
-    return sumcheck_prove_host<D>(t, sc, engine, a, b, n, sum, s, after_first);
+    return sumcheck_prove_host<D>(t, sc, engine, a, b, n, sum, s, after_first, keep);
+  if (keep && !keep->x.empty()) {
+    host_pair_store<D>(keep->x, keep->y, a, b, s);
+    *keep = HostPair<D>{};
+  }
   if (n >= 16 && (n & (n - 1)) == 0 && sc.num_rounds >= 2)
     return sumcheck_prove_pairs<D>(t, sc, engine, a_src, a_Ds, a, b, n, sum, s, after_first, view);
   if (view) covview_write_dev(D, *view, b, n, s);
@@ -1171,9 +1218,10 @@ void prove_impl(const WhirCfg& cfg, Transcript& t, const uint64_t* const* vecs, 
     for (size_t o = 0; o < nood; o++) the_sum = gl::eadd<D>(the_sum, gl::emul<D>(crlc[np + o], rlc_dot(&omat[o * V])));
   }
   std::vector<E<D>> fr;
+  HostPair<D> fin_pair;  // the final vectors, when the sumcheck before them ran on the host
   if (has_constraints) {
     fr = sumcheck_prove<D>(t, cfg.initial_sumcheck, eng, a0, a0_Ds, vec.as<uint64_t>(), cov.as<uint64_t>(), n,
-                           the_sum, s, {}, use_view ? &view : nullptr);
+                           the_sum, s, {}, use_view ? &view : nullptr, cfg.rounds.empty() ? &fin_pair : nullptr);
   } else {
     for (size_t i = 0; i < cfg.initial_sumcheck.num_rounds; i++) fr.push_back(verifier_field<D>(t));
     pow_prove(t, eng, cfg.initial_skip_pow, s);
@@ -1242,7 +1290,7 @@ void prove_impl(const WhirCfg& cfg, Transcript& t, const uint64_t* const* vecs, 
       }
     };
     fr = sumcheck_prove<D>(t, rc.sumcheck, eng, vec.as<uint64_t>(), D, vec.as<uint64_t>(), cov.as<uint64_t>(), n,
-                           the_sum, s, finish_open);
+                           the_sum, s, finish_open, nullptr, &rc == &cfg.rounds.back() ? &fin_pair : nullptr);
     eval_point.insert(eval_point.end(), fr.begin(), fr.end());
     held = std::move(nw);
     prev_cfg = &rc.irs;
@@ -1251,8 +1299,19 @@ void prove_impl(const WhirCfg& cfg, Transcript& t, const uint64_t* const* vecs, 
   }
   // Send the final vector directly.
   WHIR_REQUIRE(n == cfg.final_sumcheck.initial_size, "final vector length mismatch");
-  std::vector<uint64_t> fin(n * D);
-  download_sync(fin.data(), vec.ptr, n * D * 8, s);
+  std::vector<uint64_t> fin;
+  if (!fin_pair.x.empty()) {
+    for (const auto& e : fin_pair.x) push<D>(fin, e);
+  } else if (n * D <= HOST_STAGE_WORDS) {
+    const MoveSeg seg{host_stage(), vec.as<uint64_t>(), n * D};
+    mailbox_arm(s);
+    move_words(&seg, 1, s, true);
+    mailbox_wait(s);
+    fin.assign(seg.dst, seg.dst + n * D);
+  } else {
+    fin.resize(n * D);
+    download_sync(fin.data(), vec.ptr, n * D * 8, s);
+  }
   for (size_t i = 0; i < n; i++) t.prover_field(D, &fin[i * D], 1);
   pow_prove(t, eng, cfg.final_pow, s);
   // The final opening is queued ahead of the final sumcheck's first pass and read back
@@ -1264,7 +1323,7 @@ void prove_impl(const WhirCfg& cfg, Transcript& t, const uint64_t* const* vecs, 
     irs_open_finish(t, fopens, rows, vals, s);
   };
   fr = sumcheck_prove<D>(t, cfg.final_sumcheck, eng, vec.as<uint64_t>(), D, vec.as<uint64_t>(), cov.as<uint64_t>(),
-                         n, the_sum, s, finish_final);
+                         n, the_sum, s, finish_final, nullptr, &fin_pair);
   eval_point.insert(eval_point.end(), fr.begin(), fr.end());
   if (eval_point_out)
     for (size_t i = 0; i < eval_point.size(); i++)

@@ -197,8 +197,7 @@ hipStream_t thread_stream() {
   return t_stream.s;
 }
 
-void upload_async(void* dst, const void* src, size_t bytes, hipStream_t s) {
-  if (!bytes) return;
+const void* stage_async(const void* src, size_t bytes, hipStream_t s) {
   Staging& st = t_staging;
   int dev = 0;
   WHIR_HIP(hipGetDevice(&dev));
@@ -211,19 +210,56 @@ void upload_async(void* dst, const void* src, size_t bytes, hipStream_t s) {
     st.off = 0;
     st.device = dev;
   }
-  if (bytes > st.cap / 4) {  // large: plain copy, then wait so `src` may be released
-    WHIR_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s));
-    WHIR_HIP(hipStreamSynchronize(s));
-    return;
-  }
+  if (bytes > st.cap / 4) return nullptr;
   if (st.off + bytes > st.cap) {
     WHIR_HIP(hipEventRecord(st.wrap, s));
     WHIR_HIP(hipEventSynchronize(st.wrap));
     st.off = 0;
   }
-  memcpy(st.host + st.off, src, bytes);
-  WHIR_HIP(hipMemcpyAsync(dst, st.host + st.off, bytes, hipMemcpyHostToDevice, s));
+  uint8_t* at = (uint8_t*)st.host + st.off;
+  memcpy(at, src, bytes);
   st.off += (bytes + 255) & ~(size_t)255;
+  return at;
+}
+
+void upload_async(void* dst, const void* src, size_t bytes, hipStream_t s) {
+  if (!bytes) return;
+  if (const void* at = stage_async(src, bytes, s)) {
+    WHIR_HIP(hipMemcpyAsync(dst, at, bytes, hipMemcpyHostToDevice, s));
+    return;
+  }
+  // large: plain copy, then wait so `src` may be released
+  WHIR_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s));
+  WHIR_HIP(hipStreamSynchronize(s));
+}
+
+namespace {
+constexpr int MOVE_SEGS = 8;
+struct MoveArgs {
+  MoveSeg seg[MOVE_SEGS];
+  int n;
+};
+// A few KB at most: one block, so that it can raise the flag after its last store.
+__global__ __launch_bounds__(256) void k_move(MoveArgs a, MailboxSig sig) {
+  for (int k = 0; k < a.n; k++)
+    for (size_t i = threadIdx.x; i < a.seg[k].words; i += blockDim.x) a.seg[k].dst[i] = a.seg[k].src[i];
+  if (sig.flag) {
+    __syncthreads();
+    if (threadIdx.x == 0) mailbox_raise(sig);
+  }
+}
+}  // namespace
+
+void move_words(const MoveSeg* segs, size_t n, hipStream_t s, bool raise) {
+  for (size_t i = 0; i < n; i += MOVE_SEGS) {
+    MoveArgs a{};
+    a.n = (int)std::min<size_t>(MOVE_SEGS, n - i);
+    std::copy(segs + i, segs + i + a.n, a.seg);
+    // (any mailbox word names the stream's armed wait)
+    const MailboxSig sig = raise && i + MOVE_SEGS >= n ? mailbox_take(result_mailbox(s)) : MailboxSig{};
+    k_move<<<1, 256, 0, s>>>(a, sig);
+    WHIR_HIP(hipGetLastError());
+  }
 }
 
 namespace {
