@@ -29,6 +29,15 @@ def test_stir_terms_over_short_and_long_vectors(nv, D, lir, sec):
     check(nv, D, W.HASH_BLAKE3, 4, 4, lir, 1, sec)
 
 
+# STIR terms in one launch and the sizes beside it: 16 to 256 lanes a block, one and several
+# blocks, vectors shorter than a block, point counts on both sides of the rule.
+@pytest.mark.parametrize("nv,D,k,lir,sec", [(6, 2, 2, 1, 32), (7, 1, 3, 1, 32), (8, 3, 3, 2, 80), (11, 2, 1, 1, 100),
+                                            (14, 2, 4, 1, 128), (16, 3, 4, 1, 100), (17, 2, 4, 1, 100),
+                                            (18, 2, 4, 3, 60), (18, 2, 4, 1, 110), (20, 3, 4, 2, 60), (20, 1, 3, 1, 40)])
+def test_stir_terms_in_one_launch(nv, D, k, lir, sec):
+    check(nv, D, W.HASH_BLAKE3, k, k, lir, 1, sec)
+
+
 # Sumcheck passes that sum two rounds: 2^10 and 2^11 elements are the last that one block
 # and the first that several blocks sum; odd round counts end with a pass of one round's two
 # sums; the initial round runs over tables of 1 to 2^6 blocks.

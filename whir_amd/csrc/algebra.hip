@@ -1255,6 +1255,123 @@ static void geo_terms_t(uint64_t* acc, size_t n, bool accumulate, const uint64_t
   WHIR_HIP(hipGetLastError());
 }
 
+// The same terms over a short vector in one launch: a block makes its own factors in LDS
+// (HI of its row h, one twiddle product per in-domain point; for an OOD point x^l as the
+// product of x^(16 a) and x^b, l = 16 a + b), deals the points to the groups of LW lanes that
+// its 1024 threads form, takes LO of an in-domain point straight from the twiddle tables, and
+// adds the groups in LDS.
+// Its rule: up to 64 blocks of 16 to 256 lanes (every block reads all the inputs, from host
+// memory), 256 lanes above; points times lanes at most 2^14, since a lane's turns over the
+// points gather from the twiddle tables.  Fp2 on MI355X against the table launch, k_geo and the
+// 3 us between them: 2^10 elements, 180 points 9 us against 25; 2^12, 85 points 8 against 20;
+// 2^13, 85 points 20 against 29; 2^16, 45 points 12 against 20; but 2^14, 85 points 32 against 30.
+constexpr size_t GEO_SHORT_N = (size_t)1 << 16, GEO_SHORT_WORK = (size_t)1 << 14;
+constexpr size_t GEO_SHORT_M = 256, GEO_SHORT_ME = 4, GEO_SHORT_IN = 1536;
+struct GeoShort {
+  uint64_t N;
+  uint32_t m_e, m_b, lw;          // points; LW = 2^lw
+  uint32_t in_t, in_sq, nsq, words;  // inputs: exponents, then scalars, then per OOD point x^(2^k), k < nsq
+};
+
+template <int D>
+__global__ __launch_bounds__(1024) void k_geo_short(uint64_t* acc, size_t n, int accumulate, GeoShort L,
+                                                    const uint64_t* in_dev, CovIn in_arg, TwTable tw) {
+  __shared__ uint64_t in[GEO_SHORT_IN], hi[GEO_SHORT_M * D], ab[GEO_SHORT_ME * 32 * D], part[D][1024];
+  const uint32_t tid = threadIdx.x;
+  const uint64_t h = blockIdx.x;
+  for (uint32_t i = tid; i < L.words; i += 1024) in[i] = in_dev ? in_dev[i] : in_arg.w[i];
+  __syncthreads();
+  for (uint32_t e = tid; e < L.m_b + L.m_e * 33; e += 1024) {
+    if (e < L.m_b) {
+      const uint64_t x = tw_at(tw, ((h << L.lw) * in[e]) & (L.N - 1));
+      st<D>(hi, L.m_e + e, gl::escale<D>(ld<D>(in + L.in_t, L.m_e + e), x));
+    } else {
+      const uint32_t j = (e - L.m_b) / 33, i = (e - L.m_b) % 33;
+      Ext<D> v = i == 32 ? ld<D>(in + L.in_t, j) : gl::ext_base<D>(1);
+      const uint64_t* sq = in + L.in_sq + j * L.nsq * D;
+#pragma unroll 1
+      for (uint64_t x = i == 32 ? h << L.lw : i < 16 ? i << 4 : i - 16; x; x &= x - 1)
+        v = gl::emul<D>(v, ld<D>(sq, __builtin_ctzll(x)));
+      if (i == 32) st<D>(hi, j, v);
+      else st<D>(ab, j * 32 + i, v);
+    }
+  }
+  __syncthreads();
+  const uint32_t LW = 1u << L.lw, l = tid & (LW - 1), G = 1024u >> L.lw;
+  gl::Wide W[D];
+  gl::wide_zero<D>(W);
+#pragma unroll 4
+  for (uint32_t j = tid >> L.lw; j < L.m_b; j += G) {
+    const uint64_t lo = tw_at(tw, (l * in[j]) & (L.N - 1));
+#pragma unroll
+    for (int d = 0; d < D; d++) gl::wide_mac(W[d], hi[(L.m_e + j) * D + d], lo);
+  }
+  // (from the last group on: the first ones have the odd in-domain points)
+#pragma unroll 1
+  for (uint32_t j = G - 1 - (tid >> L.lw); j < L.m_e; j += G)
+    gl::emul_acc<D>(W, ld<D>(hi, j), gl::emul<D>(ld<D>(ab, j * 32 + (l >> 4)), ld<D>(ab, j * 32 + 16 + (l & 15))));
+  const Ext<D> sum = gl::ext_reduce<D>(W);
+#pragma unroll
+  for (int d = 0; d < D; d++) part[d][tid] = sum.c[d];
+#pragma unroll 1
+  for (uint32_t s = 512; s >= LW; s >>= 1) {
+    __syncthreads();
+    if (tid < s)
+#pragma unroll
+      for (int d = 0; d < D; d++) part[d][tid] = gl::add(part[d][tid], part[d][tid + s]);
+  }
+  const size_t i = (h << L.lw) + l;
+  if (tid < LW && i < n) {
+    Ext<D> v;
+#pragma unroll
+    for (int d = 0; d < D; d++) v.c[d] = part[d][tid];
+    st<D>(acc, i, accumulate ? gl::eadd<D>(ld<D>(acc, i), v) : v);
+  }
+}
+
+template <int D>
+static bool geo_short_t(uint64_t* acc, size_t n, bool accumulate, const uint64_t* scalars, const uint64_t* ext_points,
+                        size_t m_e, const uint64_t* exps, size_t m_b, int logN, hipStream_t s) {
+  const size_t m = m_e + m_b;
+  GeoShort L{};
+  for (L.nsq = 8; ((size_t)1 << L.nsq) < n;) L.nsq++;
+  L.words = (uint32_t)std::min<size_t>(m_b + m * D + m_e * L.nsq * D, ~0u);
+  if (n > GEO_SHORT_N || m > GEO_SHORT_M || m_e > GEO_SHORT_ME || L.words > GEO_SHORT_IN) return false;
+  L.N = (uint64_t)1 << logN;
+  L.m_e = (uint32_t)m_e;
+  L.m_b = (uint32_t)m_b;
+  L.in_t = (uint32_t)m_b;
+  L.in_sq = (uint32_t)(m_b + m * D);
+  for (L.lw = 4; L.lw < 8 && ((size_t)64 << L.lw) < n;) L.lw++;
+  if ((m << L.lw) > GEO_SHORT_WORK) return false;
+  const size_t H = (n + ((size_t)1 << L.lw) - 1) >> L.lw;
+  std::vector<uint64_t> in(exps, exps + m_b);
+  in.insert(in.end(), scalars, scalars + m * D);
+  for (size_t j = 0; j < m_e; j++) {
+    Ext<D> x;
+    for (int d = 0; d < D; d++) x.c[d] = ext_points[j * D + d];
+    for (uint32_t k = 0; k < L.nsq; k++) {
+      in.insert(in.end(), x.c, x.c + D);
+      x = gl::emul<D>(x, x);
+    }
+  }
+  CovIn args{};
+  const uint64_t* in_dev = nullptr;
+  DevBuf buf;
+  if (in.size() <= COV_ARG_WORDS) {
+    std::copy(in.begin(), in.end(), args.w);
+  } else if (!(in_dev = (const uint64_t*)stage_async(in.data(), in.size() * 8, s))) {
+    buf = DevBuf(in.size() * 8, s);
+    upload_async(buf.ptr, in.data(), in.size() * 8, s);
+    in_dev = buf.as<uint64_t>();
+  }
+  const TwTable tw = m_b ? twiddles(logN) : TwTable{};
+  ProfScope prof(kernel_name("k_geo_short", D), s, 8.0 * D * (accumulate ? 2.0 : 1.0) * (double)n);
+  k_geo_short<D><<<(unsigned)H, 1024, 0, s>>>(acc, n, accumulate ? 1 : 0, L, in_dev, args, tw);
+  WHIR_HIP(hipGetLastError());
+  return true;
+}
+
 // WHIR_COV_GEO=0 keeps power terms on the one-pass kernel (for comparison).
 static bool geo_path_enabled() {
   static const bool on = [] {
@@ -1521,6 +1638,15 @@ void covector_stir_dev(int D, uint64_t* acc, size_t n, bool accumulate, const ui
                        const uint64_t* ext_points, size_t m_e, const uint64_t* exps, const uint64_t* points, size_t m_b,
                        int logN, hipStream_t s) {
   const size_t m = m_e + m_b;
+  if (geo_path_enabled() && m && n && logN <= 62) {
+    bool done = false;
+    switch (D) {
+      case 1: done = geo_short_t<1>(acc, n, accumulate, scalars, ext_points, m_e, exps, m_b, logN, s); break;
+      case 2: done = geo_short_t<2>(acc, n, accumulate, scalars, ext_points, m_e, exps, m_b, logN, s); break;
+      case 3: done = geo_short_t<3>(acc, n, accumulate, scalars, ext_points, m_e, exps, m_b, logN, s); break;
+    }
+    if (done) return;
+  }
   if (!geo_path_enabled() || m < 8 || !n || n % 256 || logN > 62) {
     // the one-pass kernel, with every point as a field element (in-domain points lifted)
     std::vector<uint64_t> pts(ext_points, ext_points + m_e * D);
