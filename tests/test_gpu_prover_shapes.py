@@ -1,5 +1,7 @@
 """Proofs at the sizes where a kernel of the prover changes shape: the GPU proof equals the
 oracle's byte for byte."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -68,3 +70,21 @@ def test_out_of_domain_values_of_batches(nv, D, B, NW):
     _, _, narg, hints, _ = oracle_batch(nv, D, B, NW, vecs, points, params, pid, sid)
     _, gnarg, ghints, _ = gpu_batch(nv, D, B, NW, vecs, points, params, pid, sid)
     assert gnarg == narg and ghints == hints
+
+
+# A round polynomial and a fold with the next one: one block (up to 2^10 pairs), several, several
+# turns; lengths that are no power of two.
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 64, 127, 2047, 2048, 2049, 4096, 4097, 8192, 100001, 2**21 + 3])
+@pytest.mark.parametrize("D", [1, 2, 3])
+def test_sumcheck_rounds_on_the_device(n, D):
+    a, b, w = rnd_np(n, n * D), rnd_np(n + 1, n * D), rnd_np(n + 2, D)
+    da, db = W.DeviceBuffer.from_array(a), W.DeviceBuffer.from_array(b)
+    out = np.zeros(2 * D, dtype=np.uint64)
+    W._call("whir_sumcheck_polynomial_dev", D, da.ptr, db.ptr, n, W._p64(out))
+    assert np.array_equal(out, np.concatenate(O.sumcheck_poly(D, a, b)))
+    m = ctypes.c_size_t()
+    W._call("whir_fold_and_compute_polynomial_dev", D, da.ptr, db.ptr, n, W._p64(w), W._p64(out), ctypes.byref(m))
+    fa, fb = O.fold(D, a, w), O.fold(D, b, w)
+    assert m.value * D == fa.size
+    assert np.array_equal(da.to_array()[:fa.size], fa) and np.array_equal(db.to_array()[:fb.size], fb)
+    assert np.array_equal(out, np.concatenate(O.sumcheck_poly(D, fa, fb)))

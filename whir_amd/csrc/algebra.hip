@@ -133,9 +133,8 @@ static void finish_reduce(const uint64_t* parts, unsigned nparts, uint64_t* out,
 
 static unsigned grid_for(size_t n) { return (unsigned)std::min<size_t>(blocks_for(n, RT), MAX_BLOCKS); }
 
-// Up to this many element pairs a reducing pass runs as one block (four pairs per
-// lane), which stores its sums directly: cheaper than a second launch (256 and 64
-// measured no faster at d = 24 on MI355X).
+// Up to this many element pairs a reducing pass runs as one block of up to 1024 threads,
+// which stores its sums directly: cheaper than a second launch.
 static constexpr size_t SMALL_PAIRS = 1024;
 
 // Pass a small host constant (D words) to kernels by value.
@@ -168,25 +167,38 @@ __device__ __forceinline__ Ext<D> mulx(const uint64_t* a, size_t i, const Ext<D>
   else return gl::escale<D>(b, a[i]);
 }
 
+// w += a b with a embedded from Ds words.
 template <int Ds, int D>
-__global__ __launch_bounds__(RT) void k_sc_poly(const uint64_t* __restrict__ a, const uint64_t* __restrict__ b,
-                                                size_t half, size_t nhi, uint64_t* parts, MailboxSig sig) {
-  Ext<D> acc[2] = {gl::ext_zero<D>(), gl::ext_zero<D>()};
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < half; i += (size_t)gridDim.x * blockDim.x) {
-    const Ext<D> b0 = ld<D>(b, i);
-    const Ext<D> p0 = mulx<Ds, D>(a, i, b0);
-    acc[0] = gl::eadd<D>(acc[0], p0);
-    if (i < nhi) {
-      const Ext<D> db = gl::esub<D>(ld<D>(b, half + i), b0);
-      if constexpr (Ds == D) {
-        acc[1] = gl::eadd<D>(acc[1], gl::emul<D>(gl::esub<D>(ld<D>(a, half + i), ld<D>(a, i)), db));
-      } else {
-        acc[1] = gl::eadd<D>(acc[1], gl::escale<D>(db, gl::sub(a[half + i], a[i])));
-      }
-    } else {
-      acc[1] = gl::eadd<D>(acc[1], p0);  // implicit zero padding: (0 - a)(0 - b) = a b
-    }
+__device__ __forceinline__ void mulx_acc(gl::Wide (&w)[D], const Ext<Ds>& a, const Ext<D>& b) {
+  if constexpr (Ds == D) {
+    gl::emul_acc<D>(w, a, b);
+  } else {
+#pragma unroll
+    for (int d = 0; d < D; d++) gl::wide_mac(w[d], a.c[0], b.c[d]);
   }
+}
+
+// The products are summed unreduced (emul_acc) and reduced once per lane.
+template <int Ds, int D>
+__global__ __launch_bounds__(1024) void k_sc_poly(const uint64_t* __restrict__ a, const uint64_t* __restrict__ b,
+                                                size_t half, size_t nhi, uint64_t* parts, MailboxSig sig) {
+  gl::Wide w[2][D];
+  gl::wide_zero<D>(w[0]);
+  gl::wide_zero<D>(w[1]);
+#pragma unroll 1
+  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < half; i += (size_t)gridDim.x * blockDim.x) {
+    const Ext<Ds> a0 = ld<Ds>(a, i);
+    const Ext<D> b0 = ld<D>(b, i);
+    Ext<Ds> a1 = gl::ext_zero<Ds>();  // implicit zero padding past the end
+    Ext<D> b1 = gl::ext_zero<D>();
+    if (i < nhi) {
+      a1 = ld<Ds>(a, half + i);
+      b1 = ld<D>(b, half + i);
+    }
+    mulx_acc<Ds, D>(w[0], a0, b0);
+    mulx_acc<Ds, D>(w[1], gl::esub<Ds>(a1, a0), gl::esub<D>(b1, b0));
+  }
+  Ext<D> acc[2] = {gl::ext_reduce<D>(w[0]), gl::ext_reduce<D>(w[1])};
   block_reduce_store<D, 2>(acc, parts + (size_t)blockIdx.x * 2 * D, sig);
 }
 
@@ -212,7 +224,7 @@ static void sc_poly(const uint64_t* a, const uint64_t* b, size_t n, uint64_t* ou
   DevBuf parts(g == 1 ? 0 : (size_t)g * 2 * D * 8, s);
   {
     ProfScope prof(kernel_name("k_sc_poly", Ds, D), s, 8.0 * (Ds + D) * (double)n);
-    k_sc_poly<Ds, D><<<g, RT, 0, s>>>(a, b, half, nhi, g == 1 ? out : parts.as<uint64_t>(),
+    k_sc_poly<Ds, D><<<g, g == 1 ? reduce_threads(half) : RT, 0, s>>>(a, b, half, nhi, g == 1 ? out : parts.as<uint64_t>(),
                                       g == 1 ? mailbox_take(out) : MailboxSig{});
     WHIR_HIP(hipGetLastError());
   }
@@ -349,32 +361,66 @@ size_t fold_both_dev(int Ds, int D, const uint64_t* a_in, uint64_t* a_out, uint6
 }
 
 // ------------------------------------------------------------------ fused fold + polynomial
+// The value of lane CTRL[l] of each quad of lanes (quad_perm: two bits per lane l).
+template <int CTRL>
+__device__ __forceinline__ uint64_t quad_get(uint64_t v) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)v, CTRL, 0xf, 0xf, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(v >> 32), CTRL, 0xf, 0xf, true);
+  return ((uint64_t)hi << 32) | lo;
+}
+template <int CTRL, int D>
+__device__ __forceinline__ Ext<D> quad_get(const Ext<D>& v) {
+  Ext<D> r;
+#pragma unroll
+  for (int d = 0; d < D; d++) r.c[d] = quad_get<CTRL>(v.c[d]);
+  return r;
+}
+constexpr int quad_ctrl(int a, int b, int c, int d) { return a | b << 2 | c << 4 | d << 6; }
+
+// Lane 0 of a pair of lanes: its own value; lane 1: its value less lane 0's.
+template <int D>
+__device__ __forceinline__ Ext<D> pair_factor(const Ext<D>& x) {
+  const Ext<D> d = gl::esub<D>(x, quad_get<quad_ctrl(0, 0, 2, 2)>(x));
+  Ext<D> p;
+#pragma unroll
+  for (int k = 0; k < D; k++) p.c[k] = (threadIdx.x & 1) ? d.c[k] : x.c[k];
+  return p;
+}
+
 // Fold a (Ds words, into a_out) and b (in place) by w, then the round polynomial of
 // the folded pair.  Folded length h = next_pow2(n)/2 (a power of two >= 2); the new
-// pairs are (i, h/2 + i).  Lane i writes positions i and h/2 + i only and reads
-// i, h/2 + i, h + i, h + h/2 + i, so a_out may alias a_in when Ds == D.
+// pairs are (i, h/2 + i), h/2 = q.  Two lanes share a pair: lane l folds position l q + i of
+// both vectors (it writes that position and reads it and h + it, so a_out may alias a_in when
+// Ds == D), then lane 0 takes the product of the low halves and lane 1 that of the
+// differences: half the code and twice the lanes of a lane per pair.  Fp2 on MI355X: 2^12
+// elements 17 -> 12 us, 2^17 9.2 -> 7.5, 2^20 16 -> 17; long vectors move 5 TB/s either way.
 template <int Ds, int D>
-__global__ __launch_bounds__(RT) void k_fold_poly(const uint64_t* a_in, uint64_t* a_out, uint64_t* b, size_t h,
+__global__ __launch_bounds__(1024) void k_fold_poly(const uint64_t* a_in, uint64_t* a_out, uint64_t* b, size_t h,
                                                   size_t nhi, Ext<D> w, Ext<D> om, uint64_t* parts,
                                                   MailboxSig sig) {
-  Ext<D> acc[2] = {gl::ext_zero<D>(), gl::ext_zero<D>()};
-  const size_t q = h >> 1;
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < q; i += (size_t)gridDim.x * blockDim.x) {
-    Ext<D> a0 = fold_at<Ds, D>(a_in, i, h, nhi, w, om), a1 = fold_at<Ds, D>(a_in, q + i, h, nhi, w, om);
-    Ext<D> b0 = fold_at<D, D>(b, i, h, nhi, w, om), b1 = fold_at<D, D>(b, q + i, h, nhi, w, om);
-    st<D>(a_out, i, a0); st<D>(a_out, q + i, a1);
-    st<D>(b, i, b0); st<D>(b, q + i, b1);
-    acc[0] = gl::eadd<D>(acc[0], gl::emul<D>(a0, b0));
-    acc[1] = gl::eadd<D>(acc[1], gl::emul<D>(gl::esub<D>(a1, a0), gl::esub<D>(b1, b0)));
+  gl::Wide acc[D];
+  gl::wide_zero<D>(acc);
+  const size_t q = h >> 1, l = threadIdx.x & 1;
+#pragma unroll 1
+  for (size_t i = (blockIdx.x * (size_t)blockDim.x + threadIdx.x) >> 1; i < q;
+       i += ((size_t)gridDim.x * blockDim.x) >> 1) {
+    const size_t t = l * q + i;
+    const Ext<D> x = fold_at<Ds, D>(a_in, t, h, nhi, w, om), y = fold_at<D, D>(b, t, h, nhi, w, om);
+    st<D>(a_out, t, x);
+    st<D>(b, t, y);
+    gl::emul_acc<D>(acc, pair_factor<D>(x), pair_factor<D>(y));
   }
-  block_reduce_store<D, 2>(acc, parts + (size_t)blockIdx.x * 2 * D, sig);
+  Ext<D> v[1] = {gl::ext_reduce<D>(acc)};
+  __shared__ uint64_t tot[2 * D];
+  block_role_sum<D, 1, 2>(v, tot);
+  store_words<2 * D>(threadIdx.x < 2 * D ? tot[threadIdx.x] : 0, parts + (size_t)blockIdx.x * 2 * D, sig);
 }
 
 // Block partials of one fold + polynomial pass: none when one block does it all.
 static unsigned fold_poly_grid(size_t n) {
   if (n <= 2) return 1;
   const size_t q = (next_pow2(n) >> 1) >> 1;
-  return q <= SMALL_PAIRS ? 1u : grid_for(q);
+  return q <= SMALL_PAIRS ? 1u : grid_for(2 * q);
 }
 
 // parts_buf: caller-provided room for the block partials (fold_poly_parts_words), or
@@ -397,7 +443,7 @@ static size_t fold_poly_t(const uint64_t* a_in, uint64_t* a_out, uint64_t* b, si
   uint64_t* pp = parts_buf ? parts_buf : parts.as<uint64_t>();
   {
     ProfScope prof(kernel_name("k_fold_poly", Ds, D), s, 8.0 * ((Ds + D) * (double)n + 2.0 * D * h));
-    k_fold_poly<Ds, D><<<g, RT, 0, s>>>(a_in, a_out, b, h, nhi, ww, om, g == 1 ? out : pp,
+    k_fold_poly<Ds, D><<<g, g == 1 ? reduce_threads(h) : RT, 0, s>>>(a_in, a_out, b, h, nhi, ww, om, g == 1 ? out : pp,
                                         g == 1 ? mailbox_take(out) : MailboxSig{});
     WHIR_HIP(hipGetLastError());
   }
@@ -519,22 +565,6 @@ __global__ __launch_bounds__(RT) void k_fold4(const uint64_t* a_in, uint64_t* a_
   }
 }
 
-// The value of lane CTRL[l] of each quad of lanes (quad_perm: two bits per lane l).
-template <int CTRL>
-__device__ __forceinline__ uint64_t quad_get(uint64_t v) {
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)v, CTRL, 0xf, 0xf, true);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(v >> 32), CTRL, 0xf, 0xf, true);
-  return ((uint64_t)hi << 32) | lo;
-}
-template <int CTRL, int D>
-__device__ __forceinline__ Ext<D> quad_get(const Ext<D>& v) {
-  Ext<D> r;
-#pragma unroll
-  for (int d = 0; d < D; d++) r.c[d] = quad_get<CTRL>(v.c[d]);
-  return r;
-}
-constexpr int quad_ctrl(int a, int b, int c, int d) { return a | b << 2 | c << 4 | d << 6; }
-
 // The second factor of a quad's lane: the quarter differences 2 - 0, 3 - 1, 3 - 2, 1 - 0,
 // and for lane 3 in place of its own quarter (3 - 2) - (1 - 0) as the first factor.
 template <int D>
@@ -582,14 +612,6 @@ __global__ __launch_bounds__(1024) void k_sc_pair(const uint64_t* a_in, uint64_t
   for (int j = 0; j < NP; j++) gl::wide_zero<D>(w[j]);
   const size_t q = L >> 2, l = threadIdx.x & 3;
   const size_t step = ((size_t)gridDim.x * blockDim.x) >> 2;
-  auto mac = [&](gl::Wide(&acc)[D], const Ext<Dx>& x, const Ext<D>& y) {
-    if constexpr (Dx == D) {
-      gl::emul_acc<D>(acc, x, y);
-    } else {
-#pragma unroll
-      for (int d = 0; d < D; d++) gl::wide_mac(acc[d], x.c[0], y.c[d]);
-    }
-  };
 #pragma unroll 1
   for (size_t i = (blockIdx.x * (size_t)blockDim.x + threadIdx.x) >> 2; i < q; i += step) {
     const size_t t = l * q + i;
@@ -609,10 +631,10 @@ __global__ __launch_bounds__(1024) void k_sc_pair(const uint64_t* a_in, uint64_t
       Ext<D> py, qy;
       quad_factors<Dx>(x, px, qx);
       quad_factors<D>(y, py, qy);
-      mac(w[0], px, py);
-      mac(w[1], qx, qy);
+      mulx_acc<Dx, D>(w[0], px, py);
+      mulx_acc<Dx, D>(w[1], qx, qy);
     } else {
-      mac(w[0], quad_factor2<Dx>(x), quad_factor2<D>(y));
+      mulx_acc<Dx, D>(w[0], quad_factor2<Dx>(x), quad_factor2<D>(y));
     }
   }
   Ext<D> v[NP];

@@ -424,10 +424,12 @@ int whir_sumcheck_polynomial_dev(int D, const uint64_t* a, const uint64_t* b, si
   API_BEGIN
   check_degree(D);
   hipStream_t s = thread_stream();
-  DevBuf o(2 * D * 8, s);
-  sumcheck_poly_dev(D, a, b, n, o.as<uint64_t>(), s);
-  WHIR_HIP(hipMemcpyAsync(out, o.ptr, 2 * D * 8, hipMemcpyDeviceToHost, s));
-  WHIR_HIP(hipStreamSynchronize(s));
+  // the sums land in the stream's mailbox: no copy, and the wait polls its flag
+  uint64_t* mb = result_mailbox(s);
+  mailbox_arm(s);
+  sumcheck_poly_dev(D, a, b, n, mb, s);
+  mailbox_wait(s);
+  memcpy(out, mb, 2 * D * 8);
   API_END
 }
 
@@ -470,10 +472,11 @@ int whir_fold_and_compute_polynomial_dev(int D, uint64_t* a, uint64_t* b, size_t
   API_BEGIN
   check_degree(D);
   hipStream_t s = thread_stream();
-  DevBuf o(2 * D * 8, s);
-  *new_len = fold_and_poly_dev(D, a, b, n, w, o.as<uint64_t>(), s);
-  WHIR_HIP(hipMemcpyAsync(out, o.ptr, 2 * D * 8, hipMemcpyDeviceToHost, s));
-  WHIR_HIP(hipStreamSynchronize(s));
+  uint64_t* mb = result_mailbox(s);
+  mailbox_arm(s);
+  *new_len = fold_and_poly_dev(D, a, b, n, w, mb, s);
+  mailbox_wait(s);
+  memcpy(out, mb, 2 * D * 8);
   API_END
 }
 

@@ -384,7 +384,7 @@ struct OpenLaunch {
 
 // Openings of at most this many values and nodes read their indices and weights in pinned
 // host memory.
-constexpr size_t OPEN_IN_PLACE = 4096;
+constexpr size_t OPEN_IN_PLACE = 8192;
 
 OpenLaunch open_rows_launch(const DevWitness& w, const std::vector<size_t>& idx, hipStream_t s, int D,
                             const uint64_t* wts, size_t off) {
