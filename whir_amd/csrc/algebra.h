@@ -71,18 +71,15 @@ size_t covview_words(int D, size_t np, size_t m, size_t nv);
 // np eq terms (points of nv elements, scalars), then m geometric terms; tables in buf.
 CovView covview_build_dev(int D, uint64_t* buf, size_t nv, const uint64_t* eq_points, const uint64_t* eq_scalars,
                           size_t np, const uint64_t* scalars, const uint64_t* points, size_t m, hipStream_t st);
-// The view of y folded by r1 then r2 (sumcheck_pair_dev's double fold): hi tables of
-// nhi / 4 elements written to out_hi (nt nhi / 4 elements).  Needs nhi >= 4.
-CovView covview_fold2_dev(int D, const CovView& v, const uint64_t* r1, const uint64_t* r2, uint64_t* out_hi,
-                          hipStream_t st);
 // y(i) for i < n into out.
 void covview_write_dev(int D, const CovView& v, uint64_t* out, size_t n, hipStream_t st);
-// sumcheck_pair_dev with b given by a view: mode 0 reads y from v instead of b; modes
-// 1-3 take v as the view of the covector ALREADY folded by (r1, r2) (covview_fold2_dev)
-// and write its values into b (length L), so b holds the folded covector afterwards.
+// sumcheck_pair_dev with b given by a view: mode 0 reads y from v instead of b; modes 1-3
+// fold v by (r1, r2) along with a (v covers 4 L elements).  Modes 1 and 2 write the folded high
+// tables to hi_out (nt nhi / 4 elements: with them v is the folded covector's view), mode 3
+// writes the folded covector's values into b (length L).
 void sumcheck_pair_view_dev(int mode, int Ds, int D, const uint64_t* a_in, uint64_t* a_out, uint64_t* b, size_t L,
-                            const uint64_t* r1, const uint64_t* r2, const CovView& v, uint64_t* dev_out,
-                            hipStream_t st);
+                            const uint64_t* r1, const uint64_t* r2, const CovView& v, uint64_t* hi_out,
+                            uint64_t* dev_out, hipStream_t st);
 
 // eval_eq (src/algebra/multilinear.rs:170-190): acc[x] += s * prod_i eq(z_i, x_i), x_0 = MSB.
 void eval_eq_dev(int D, uint64_t* acc, const uint64_t* point, size_t k, const uint64_t* scalar, hipStream_t st);

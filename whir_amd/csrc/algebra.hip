@@ -552,16 +552,41 @@ __device__ __forceinline__ Ext<D> view_at(const CovView& v, size_t i) {
   return r;
 }
 
-// The double fold alone, one output position per lane.  VIEW: b's folded values come
-// from the view v instead of from b.
+constexpr int VIEW_MAX_TERMS = 4;
+
+// The double fold alone, one output position per lane.  VIEW: b's folded values come from the
+// unfolded view v: the block folds the high-table entries of its 256 positions (at most 128, a
+// low table has at least two) into LDS first.
 template <int Ds, int D, bool VIEW>
 __global__ __launch_bounds__(RT) void k_fold4(const uint64_t* a_in, uint64_t* a_out, uint64_t* b, size_t L,
                                               Fold4<D> f, CovView v) {
-  for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < L; t += (size_t)gridDim.x * blockDim.x) {
-    const Ext<D> x = fold_twice<Ds, D>(a_in, t, L, f);
-    const Ext<D> y = VIEW ? view_at<D>(v, t) : fold_twice<D, D>(b, t, L, f);
-    st<D>(a_out, t, x);
-    st<D>(b, t, y);
+  __shared__ uint64_t hi[VIEW ? VIEW_MAX_TERMS * (RT / 2) * D : 1];
+  const size_t nhi = v.nhi >> 2;
+  const uint32_t cnt = (uint32_t)(v.sh >= 8 ? 1 : nhi < (RT >> v.sh) ? nhi : RT >> v.sh);
+  for (size_t t0 = blockIdx.x * (size_t)RT; t0 < L; t0 += (size_t)gridDim.x * RT) {
+    const size_t t = t0 + threadIdx.x, h0 = t0 >> v.sh;
+    if constexpr (VIEW) {
+      for (uint32_t e = threadIdx.x; e < v.nt * cnt; e += RT)
+        st<D>(hi, e, fold_twice<D, D>(v.hi + (size_t)(e / cnt) * v.nhi * D, h0 + e % cnt, nhi, f));
+      __syncthreads();
+    }
+    if (t < L) {
+      Ext<D> y;
+      if constexpr (VIEW) {
+        gl::Wide w[D];
+        gl::wide_zero<D>(w);
+        const size_t l = t & (((size_t)1 << v.sh) - 1);
+#pragma unroll 1
+        for (uint32_t k = 0; k < v.nt; k++)
+          gl::emul_acc<D>(w, ld<D>(hi, k * cnt + (uint32_t)((t >> v.sh) - h0)), ld<D>(v.lo, ((size_t)k << v.sh) + l));
+        y = gl::ext_reduce<D>(w);
+      } else {
+        y = fold_twice<D, D>(b, t, L, f);
+      }
+      st<D>(a_out, t, fold_twice<Ds, D>(a_in, t, L, f));
+      st<D>(b, t, y);
+    }
+    if constexpr (VIEW) __syncthreads();
   }
 }
 
@@ -743,18 +768,24 @@ void sumcheck_pair_dev(int mode, int Ds, int D, const uint64_t* a_in, uint64_t* 
 // (Qb = L/4 / 2^sh blocks per quarter): the inner products run against the low tables
 // (a base-field x costs D products per term, summed as 128-bit values and reduced once
 // per block), and the high tables enter once per block.  One GPU block per (a, h).
-constexpr int VIEW_MAX_TERMS = 4;
-
 template <int Ds, int D, bool FOLD, int NT>
 __global__ __launch_bounds__(RT) void k_view_pass(const uint64_t* a_in, uint64_t* a_out, size_t L, Fold4<D> f,
-                                                  CovView v, uint64_t* parts) {
+                                                  CovView v, uint64_t* hi_out, uint64_t* parts) {
   const size_t q = L >> 2, B = (size_t)1 << v.sh, Qb = q >> v.sh;
   const size_t a = blockIdx.x / Qb, h = blockIdx.x % Qb;
   const size_t base = a * q + h * B;
   // thread 4 t + b ends with term t of quarter b: its high-table factor is read here
   const unsigned et = threadIdx.x >> 2, eb = threadIdx.x & 3;
   Ext<D> hi = gl::ext_zero<D>();
-  if (et < NT) hi = ld<D>(v.hi, (size_t)et * v.nhi + eb * Qb + h);
+  if (et < NT) {
+    if constexpr (FOLD) {  // v is not folded yet: fold the entry, and keep it for the next pass
+      const size_t nhi = v.nhi >> 2, e = eb * Qb + h;
+      hi = fold_twice<D, D>(v.hi + et * v.nhi * D, e, nhi, f);
+      if (a == 0) st<D>(hi_out, et * nhi + e, hi);
+    } else {
+      hi = ld<D>(v.hi, (size_t)et * v.nhi + eb * Qb + h);
+    }
+  }
   Ext<D> P[NT];
   if constexpr (!FOLD && Ds == 1) {
     gl::Wide W[NT][D];
@@ -853,7 +884,7 @@ __global__ __launch_bounds__(1024) void k_view_reduce(const uint64_t* parts, siz
 
 template <int Ds, int D>
 static void view_pass_t(int mode, const uint64_t* a_in, uint64_t* a_out, size_t L, const uint64_t* r1,
-                        const uint64_t* r2, const CovView& v, uint64_t* out, hipStream_t s) {
+                        const uint64_t* r2, const CovView& v, uint64_t* hi_out, uint64_t* out, hipStream_t s) {
   const size_t Qb = (L >> 2) >> v.sh;
   const unsigned blocks = (unsigned)(4 * Qb);
   DevBuf parts((size_t)blocks * 4 * D * 8, s);
@@ -864,8 +895,8 @@ static void view_pass_t(int mode, const uint64_t* a_in, uint64_t* a_out, size_t 
     uint64_t* pp = parts.as<uint64_t>();
     auto go = [&](auto nt) {
       constexpr int NT = decltype(nt)::value;
-      if (mode == 0) k_view_pass<Ds, D, false, NT><<<blocks, RT, 0, s>>>(a_in, a_out, L, f, v, pp);
-      else k_view_pass<Ds, D, true, NT><<<blocks, RT, 0, s>>>(a_in, a_out, L, f, v, pp);
+      if (mode == 0) k_view_pass<Ds, D, false, NT><<<blocks, RT, 0, s>>>(a_in, a_out, L, f, v, hi_out, pp);
+      else k_view_pass<Ds, D, true, NT><<<blocks, RT, 0, s>>>(a_in, a_out, L, f, v, hi_out, pp);
     };
     switch (v.nt) {
       case 1: go(std::integral_constant<int, 1>{}); break;
@@ -881,24 +912,27 @@ static void view_pass_t(int mode, const uint64_t* a_in, uint64_t* a_out, size_t 
 }
 
 void sumcheck_pair_view_dev(int mode, int Ds, int D, const uint64_t* a_in, uint64_t* a_out, uint64_t* b, size_t L,
-                            const uint64_t* r1, const uint64_t* r2, const CovView& v, uint64_t* out, hipStream_t s) {
+                            const uint64_t* r1, const uint64_t* r2, const CovView& v, uint64_t* hi_out, uint64_t* out,
+                            hipStream_t s) {
   WHIR_REQUIRE(v.nt > 0 && v.nt <= VIEW_MAX_TERMS && v.hi && v.lo, "sumcheck pair: bad covector view");
-  WHIR_REQUIRE(((size_t)v.nhi << v.sh) == L, "sumcheck pair: covector view length mismatch");
+  const size_t nhi = mode == 0 ? v.nhi : v.nhi >> 2;
+  WHIR_REQUIRE(v.sh >= 1 && nhi > 0 && (nhi << v.sh) == L, "sumcheck pair: covector view length mismatch");
   if (mode == 3) {  // the double fold alone; it writes the view's values into b
     sc_pair_any<true>(mode, Ds, D, a_in, a_out, b, L, r1, r2, out, v, s);
     return;
   }
-  WHIR_REQUIRE(v.nhi >= 4 && mode >= 0 && mode <= 2, "sumcheck pair: covector view too short for a view pass");
+  WHIR_REQUIRE(nhi >= 4 && mode >= 0 && mode <= 2, "sumcheck pair: covector view too short for a view pass");
+  WHIR_REQUIRE(mode == 0 || hi_out, "sumcheck pair: no room for the folded high tables");
   if (Ds == D) {
     switch (D) {
-      case 1: return view_pass_t<1, 1>(mode, a_in, a_out, L, r1, r2, v, out, s);
-      case 2: return view_pass_t<2, 2>(mode, a_in, a_out, L, r1, r2, v, out, s);
-      case 3: return view_pass_t<3, 3>(mode, a_in, a_out, L, r1, r2, v, out, s);
+      case 1: return view_pass_t<1, 1>(mode, a_in, a_out, L, r1, r2, v, hi_out, out, s);
+      case 2: return view_pass_t<2, 2>(mode, a_in, a_out, L, r1, r2, v, hi_out, out, s);
+      case 3: return view_pass_t<3, 3>(mode, a_in, a_out, L, r1, r2, v, hi_out, out, s);
     }
   } else if (Ds == 1) {
     switch (D) {
-      case 2: return view_pass_t<1, 2>(mode, a_in, a_out, L, r1, r2, v, out, s);
-      case 3: return view_pass_t<1, 3>(mode, a_in, a_out, L, r1, r2, v, out, s);
+      case 2: return view_pass_t<1, 2>(mode, a_in, a_out, L, r1, r2, v, hi_out, out, s);
+      case 3: return view_pass_t<1, 3>(mode, a_in, a_out, L, r1, r2, v, hi_out, out, s);
     }
   }
   throw Error("sumcheck pair: extension degree must be 1, 2 or 3");
@@ -1516,50 +1550,56 @@ void covector_dev(int D, uint64_t* acc, size_t n, bool accumulate, const uint64_
 //   geo: hi[h] = t_j x_j^(h 2^sh), lo[l] = x_j^l.
 struct CovViewPlan {
   size_t np, m, nv, sh, nhi, nlo;
-  size_t in_z, in_s, in_x, in_t;  // input offsets (words)
-  size_t hi, lo;                  // table offsets (words)
+  size_t in_z, in_s, in_t, in_sq;  // input offsets (words); in_sq: per point x^(2^b), b < nv
+  size_t hi, lo;                   // table offsets (words)
 };
 
+// A block makes 256 consecutive entries of one table.  An entry is a product over the bits of
+// its index, (bit ? f1 : f0) per bit, the scalar in front for a hi table: the block has the
+// pairs (f0, f1) in LDS, forms the 16 products of each half of the low byte and the product of
+// the bits above it, and an entry is two products (the tables of 2^14 coefficients on MI355X
+// 4.1 us; 9.0 when every entry was a chain of its own products or a power by squaring).
 template <int D>
-__global__ void k_covview_tables(uint64_t* buf, CovViewPlan L, const uint64_t* in_dev, CovIn in_arg) {
-  size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-  const size_t nt = L.np + L.m, k1 = L.nv - L.sh;
-  if (e < nt * L.nhi) {
-    const size_t k = e / L.nhi, h = e % L.nhi;
-    Ext<D> v;
+__global__ __launch_bounds__(256) void k_covview_tables(uint64_t* buf, CovViewPlan L, const uint64_t* in_dev,
+                                                        CovIn in_arg) {
+  __shared__ uint64_t f[64 * 2 * D], half[32 * D], top[D];
+  const uint32_t tid = threadIdx.x;
+  const size_t bh = (L.nhi + 255) >> 8, bl = (L.nlo + 255) >> 8;
+  const size_t k = blockIdx.x / (bh + bl), c = blockIdx.x % (bh + bl);
+  const bool hi = c < bh;
+  const size_t chunk = hi ? c : c - bh, size = hi ? L.nhi : L.nlo;
+  const int bits = (int)(hi ? L.nv - L.sh : L.sh);
+  if (tid < (uint32_t)bits) {  // bit tid of the index
+    Ext<D> f0 = gl::ext_base<D>(1), f1;
     if (k < L.np) {
-      v = in_ld<D>(in_dev, in_arg, L.in_s, k);
-      for (size_t q = 0; q < k1; q++) {
-        const Ext<D> zq = in_ld<D>(in_dev, in_arg, L.in_z, k * L.nv + q);
-        v = gl::emul<D>(v, ((h >> (k1 - 1 - q)) & 1) ? zq : gl::esub<D>(gl::ext_base<D>(1), zq));
-      }
+      f1 = in_ld<D>(in_dev, in_arg, L.in_z, k * L.nv + (hi ? L.nv - L.sh : L.nv) - 1 - tid);
+      f0 = gl::esub<D>(f0, f1);
     } else {
-      const size_t j = k - L.np;
-      v = gl::emul<D>(in_ld<D>(in_dev, in_arg, L.in_t, j),
-                      gl::epow<D>(in_ld<D>(in_dev, in_arg, L.in_x, j), (uint64_t)h << L.sh));
+      f1 = in_ld<D>(in_dev, in_arg, L.in_sq, (k - L.np) * L.nv + (hi ? L.sh : 0) + tid);
     }
-    st<D>(buf + L.hi, e, v);
-    return;
+    st<D>(f, 2 * tid, f0);
+    st<D>(f, 2 * tid + 1, f1);
   }
-  e -= nt * L.nhi;
-  if (e >= nt * L.nlo) return;
-  const size_t k = e / L.nlo, l = e % L.nlo;
-  Ext<D> v;
-  if (k < L.np) {
-    v = gl::ext_base<D>(1);
-    for (size_t q = 0; q < L.sh; q++) {
-      const Ext<D> zq = in_ld<D>(in_dev, in_arg, L.in_z, k * L.nv + k1 + q);
-      v = gl::emul<D>(v, ((l >> (L.sh - 1 - q)) & 1) ? zq : gl::esub<D>(gl::ext_base<D>(1), zq));
-    }
-  } else {
-    v = gl::epow<D>(in_ld<D>(in_dev, in_arg, L.in_x, k - L.np), l);
+  Ext<D> v = gl::ext_base<D>(1);
+  if (tid == 64 && hi) v = k < L.np ? in_ld<D>(in_dev, in_arg, L.in_s, k) : in_ld<D>(in_dev, in_arg, L.in_t, k - L.np);
+  __syncthreads();
+  if (tid < 32 || tid == 64) {  // bits 0..3, bits 4..7, and from 8 on
+    const size_t e = tid < 32 ? tid & 15 : chunk;
+    const int b0 = tid < 16 ? 0 : tid < 32 ? 4 : 8, b1 = tid < 32 ? b0 + 4 : bits;
+#pragma unroll 1
+    for (int b = b0; b < b1 && b < bits; b++) v = gl::emul<D>(v, ld<D>(f, 2 * b + ((e >> (b - b0)) & 1)));
+    st<D>(tid < 32 ? half : top, tid < 32 ? tid : 0, v);
   }
-  st<D>(buf + L.lo, e, v);
+  __syncthreads();
+  const size_t e = (chunk << 8) + tid;
+  if (e < size)
+    st<D>(buf + (hi ? L.hi : L.lo), k * size + e,
+          gl::emul<D>(gl::emul<D>(ld<D>(half, tid & 15), ld<D>(half, 16 + (tid >> 4))), ld<D>(top, 0)));
 }
 
 size_t covview_words(int D, size_t np, size_t m, size_t nv) {
   const size_t sh = nv - nv / 2, nt = np + m;
-  return (np * nv + np + 2 * m) * D + nt * (((size_t)1 << (nv - sh)) + ((size_t)1 << sh)) * D;
+  return (np * nv + np + m + m * nv) * D + nt * (((size_t)1 << (nv - sh)) + ((size_t)1 << sh)) * D;
 }
 
 template <int D>
@@ -1577,10 +1617,17 @@ static CovView covview_build_t(uint64_t* buf, size_t nv, const uint64_t* eq_poin
   in.insert(in.end(), eq_points, eq_points + np * nv * D);
   L.in_s = in.size();
   in.insert(in.end(), eq_scalars, eq_scalars + np * D);
-  L.in_x = in.size();
-  in.insert(in.end(), points, points + m * D);
   L.in_t = in.size();
   in.insert(in.end(), scalars, scalars + m * D);
+  L.in_sq = in.size();
+  for (size_t j = 0; j < m; j++) {
+    Ext<D> x;
+    for (int d = 0; d < D; d++) x.c[d] = points[j * D + d];
+    for (size_t b = 0; b < nv; b++) {
+      in.insert(in.end(), x.c, x.c + D);
+      x = gl::emul<D>(x, x);
+    }
+  }
   const bool by_arg = in.size() <= COV_ARG_WORDS;
   const size_t nt = np + m;
   L.hi = in.size();  // the input region stays reserved either way (covview_words)
@@ -1588,8 +1635,8 @@ static CovView covview_build_t(uint64_t* buf, size_t nv, const uint64_t* eq_poin
   CovIn args{};
   if (by_arg) std::copy(in.begin(), in.end(), args.w);
   else upload_async(buf, in.data(), in.size() * 8, s);
-  const size_t entries = nt * (L.nhi + L.nlo);
-  k_covview_tables<D><<<blocks_for(entries, RT), RT, 0, s>>>(buf, L, by_arg ? nullptr : buf, args);
+  const size_t blocks = nt * (((L.nhi + 255) >> 8) + ((L.nlo + 255) >> 8));
+  k_covview_tables<D><<<(unsigned)blocks, 256, 0, s>>>(buf, L, by_arg ? nullptr : buf, args);
   WHIR_HIP(hipGetLastError());
   CovView v;
   v.hi = buf + L.hi;
@@ -1612,35 +1659,9 @@ CovView covview_build_dev(int D, uint64_t* buf, size_t nv, const uint64_t* eq_po
 }
 
 template <int D>
-__global__ void k_covview_fold2(const uint64_t* hi, uint64_t* out, size_t nt, size_t nhi, Fold4<D> f) {
-  const size_t q = nhi >> 2;
-  const size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-  if (e >= nt * q) return;
-  const size_t k = e / q, t = e % q;
-  st<D>(out, e, fold_twice<D, D>(hi + k * nhi * D, t, q, f));
-}
-
-template <int D>
 __global__ void k_covview_write(CovView v, uint64_t* out, size_t n) {
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
     st<D>(out, i, view_at<D>(v, i));
-}
-
-CovView covview_fold2_dev(int D, const CovView& v, const uint64_t* r1, const uint64_t* r2, uint64_t* out_hi,
-                          hipStream_t s) {
-  WHIR_REQUIRE(v.nt > 0 && v.nhi >= 4, "covector view: nothing left to fold in the high tables");
-  const size_t n = (size_t)v.nt * (v.nhi >> 2);
-  switch (D) {
-    case 1: k_covview_fold2<1><<<blocks_for(n, RT), RT, 0, s>>>(v.hi, out_hi, v.nt, v.nhi, host_fold4<1>(r1, r2)); break;
-    case 2: k_covview_fold2<2><<<blocks_for(n, RT), RT, 0, s>>>(v.hi, out_hi, v.nt, v.nhi, host_fold4<2>(r1, r2)); break;
-    case 3: k_covview_fold2<3><<<blocks_for(n, RT), RT, 0, s>>>(v.hi, out_hi, v.nt, v.nhi, host_fold4<3>(r1, r2)); break;
-    default: throw Error("covector view: extension degree must be 1, 2 or 3");
-  }
-  WHIR_HIP(hipGetLastError());
-  CovView f = v;
-  f.hi = out_hi;
-  f.nhi = v.nhi >> 2;
-  return f;
 }
 
 void covview_write_dev(int D, const CovView& v, uint64_t* out, size_t n, hipStream_t s) {

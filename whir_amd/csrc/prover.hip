@@ -534,12 +534,15 @@ std::vector<E<D>> sumcheck_prove_pairs(Transcript& t, const SumcheckCfg& sc, int
   CovView cur = view ? *view : CovView{};  // cur.nt == 0: b holds the covector
   DevBuf folded_hi[2];                      // high tables of the folded views, in turn
   int fh = 0;
-  // The view folded by the pending pair (the pass that folds the vectors uses it).
-  auto fold_view = [&](const E<D>& r1, const E<D>& r2) {
+  // A pass that folds the vectors reads the view as it is and leaves its folded high tables here.
+  auto fold_room = [&] {
     folded_hi[fh] = DevBuf((size_t)cur.nt * (cur.nhi >> 2) * D * 8, s);
-    const CovView f = covview_fold2_dev(D, cur, r1.c, r2.c, folded_hi[fh].as<uint64_t>(), s);
+    return folded_hi[fh].as<uint64_t>();
+  };
+  auto folded = [&] {
+    cur.hi = folded_hi[fh].as<uint64_t>();
+    cur.nhi >>= 2;
     fh ^= 1;
-    return f;
   };
   // A view pass needs four high-table blocks per quarter (two more bits to fold).
   auto view_ok = [&](size_t folds) { return cur.nt && (cur.nhi >> (2 * folds)) >= 4; };
@@ -573,12 +576,12 @@ std::vector<E<D>> sumcheck_prove_pairs(Transcript& t, const SumcheckCfg& sc, int
       // round k's polynomial and round k+1's coefficients, folding the pending pair first
       if (cur.nt && !view_ok(pend.empty() ? 0 : 1)) materialize();
       if (pend.empty()) {
-        if (cur.nt) sumcheck_pair_view_dev(0, a_Ds, D, a_src, a, b, len, nullptr, nullptr, cur, mbox, s);
+        if (cur.nt) sumcheck_pair_view_dev(0, a_Ds, D, a_src, a, b, len, nullptr, nullptr, cur, nullptr, mbox, s);
         else sumcheck_pair_dev(0, a_Ds, D, a_src, a, b, len, nullptr, nullptr, mbox, s);
       } else {
         if (cur.nt) {
-          cur = fold_view(pend[0], pend[1]);
-          sumcheck_pair_view_dev(1, a_Ds, D, a_src, a, b, len, pend[0].c, pend[1].c, cur, mbox, s);
+          sumcheck_pair_view_dev(1, a_Ds, D, a_src, a, b, len, pend[0].c, pend[1].c, cur, fold_room(), mbox, s);
+          folded();
         } else {
           sumcheck_pair_dev(1, a_Ds, D, a_src, a, b, len, pend[0].c, pend[1].c, mbox, s);
         }
@@ -603,8 +606,8 @@ std::vector<E<D>> sumcheck_prove_pairs(Transcript& t, const SumcheckCfg& sc, int
       if (pend.size() == 2) {
         if (cur.nt && !view_ok(1)) materialize();
         if (cur.nt) {
-          cur = fold_view(pend[0], pend[1]);
-          sumcheck_pair_view_dev(2, a_Ds, D, a_src, a, b, len, pend[0].c, pend[1].c, cur, mbox, s);
+          sumcheck_pair_view_dev(2, a_Ds, D, a_src, a, b, len, pend[0].c, pend[1].c, cur, fold_room(), mbox, s);
+          folded();
         } else {
           sumcheck_pair_dev(2, a_Ds, D, a_src, a, b, len, pend[0].c, pend[1].c, mbox, s);
         }
@@ -630,9 +633,8 @@ std::vector<E<D>> sumcheck_prove_pairs(Transcript& t, const SumcheckCfg& sc, int
   if (pend.size() == 2) {
     if (cur.nt && cur.nhi < 4) materialize();
     if (cur.nt) {
-      const CovView f = fold_view(pend[0], pend[1]);
+      sumcheck_pair_view_dev(3, a_Ds, D, a_src, a, b, len, pend[0].c, pend[1].c, cur, nullptr, nullptr, s);  // writes b
       cur = CovView{};
-      sumcheck_pair_view_dev(3, a_Ds, D, a_src, a, b, len, pend[0].c, pend[1].c, f, nullptr, s);  // writes b
     } else {
       sumcheck_pair_dev(3, a_Ds, D, a_src, a, b, len, pend[0].c, pend[1].c, nullptr, s);
     }
