@@ -27,7 +27,7 @@ def test_tree_of_every_shape_matches_oracle(D, log, cols):
     assert dn.to_array(np.uint8).tobytes() == exp
 
 
-@pytest.mark.parametrize("log", [1, 2, 8, 9, 10, 11, 12, 16, 17, 19])
+@pytest.mark.parametrize("log", [1, 2, 8, 9, 10, 11, 12, 16, 17, 18, 19])
 def test_levels_above_given_leaves_match_oracle(log):
     leaves = np.random.default_rng(log).integers(0, 256, size=32 << log, dtype=np.uint8).tobytes()
     assert W.merkle_commit(W.HASH_BLAKE3, leaves) == O.merkle_commit(W.HASH_BLAKE3, leaves)

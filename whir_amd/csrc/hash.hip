@@ -517,16 +517,13 @@ static bool b3q_enabled() {
   }();
   return on;
 }
-// A launch takes the quad kernel while its first phase has at most this many lanes
-// (one wave per SIMD): there each level costs one compression's latency, which the
-// quads cut; on more lanes the launch is bound by instruction issue, and the quads'
-// extra instructions (DPP moves, per-lane message reads, four lanes of G) cost more
-// than they save.  Measured on MI355X per launch, pairs per lane (one lane / quad):
-// one block 16.0 / 10.1 us, 2^16 nodes (128 blocks) 19.2 / 12.9, 2^17 nodes 19.4 /
-// 13.6, 2^18 nodes (2^17 lanes) 25.1 / 26.0; eight nodes per lane from 2^19 nodes
-// (which k_merkle_wide takes first anyway) 38.4 us as quads against 32.2 us for
-// k_merkle_wide and the quad launch above it.
-static constexpr size_t B3Q_MAX_LANES = (size_t)1 << 16;
+// A launch takes the quad kernel while its first phase makes at most this many nodes (two
+// blocks of 1024 threads a CU): there a level costs one compression's latency, which the quads
+// cut; with more the launch is bound by instruction issue, and the quads' extra instructions
+// (DPP moves, message reads by every lane, four lanes of G) cost more than they save.  Measured
+// on MI355X per launch (one lane a node / quad): 2^7 nodes to the root 14.5 us / 8.4, 2^8 15.2 /
+// 9.0, nine levels of 2^16 and 2^17 nodes 20 / 12.2, of 2^18 26 / 19.
+static constexpr size_t B3Q_MAX_LANES = (size_t)1 << 17;
 
 // Three Merkle levels above a level of width w (w % 2^11 == 0): lane g reduces nodes
 // 8g..8g+7 to one in registers and stores the seven nodes it makes.  No lane idles
