@@ -115,7 +115,8 @@ int whir_rs_interleaved_encode_dev(int degree, const uint64_t *messages, size_t 
  * on the schedule.  Pinned schedules are used whether or not tuning is on.
  * Variants are 2-bit masks (bit 1: LDS padding, bit 0: radix 16); tiles are u64
  * words of LDS (4096, or 8192 where the device allows it); log_c1 = 0 for shapes
- * with log2 C <= 11 (one pass). */
+ * with log2 C <= 11 (one pass).  A pinned schedule runs the butterfly kernels; shapes
+ * whose table entry says "matrix_cores": true are faster left unpinned. */
 int whir_ntt_autotune(int enable);
 int whir_ntt_set_schedule(int degree, size_t log_n, size_t log_c, size_t num_messages, int log_c1, int variant1,
                           int tile1, int variant2, int tile2);
