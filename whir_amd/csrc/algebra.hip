@@ -1731,7 +1731,7 @@ void geometric_accumulate_dev(int D, uint64_t* acc, size_t n, const uint64_t* sc
 // 27 KB of a lane that steps its own power through sixteen unrolled elements.
 static constexpr int UNI_MP = 4;   // points per launch
 static constexpr int UNI_MV = 16;  // vectors per launch, times points (both rounded up to a power of two)
-static constexpr int UNI_PW = 32;  // squares x^(2^b): vectors of less than 2^32 elements
+static constexpr int UNI_PW = 32;  // squares x^(2^b): vectors of up to 2^32 elements
 static constexpr int UNI_K = 16;   // elements per thread of a segment of k_uni_many
 
 // Per point: the squares x^(2^b), then the powers x^(k T).  MP points (at most 3.6 KB, 0.7 to
@@ -1881,7 +1881,7 @@ static void uni_launch(const uint64_t* const* c, int count, size_t n, const uint
   const size_t S = (size_t)K << U.lt, segs = (n + S - 1) / S;
   U.G = (segs + MAX_BLOCKS - 1) / MAX_BLOCKS;
   const size_t nb = (segs + U.G - 1) / U.G;
-  WHIR_REQUIRE((uint64_t)(nb - 1) * U.G * ((uint64_t)K << U.lt) < ((uint64_t)1 << UNI_PW), "univariate: vector too long");
+  WHIR_REQUIRE(n <= ((size_t)1 << UNI_PW), "univariate: vector too long");
   for (int j = 0; j < m; j++) {
     Ext<D> p, k = gl::ext_base<D>(1);
     for (int d = 0; d < D; d++) p.c[d] = xs[j * D + d];
