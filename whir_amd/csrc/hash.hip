@@ -21,6 +21,7 @@
 #include <type_traits>
 #include "hash_dev.h"
 #include "keccak_host.h"
+#include "tree_plan.h"
 
 #include <algorithm>
 #include <cstring>
@@ -227,8 +228,6 @@ void gather_hashes_dev(const uint8_t* nodes, const uint64_t* idx, size_t k, uint
   WHIR_HIP(hipGetLastError());
 }
 
-static constexpr int MERKLE_THREADS = 256;
-static constexpr int MERKLE_SPAN_LOG = 11;  // input nodes per block: 256 lanes x 8
 
 // 64-byte node pair (two 8-word digests) as a hash input.
 struct PairReader {
@@ -294,19 +293,11 @@ __device__ __forceinline__ void reduce_levels(uint32_t (&h)[NH][8], uint8_t* nod
 // lane, every lane busy) to one in registers; after it, one level per phase (lane i
 // hashes the pair 2i, 2i + 1 from LDS), which keeps the chain of dependent hashes
 // short once few nodes are left.
-// Largest first-phase group (2^G nodes per lane).  Eight for every engine: for the
-// Keccak engines four-node groups (122 instead of 180 registers) measured 4% slower
-// on MI355X and pairs 40% slower, the longer chains of dependent hashes costing more
-// than the occupancy gained.
-template <int ENG>
-constexpr int merkle_gmax() { return 3; }
-static int merkle_gmax_rt(int) { return 3; }
-
 template <int ENG>
 __global__ __launch_bounds__(MERKLE_THREADS) void k_merkle_sub(uint8_t* __restrict__ nodes, size_t W, size_t w,
                                                                int L, int G1, uint32_t* root_out, BatchTab tab,
                                                                MailboxSig sig) {
-  constexpr int NH = 1 << merkle_gmax<ENG>();
+  constexpr int NH = 1 << MERKLE_GMAX;
   __shared__ uint32_t buf[2][MERKLE_THREADS][8];
   size_t blk = blockIdx.x;
   if (tab.nodes) {
@@ -455,7 +446,6 @@ __device__ __forceinline__ uint32_t b3q_at(uint32_t node) { return (node >> 1) *
 // after level, to one node, through `dst` (half as large) and back; quad i makes nodes i, i +
 // quads, ... of each level and stores them to the tree.  Whole block; returns where the last
 // node is.
-constexpr int B3Q_THREADS = 4 * MERKLE_THREADS;
 __device__ __forceinline__ uint32_t* b3q_levels(uint32_t* src, uint32_t* dst, const B3QLane& ql, uint32_t* nodes32,
                                                 size_t W, size_t width, size_t first, int L) {
   const uint32_t q = threadIdx.x & 3, qi = threadIdx.x >> 2, nq = blockDim.x >> 2;
@@ -484,8 +474,6 @@ __device__ __forceinline__ uint32_t* b3q_levels(uint32_t* src, uint32_t* dst, co
 }
 
 // k_merkle_sub for BLAKE3 with a quad per node (pairs only: G1 = 1), four times the threads.
-// A level of 2^10 nodes goes to the root in one launch, its first level in two rounds.
-constexpr int B3Q_MAX_L = 10;
 __global__ __launch_bounds__(B3Q_THREADS) void k_merkle_sub_b3q(uint8_t* __restrict__ nodes, size_t W, size_t w,
                                                                  int L, uint32_t* root_out, BatchTab tab,
                                                                  MailboxSig sig) {
@@ -517,14 +505,6 @@ static bool b3q_enabled() {
   }();
   return on;
 }
-// A launch takes the quad kernel while its first phase makes at most this many nodes (two
-// blocks of 1024 threads a CU): there a level costs one compression's latency, which the quads
-// cut; with more the launch is bound by instruction issue, and the quads' extra instructions
-// (DPP moves, message reads by every lane, four lanes of G) cost more than they save.  Measured
-// on MI355X per launch (one lane a node / quad): 2^7 nodes to the root 14.5 us / 8.4, 2^8 15.2 /
-// 9.0, nine levels of 2^16 and 2^17 nodes 20 / 12.2, of 2^18 26 / 19.
-static constexpr size_t B3Q_MAX_LANES = (size_t)1 << 17;
-
 // Three Merkle levels above a level of width w (w % 2^11 == 0): lane g reduces nodes
 // 8g..8g+7 to one in registers and stores the seven nodes it makes.  No lane idles
 // and nothing waits at a barrier, which matters on levels wide enough to keep every
@@ -550,11 +530,6 @@ __global__ __launch_bounds__(MERKLE_THREADS) void k_merkle_wide(uint8_t* __restr
   reduce_levels<3, ENG, 8>(h, nodes, W, w, f);
 }
 
-// Levels at least this wide go through k_merkle_wide (2^16 lanes and more: a wave or
-// more per SIMD).  Measured on MI355X, d = 26 SHA3 proofs: 20.6 -> 19.2 ms with 2^19
-// or 2^18, 19.6 ms with 2^20; BLAKE3 trees, latency-bound at these widths, unchanged.
-static constexpr size_t MERKLE_WIDE_MIN = (size_t)1 << 19;
-
 // Merkle levels above a level of width w (a power of two) already in place.  The
 // root also goes to root_out (32 bytes) when given.  With a batch table, the same
 // levels of `count` trees (root i to tab.roots + 32 i).  With stop > 1 the launches end
@@ -568,44 +543,33 @@ static size_t merkle_from(int engine, uint8_t* nodes, size_t W, size_t w, hipStr
     if (root_out) WHIR_HIP(hipMemcpyAsync(root_out, nodes + 32 * (2 * W - 2), 32, hipMemcpyDefault, st));
     return w;
   }
-  while (w >= MERKLE_WIDE_MIN) {
-    const size_t blocks = w / ((size_t)MERKLE_THREADS << 3);
-    ProfScope prof("k_merkle_wide", st, 32.0 * (double)(w + (w >> 1) + (w >> 2) + (w >> 3)) * count);
-    tab.per = (uint32_t)blocks;
-    engine_switch(engine, [&](auto E) {
-      k_merkle_wide<decltype(E)::value><<<(unsigned)(blocks * count), MERKLE_THREADS, 0, st>>>(nodes, W, w, tab);
-    });
-    WHIR_HIP(hipGetLastError());
-    w >>= 3;
-  }
+  const bool quads = engine == ENG_BLAKE3 && b3q_enabled();
   while (w > stop) {
-    // Wide levels: eight nodes per lane first (2^11 per block); otherwise pairs
-    // (2^9 per block), which has the shortest chain of dependent hashes.
-    const int G1 = w >= ((size_t)MERKLE_THREADS << MERKLE_SPAN_LOG) ? merkle_gmax_rt(engine) : 1;
-    const bool quads = engine == ENG_BLAKE3 && b3q_enabled() && G1 == 1;
-    const int maxL = quads && w == ((size_t)1 << B3Q_MAX_L) ? B3Q_MAX_L : MERKLE_SPAN_LOG - 3 + G1;
-    int L = 0;
-    while (L < maxL && ((size_t)2 << L) <= w && (w >> (L + 1)) >= stop) L++;
-    const size_t blocks = w >> L;
-    const size_t lanes = ((size_t)1 << L) >> std::min(L, G1);  // nodes made by the first phase
-    const bool quad = quads && blocks * count * lanes <= B3Q_MAX_LANES;
-    const unsigned threads = quad ? (unsigned)std::max<size_t>(64, std::min<size_t>(B3Q_THREADS, 4 * lanes))
-                                  : (unsigned)std::max<size_t>(64, std::min<size_t>(MERKLE_THREADS, lanes));
-    ProfScope prof(quad ? "k_merkle_sub_b3q" : "k_merkle_sub", st, 32.0 * (double)(2 * w - (w >> L)) * count);
-    tab.per = (uint32_t)blocks;
-    uint32_t* ro = blocks == 1 ? (tab.nodes ? (uint32_t*)tab.roots : (uint32_t*)root_out) : nullptr;
-    // The launch that makes a single tree's root is the last of the commit.
-    const MailboxSig sig = blocks == 1 && !tab.nodes && ro ? mailbox_take(ro) : MailboxSig{};
-    if (quad) {
-      k_merkle_sub_b3q<<<(unsigned)(blocks * count), threads, 0, st>>>(nodes, W, w, L, ro, tab, sig);
-    } else {
+    const MerkleStep p = merkle_step(quads, w, count, stop);
+    const unsigned grid = (unsigned)(p.blocks * count);
+    const double bytes = 32.0 * (double)(2 * w - (w >> p.L)) * count;
+    tab.per = (uint32_t)p.blocks;
+    if (p.kernel == MerkleStep::WIDE) {
+      ProfScope prof("k_merkle_wide", st, bytes);
       engine_switch(engine, [&](auto E) {
-        k_merkle_sub<decltype(E)::value><<<(unsigned)(blocks * count), threads, 0, st>>>(nodes, W, w, L, G1, ro,
-                                                                                         tab, sig);
+        k_merkle_wide<decltype(E)::value><<<grid, p.threads, 0, st>>>(nodes, W, w, tab);
       });
+    } else {
+      const bool quad = p.kernel == MerkleStep::SUB_QUAD;
+      ProfScope prof(quad ? "k_merkle_sub_b3q" : "k_merkle_sub", st, bytes);
+      uint32_t* ro = p.blocks == 1 ? (tab.nodes ? (uint32_t*)tab.roots : (uint32_t*)root_out) : nullptr;
+      // The launch that makes a single tree's root is the last of the commit.
+      const MailboxSig sig = p.blocks == 1 && !tab.nodes && ro ? mailbox_take(ro) : MailboxSig{};
+      if (quad) {
+        k_merkle_sub_b3q<<<grid, p.threads, 0, st>>>(nodes, W, w, p.L, ro, tab, sig);
+      } else {
+        engine_switch(engine, [&](auto E) {
+          k_merkle_sub<decltype(E)::value><<<grid, p.threads, 0, st>>>(nodes, W, w, p.L, p.G, ro, tab, sig);
+        });
+      }
     }
     WHIR_HIP(hipGetLastError());
-    w >>= L;
+    w >>= p.L;
   }
   return w;
 }
