@@ -16,6 +16,8 @@ pytestmark = pytest.mark.gpu
 SHAPES = [
     (256, 15, 4, 1), (257, 15, 4, 1),  # 2^12 rows: a level of 2^10 nodes, in one launch up to 256 trees
     (257, 11, 2, 1),                   # 2^10 rows of four words: the same level above separate leaves
+    (128, 12, 4, 1), (129, 12, 4, 1), (513, 14, 6, 1),  # 2^9 rows: a tree is one block of a row per lane
+    (65, 13, 4, 1),                    # 2^10 rows of the same kernel, two nodes a tree left
 ]
 
 

@@ -587,7 +587,6 @@ void merkle_build_dev(int engine, uint8_t* nodes, size_t num_leaves, hipStream_t
 // with the two Merkle levels above them: lane g hashes rows 4g..4g+3, their two
 // parents and the grandparent, all in registers, reading each row's words straight
 // from HBM (for a fixed word, consecutive lanes read consecutive rows).
-static constexpr int TREE_THREADS = 256;
 
 template <int D>
 __device__ __forceinline__ void row_block(const uint64_t* __restrict__ cw, size_t N, size_t r, size_t b,
@@ -810,7 +809,6 @@ __global__ __launch_bounds__(B3Q_THREADS) void k_leaves_tree_b3q(const uint64_t*
 }
 
 // Between the two: one row per lane, then the block's 2^9 digests paired to one by quads.
-constexpr int B3H_LOG = 9;
 template <int D>
 __global__ __launch_bounds__(1 << B3H_LOG) void k_leaves_tree_b3h(const uint64_t* __restrict__ cw, size_t N, size_t M,
                                                                   uint8_t* __restrict__ nodes, BatchTab tab) {
@@ -852,40 +850,36 @@ template <int D>
 static size_t commit_cols_t(int engine, const uint64_t* cw, size_t N, size_t M, uint8_t* nodes, hipStream_t st,
                             uint8_t* root_out, BatchTab tab = {}, size_t count = 1) {
   const size_t W = M * D;
-  // Per commit (leaves and tree, 16 Fp2 columns, MI355X), one wave per 256 rows / one lane per
-  // row / a quad per row: 2^12 rows 38 / - / 20 us, 2^16 43 / 30 / 25, 2^17 48 / 32 / 42, 2^18
-  // 52 / 49 / 73, 2^19 77 / 79, 2^20 144 / 137, 2^21 235 / 244; rows of six blocks (Fp3) 2^19
-  // 110 / 106, 2^20 202 / 187, 2^21 339 / 333.
-  if (b3q_enabled() && N * count <= ((size_t)1 << 16)) {
-    int L = 0;
-    while (L < 8 && ((size_t)2 << L) <= N) L++;
-    tab.per = (uint32_t)(N >> L);
-    uint32_t* ro = tab.per == 1 ? (tab.nodes ? (uint32_t*)tab.roots : (uint32_t*)root_out) : nullptr;
-    const MailboxSig sig = tab.per == 1 && !tab.nodes && ro ? mailbox_take(ro) : MailboxSig{};
-    ProfScope prof(kernel_name("k_leaves_tree_b3q", D), st, (8.0 * (double)W * N + 64.0 * N) * count);
-    k_leaves_tree_b3q<D><<<tab.per * (unsigned)count, std::max(64, 4 << L), 0, st>>>(cw, N, M, nodes, L, ro, tab, sig);
-    WHIR_HIP(hipGetLastError());
-    return tab.per == 1 ? 0 : N >> L;
-  }
-  if (b3q_enabled() && N >= (1 << B3H_LOG) && N * count <= ((size_t)1 << (W >= 48 ? 21 : 18))) {
-    tab.per = (uint32_t)(N >> B3H_LOG);
-    ProfScope prof(kernel_name("k_leaves_tree_b3h", D), st, (8.0 * (double)W * N + 64.0 * N) * count);
-    k_leaves_tree_b3h<D><<<tab.per * (unsigned)count, 1 << B3H_LOG, 0, st>>>(cw, N, M, nodes, tab);
-    WHIR_HIP(hipGetLastError());
-    return N >> B3H_LOG;
-  }
-  tab.per = blocks_for(N / 4, TREE_THREADS);
-  const unsigned grid = tab.per * (unsigned)count;
-  const double bytes = (8.0 * (double)W * N + 32.0 * (N + N / 2 + N / 4)) * count;
-  if (N >= 256) {
-    ProfScope prof(kernel_name("k_leaves_tree_b3w", D), st, bytes);
-    k_leaves_tree_b3w<D><<<grid, TREE_THREADS, 0, st>>>(cw, N, M, nodes, tab);
-  } else {
-    ProfScope prof(kernel_name("k_leaves_tree_b3", D), st, bytes);
-    k_leaves_tree_b3<D><<<grid, TREE_THREADS, 0, st>>>(cw, N, M, nodes, tab);
+  const LeafStep p = leaf_step(b3q_enabled(), N, W, count);
+  tab.per = (uint32_t)p.blocks;
+  const unsigned grid = (unsigned)(p.blocks * count);
+  const double rows = 8.0 * (double)W * N;
+  switch (p.kernel) {
+    case LeafStep::QUAD_ROW: {
+      uint32_t* ro = p.top ? nullptr : (tab.nodes ? (uint32_t*)tab.roots : (uint32_t*)root_out);
+      const MailboxSig sig = !tab.nodes && ro ? mailbox_take(ro) : MailboxSig{};
+      ProfScope prof(kernel_name("k_leaves_tree_b3q", D), st, (rows + 64.0 * N) * count);
+      k_leaves_tree_b3q<D><<<grid, p.threads, 0, st>>>(cw, N, M, nodes, p.L, ro, tab, sig);
+      break;
+    }
+    case LeafStep::LANE_ROW: {
+      ProfScope prof(kernel_name("k_leaves_tree_b3h", D), st, (rows + 64.0 * N) * count);
+      k_leaves_tree_b3h<D><<<grid, p.threads, 0, st>>>(cw, N, M, nodes, tab);
+      break;
+    }
+    case LeafStep::WAVE: {
+      ProfScope prof(kernel_name("k_leaves_tree_b3w", D), st, (rows + 32.0 * (N + N / 2 + N / 4)) * count);
+      k_leaves_tree_b3w<D><<<grid, p.threads, 0, st>>>(cw, N, M, nodes, tab);
+      break;
+    }
+    case LeafStep::LANE_FOUR: {
+      ProfScope prof(kernel_name("k_leaves_tree_b3", D), st, (rows + 32.0 * (N + N / 2 + N / 4)) * count);
+      k_leaves_tree_b3<D><<<grid, p.threads, 0, st>>>(cw, N, M, nodes, tab);
+      break;
+    }
   }
   WHIR_HIP(hipGetLastError());
-  return N / 4;
+  return p.top;
 }
 
 void commit_cols_dev(int engine, int D, const uint64_t* cw, size_t N, size_t M, uint8_t* nodes, hipStream_t st,

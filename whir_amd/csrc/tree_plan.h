@@ -68,4 +68,35 @@ inline MerkleStep merkle_step(bool quads, size_t w, size_t count, size_t stop) {
   return {MerkleStep::SUB, L, G, w >> L, (unsigned)std::max<size_t>(64, std::min<size_t>(MERKLE_THREADS, made))};
 }
 
+// The launch that hashes the rows of `count` BLAKE3 codewords of N rows (a power of two >= 4) of
+// `words` words, and makes the first levels above them: `blocks` blocks a tree, each 2^L rows
+// to one node (the wave kernels: rows in groups of four).  top: the width of the last level
+// made, 0 when the launch hands the root over.
+struct LeafStep {
+  enum Kernel { QUAD_ROW, LANE_ROW, WAVE, LANE_FOUR } kernel;
+  int L;
+  size_t blocks;
+  unsigned threads;
+  size_t top;
+};
+constexpr int B3H_LOG = 9;         // log2 rows of a block with one lane per row
+constexpr int TREE_THREADS = 256;  // of the wave kernels
+
+// Per commit (leaves and tree, 16 Fp2 columns, MI355X), one wave per 256 rows / one lane per
+// row / a quad per row: 2^12 rows 38 / - / 20 us, 2^16 43 / 30 / 25, 2^17 48 / 32 / 42, 2^18
+// 52 / 49 / 73, 2^19 77 / 79, 2^20 144 / 137, 2^21 235 / 244; rows of six blocks (Fp3) 2^19
+// 110 / 106, 2^20 202 / 187, 2^21 339 / 333.
+inline LeafStep leaf_step(bool quads, size_t N, size_t words, size_t count) {
+  if (quads && N * count <= ((size_t)1 << 16)) {
+    const int L = merkle_levels(N, 1, 8);
+    const size_t blocks = N >> L;
+    return {LeafStep::QUAD_ROW, L, blocks, (unsigned)std::max(64, 4 << L), blocks == 1 ? 0 : blocks};
+  }
+  // (a tree of one such block would end here, and this launch does not hand roots over)
+  if (quads && N > ((size_t)1 << B3H_LOG) && N * count <= ((size_t)1 << (words >= 48 ? 21 : 18)))
+    return {LeafStep::LANE_ROW, B3H_LOG, N >> B3H_LOG, 1u << B3H_LOG, N >> B3H_LOG};
+  return {N >= 256 ? LeafStep::WAVE : LeafStep::LANE_FOUR, 2, (N / 4 + TREE_THREADS - 1) / TREE_THREADS, TREE_THREADS,
+          N / 4};
+}
+
 }  // namespace whir
