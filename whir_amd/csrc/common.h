@@ -95,7 +95,9 @@ void mailbox_arm(hipStream_t s);
 // launch after which nothing the host will read is still to be written may take it.
 MailboxSig mailbox_take(const void* out);
 #if defined(__HIP__)
-// Device side, by the one thread that stored the result (after its stores).
+// Device side, by the one thread that stored the result (after its stores), or whose wave
+// did.  Where other waves of the block stored some of it, every thread fences
+// (__threadfence_system) before the barrier that precedes this.
 __device__ inline void mailbox_raise(const MailboxSig& sig) {
   if (sig.flag) {
     __threadfence_system();

@@ -239,11 +239,14 @@ struct MoveArgs {
   MoveSeg seg[MOVE_SEGS];
   int n;
 };
-// A few KB at most: one block, so that it can raise the flag after its last store.
+// A few KB at most: one block, so that it can raise the flag after its last store.  Every
+// wave waits for its own stores before the barrier: neither the barrier nor thread 0's fence
+// waits for another wave's.
 __global__ __launch_bounds__(256) void k_move(MoveArgs a, MailboxSig sig) {
   for (int k = 0; k < a.n; k++)
     for (size_t i = threadIdx.x; i < a.seg[k].words; i += blockDim.x) a.seg[k].dst[i] = a.seg[k].src[i];
   if (sig.flag) {
+    __threadfence_system();
     __syncthreads();
     if (threadIdx.x == 0) mailbox_raise(sig);
   }
