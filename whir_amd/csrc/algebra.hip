@@ -410,6 +410,9 @@ __global__ __launch_bounds__(1024) void k_fold_poly(const uint64_t* a_in, uint64
     st<D>(b, t, y);
     gl::emul_acc<D>(acc, pair_factor<D>(x), pair_factor<D>(y));
   }
+  // A caller that has seen the flag may read the folded vectors on another stream: every
+  // wave's stores are complete before it rises.
+  if (sig.flag) __threadfence_system();
   Ext<D> v[1] = {gl::ext_reduce<D>(acc)};
   __shared__ uint64_t tot[2 * D];
   block_role_sum<D, 1, 2>(v, tot);
