@@ -692,9 +692,10 @@ static NttSched default_sched(int D, int logC, uint64_t words) {
   // of 2^4 Fp elements and 16 of 2^18 Fp3 ones measured slower (1.0-2.6x faster, MI355X),
   // but for extension codewords of 2^22 words and more over 2^11 elements: there the one
   // butterfly pass beats a column step and rows (Fp2 2^22 words 38.6 against 40.1 us, 2^24
-  // 118.8 against 132; at 2^19 15.8 against 12.0).
+  // 118.8 against 132; at 2^19 15.8 against 12.0).  Of 2^11 elements, base codewords above 2 GiB
+  // stay on the one pass too: it needs no intermediate codeword beside the output.
   int c1 = 0;
-  s.mx = mx_split(logC, &c1) && !(logC == 11 && D > 1 && words >= (1ull << 22));
+  s.mx = mx_split(logC, &c1) && !(logC == 11 && words > (D > 1 ? (1ull << 22) - 1 : 1ull << 28));
   return s;
 }
 
@@ -1071,13 +1072,15 @@ void rs_prepare(int D, uint64_t N, int logC, uint64_t M, hipStream_t st) {
 size_t rs_scratch_words(int D, uint64_t M, uint64_t N, uint64_t C) {
   int logC = log2_exact(C);
   // a matrix-core encode of 2^11 elements is a column step and rows, too
-  return logC >= MAX_PASS_LOG ? (size_t)M * N * D : 0;
+  return logC > MAX_PASS_LOG || (logC == MAX_PASS_LOG && default_sched(D, logC, M * N * D).mx) ? (size_t)M * N * D : 0;
 }
 
 void rs_encode_cols(int D, RsArgs a, uint64_t* scratch, hipStream_t st) {
   WHIR_REQUIRE(a.M > 0, "rs_encode: no messages");
   WHIR_REQUIRE(log2_exact(a.N) >= 0, "rs_encode: the device path needs a power-of-two codeword length");
   WHIR_REQUIRE(((a.N >> a.logC) << a.logC) == a.N, "rs_encode: coset size must divide the codeword length");
+  WHIR_REQUIRE(scratch || !rs_scratch_words(D, a.M, a.N, 1ull << a.logC) || (a.L == 1 && a.mask_len == 0),
+               "rs_encode: no room for the first pass's output");
   switch (D) {
     case 1: launch<1>(a, scratch, st); break;
     case 2: launch<2>(a, scratch, st); break;
