@@ -219,7 +219,8 @@ struct HostStage {
 };
 static uint64_t* host_stage() {
   thread_local HostStage st;
-  if (!st.p) WHIR_HIP(hipHostMalloc((void**)&st.p, HOST_STAGE_WORDS * 8, hipHostMallocDefault));
+  // coherent, like the mailbox: a kernel that writes it raises the host's flag itself
+  if (!st.p) WHIR_HIP(hipHostMalloc((void**)&st.p, HOST_STAGE_WORDS * 8, hipHostMallocCoherent));
   return st.p;
 }
 

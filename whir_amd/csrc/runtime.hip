@@ -205,7 +205,8 @@ const void* stage_async(const void* src, size_t bytes, hipStream_t s) {
     if (st.host) (void)hipHostFree(st.host);
     if (st.wrap) (void)hipEventDestroy(st.wrap);
     st.cap = (size_t)8 << 20;
-    WHIR_HIP(hipHostMalloc((void**)&st.host, st.cap, hipHostMallocDefault));
+    // coherent: kernels read it in place, and the same words again after a wrap
+    WHIR_HIP(hipHostMalloc((void**)&st.host, st.cap, hipHostMallocCoherent));
     WHIR_HIP(hipEventCreateWithFlags(&st.wrap, hipEventDisableTiming));
     st.off = 0;
     st.device = dev;
