@@ -360,7 +360,7 @@ __global__ __launch_bounds__(MERKLE_THREADS) void k_merkle_sub(uint8_t* __restri
 }
 
 // ------------------------------------------------------------------ BLAKE3, quad-split
-// Below 2^16 nodes a Merkle level holds less than one wave per SIMD, so each level
+// Below 2^16 nodes a Merkle level holds less than one wave per SIMD (a lane per node), so each level
 // costs the latency of one wave running a whole compression.  Here the four lanes of a
 // quad share one compression: lane q holds column q of the state (v[q], v[4+q],
 // v[8+q], v[12+q]) and runs that column's G; for the diagonal step rows 1-3 rotate by

@@ -22,15 +22,18 @@
 // DFT costs 12 (digits, recombination) and a twiddle 19, and the matrix cores, idle until
 // now, take the additions: 71 VALU instructions per element for a 2^8-point pass 2, 98 for
 // a 2^10-point one.  Measured on MI355X, 16 messages, two passes, before -> after:
-//     Fp  2^20 -> 2^22: 603 + 432 -> 351 + 314 us    Fp  2^18 -> 2^22: 548 + 366 -> 295 + 254 us
-//     Fp2 2^16 -> 2^21: 393 + 289 -> 280 + 247 us    Fp3 2^18 -> 2^21: 834 + 619 -> 470 + 505 us
-//     Fp2 2^12 -> 2^20: 284 -> 204 us                Fp3 2^14 -> 2^17: 79 -> 59 us
-//     one pass, Fp2 2^8 -> 2^19: 98 -> 62 us         Fp3 2^10 -> 2^19: 264 -> 112 us
-//     small, Fp 2^10 -> 2^11: 15.5 -> 7.3 us         Fp2 2^12 -> 2^13: 21.2 -> 12.8 us
-// Pass 2 of 2^8 and 2^9 points moves 1.07 GB in 240-250 us, 4.4 TB/s where a large copy
-// reaches 4.7: it is at the memory's rate.  Pass 1 and the 2^10-point pass 2 are bound by
-// VALU issue with four waves per SIMD; 128 registers a lane, 64 of them the matrix, allow
-// no more waves.  Measured slower: 12 waves per CU with the next tile's loads in flight in
+//     Fp  2^20 -> 2^22: 603 + 432 -> 359 + 312 us    Fp  2^18 -> 2^22: 548 + 366 -> 297 + 253 us
+//     Fp2 2^16 -> 2^21: 393 + 289 -> 282 + 246 us    Fp3 2^18 -> 2^21: 834 + 619 -> 446 + 418 us (in groups)
+//     Fp2 2^12 -> 2^20: 284 -> 210 us                Fp3 2^14 -> 2^17: 79 -> 54 us
+//     one pass, Fp2 2^8 -> 2^19: 98 -> 60 us         Fp3 2^10 -> 2^19: 264 -> 104 us
+//     small, Fp 2^10 -> 2^11: 15.5 -> 7.2 us         Fp2 2^12 -> 2^13: 21.2 -> 12.9 us
+// Pass 2 of 2^8 and 2^9 points moves 1.07 GB in 245-253 us, 4.3 TB/s where a large copy
+// reaches 4.7: it is near the memory's rate, and its waves wait 52-60% of their time.  Pass 1
+// waits 45-47% and issues 0.87-1.0 VALU instructions per SIMD and four cycles (half of them
+// half-rate 64-bit ones, whose mix allows about 1.3) with the matrix cores busy 10-28% of the
+// time: VALU issue and the latency of four waves per SIMD together.  128 registers a lane, 64
+// of them the matrix, allow no more waves; the 2^10-point pass 2 is between the two (0.68,
+// waits 51%).  Measured slower: 12 waves per CU with the next tile's loads in flight in
 // registers (pass 2 234 -> 317 us, the late tiles leave waves idle), one block of 16 waves
 // per CU, the matrices of a whole 32-point DFT in registers (8 waves per CU, 1.2x slower).
 #include "common.h"
@@ -52,12 +55,6 @@ constexpr uint32_t K0W = 0x80808080u;  // both halves of K0 = 128 (1 + 2^8 + ...
 constexpr int MAT16 = 1026;            // where the 16-point matrix starts, after the eight-point ones
 constexpr int TILE = 8192;             // words of one LDS tile (64 KiB)
 
-#ifndef T3
-#define T3 384
-#endif
-#ifndef RES
-#define RES 2
-#endif
 #define DEV __device__ __forceinline__
 // Keeps the scheduler from interleaving the eight-point transforms of a step, which would
 // need more registers than four waves per SIMD leave.

@@ -313,8 +313,7 @@ void irs_commit(Transcript& t, const IrsCfg& c, int engine, const uint64_t* cons
   } else if (nood) {
     // All samples of all vectors in shared passes, written to the mailbox (vector b at
     // words [b*nood*D, (b+1)*nood*D)); sent point-major.
-    const size_t pad = (nood + 3) / 4 * 4;
-    WHIR_REQUIRE(nvec * pad * D <= RESULT_MAILBOX_WORDS, "too many out-of-domain samples");
+    WHIR_REQUIRE(nvec * nood * D <= RESULT_MAILBOX_WORDS, "too many out-of-domain samples");
     mailbox_arm(s);
     univariate_eval_many_dev(Ds, D, vecs, nvec, c.vector_size, w.ood_points.data(), nood, mbox, s);
     mailbox_wait(s);
@@ -650,12 +649,6 @@ std::vector<E<D>> sumcheck_prove_pairs(Transcript& t, const SumcheckCfg& sc, int
   return chals;
 }
 
-//
-// after_first, when given, runs once after the first synchronization (before the first
-// message is sent), or at the end when there are no rounds: a caller that queued
-// work ahead of the sumcheck (an opening's gather) reads its results there.
-//
-// view: b given as a covector view of length n (see sumcheck_prove_pairs).
 // Sumchecks over at most this many elements run on the host: both vectors come over in
 // one wait, every round's sums, challenge and fold are host arithmetic (a few hundred
 // extension products at most), and the folded vectors go back with one copy.  On the
@@ -663,14 +656,7 @@ std::vector<E<D>> sumcheck_prove_pairs(Transcript& t, const SumcheckCfg& sc, int
 // round trip per one or two rounds.
 constexpr size_t HOST_SUMCHECK_MAX = 64;
 
-// sumcheck::Config::prove on the host for short vectors (a and b of length n in device
-// memory, extension elements): the same messages, challenges and folds as the device
-// rounds (x'_i = x_i + r (x_(h+i) - x_i), c0 = sum x_i y_i, c2 = sum dx_i dy_i over
-// i < h = n/2).
-//
-// keep: the vectors stay on the host instead (keep->x, keep->y) for a caller whose next
-// step works there, and the device copies are then out of date; vectors that are there
-// already are taken from it.
+// Both vectors of a sumcheck kept on the host.
 template <int D>
 struct HostPair {
   std::vector<E<D>> x, y;  // empty: the device holds the vectors
@@ -689,6 +675,14 @@ void host_pair_store(const std::vector<E<D>>& x, const std::vector<E<D>>& y, uin
   move_words(segs, 2, s, false);
 }
 
+// sumcheck::Config::prove on the host for short vectors (a and b of length n in device
+// memory, extension elements): the same messages, challenges and folds as the device
+// rounds (x'_i = x_i + r (x_(h+i) - x_i), c0 = sum x_i y_i, c2 = sum dx_i dy_i over
+// i < h = n/2).
+//
+// keep: the vectors stay on the host instead (keep->x, keep->y) for a caller whose next
+// step works there, and the device copies are then out of date; vectors that are there
+// already are taken from it.
 template <int D>
 std::vector<E<D>> sumcheck_prove_host(Transcript& t, const SumcheckCfg& sc, int engine, uint64_t* a, uint64_t* b,
                                       size_t& n, E<D>& sum, hipStream_t s, const std::function<void()>& after_first,
@@ -746,6 +740,13 @@ std::vector<E<D>> sumcheck_prove_host(Transcript& t, const SumcheckCfg& sc, int 
   return chals;
 }
 
+// sumcheck::Config::prove over a (a_src before its first fold) and b.
+//
+// after_first, when given, runs once after the first synchronization (before the first
+// message is sent), or at the end when there are no rounds: a caller that queued
+// work ahead of the sumcheck (an opening's gather) reads its results there.
+//
+// view: b given as a covector view of length n (see sumcheck_prove_pairs).  keep: see sumcheck_prove_host.
 template <int D>
 std::vector<E<D>> sumcheck_prove(Transcript& t, const SumcheckCfg& sc, int engine, const uint64_t* a_src, int a_Ds,
                                  uint64_t* a, uint64_t* b, size_t& n, E<D>& sum, hipStream_t s,
@@ -1123,8 +1124,7 @@ void prove_impl(const WhirCfg& cfg, Transcript& t, const uint64_t* const* vecs, 
   const size_t nood = opts.size() / D;
   std::vector<uint64_t> cross;  // cross[(j*nood + o)*D]: vector j at OOD point o
   if (W > 1 && nood) {
-    const size_t pad = (nood + 3) / 4 * 4;
-    WHIR_REQUIRE(V * pad * D <= RESULT_MAILBOX_WORDS, "too many out-of-domain cross terms");
+    WHIR_REQUIRE(V * nood * D <= RESULT_MAILBOX_WORDS, "too many out-of-domain cross terms");
     mailbox_arm(s);
     univariate_eval_many_dev(1, D, vecs, V, n, opts.data(), nood, mbox, s);
     mailbox_wait(s);
