@@ -22,8 +22,8 @@ def check(nv, D, engine, k0, k, lir, npts, sec):
     assert np.array_equal(gep, np.concatenate(ep))
 
 
-# STIR terms over 2^8 .. 2^13 elements (one row per block, the queries dealt to four groups;
-# counts that leave groups of different lengths) and over 2^19 (four rows, two groups).
+# STIR terms over 2^8 .. 2^13 elements (most of them in one launch; 2^13 with 233 points has one
+# row per block and the queries dealt to four groups) and over 2^19 (four rows, two groups).
 @pytest.mark.parametrize("nv,D,lir,sec", [(12, 2, 1, 100), (12, 1, 1, 60), (12, 3, 1, 100), (13, 2, 2, 80),
                                           (13, 3, 1, 41), (14, 1, 2, 60), (15, 2, 1, 37), (16, 3, 1, 100),
                                           (17, 2, 1, 100), (23, 2, 1, 40)])
@@ -32,7 +32,8 @@ def test_stir_terms_over_short_and_long_vectors(nv, D, lir, sec):
 
 
 # STIR terms in one launch and the sizes beside it: 16 to 256 lanes a block, one and several
-# blocks, vectors shorter than a block, point counts on both sides of the rule.
+# blocks, vectors shorter than a block, point counts on both sides of the rule.  The longest
+# first rounds (2^10 with 300 points, 2^14 with 259, 2^16, 2^17) go to the four groups, each degree.
 @pytest.mark.parametrize("nv,D,k,lir,sec", [(6, 2, 2, 1, 32), (7, 1, 3, 1, 32), (8, 3, 3, 2, 80), (11, 2, 1, 1, 100),
                                             (14, 2, 4, 1, 128), (16, 3, 4, 1, 100), (17, 2, 4, 1, 100),
                                             (18, 2, 4, 3, 60), (18, 2, 4, 1, 110), (20, 3, 4, 2, 60), (20, 1, 3, 1, 40)])
@@ -50,7 +51,7 @@ def test_sumcheck_pairs(nv, D, k0, k):
     check(nv, D, W.HASH_BLAKE3, k0, k, 1, 2, 40 if D == 1 else 80)
 
 
-# Univariate evaluation: one block of 64 to 1024 threads, several blocks of 1024 elements, and
+# Univariate evaluation: one block of 64 to 256 threads, several blocks of 1024 elements, and
 # segments of 2048 in several turns; lengths at and beside the edges.
 @pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 255, 256, 257, 1000, 1024, 4095, 4096, 4097, 5121, 2**15 + 1,
                                2**20, 2**20 + 1, 2**22 + 2049])
