@@ -338,7 +338,7 @@ def main():
         "serving": serving,
         "kernels": kernels,
         "ntt_schedules": [{k: e[k] for k in ("degree", "log_n", "log_c", "messages", "log_c1", "pass1", "pass2",
-                                             "tuned_ms", "default_ms")} for e in W.ntt_schedules()],
+                                             "matrix_cores", "tuned_ms", "default_ms")} for e in W.ntt_schedules()],
     }
     print(json.dumps(line))
 
