@@ -28,9 +28,9 @@
 //     one pass, Fp2 2^8 -> 2^19: 98 -> 60 us         Fp3 2^10 -> 2^19: 264 -> 104 us
 //     small, Fp 2^10 -> 2^11: 15.5 -> 7.2 us         Fp2 2^12 -> 2^13: 21.2 -> 12.9 us
 // Pass 2 of 2^8 and 2^9 points moves 1.07 GB in 245-253 us, 4.3 TB/s where a large copy
-// reaches 4.7: it is near the memory's rate, and its waves wait 52-60% of their time.  Pass 1
-// waits 45-47% and issues 0.87-1.0 VALU instructions per SIMD and four cycles (half of them
-// half-rate 64-bit ones, whose mix allows about 1.3) with the matrix cores busy 10-28% of the
+// reaches 4.7: it is near the memory's rate, and its waves wait 52-64% of their time.  Pass 1
+// waits 45-50% and issues 0.87-1.0 VALU instructions per SIMD and four cycles (half of them
+// half-rate 64-bit ones, whose mix allows about 1.3) with the matrix cores busy 10-27% of the
 // time: VALU issue and the latency of four waves per SIMD together.  128 registers a lane, 64
 // of them the matrix, allow no more waves; the 2^10-point pass 2 is between the two (0.68,
 // waits 51%).  Measured slower: 12 waves per CU with the next tile's loads in flight in
