@@ -228,7 +228,6 @@ void gather_hashes_dev(const uint8_t* nodes, const uint64_t* idx, size_t k, uint
   WHIR_HIP(hipGetLastError());
 }
 
-
 // 64-byte node pair (two 8-word digests) as a hash input.
 struct PairReader {
   const uint32_t* l;
@@ -505,6 +504,7 @@ static bool b3q_enabled() {
   }();
   return on;
 }
+
 // Three Merkle levels above a level of width w (w % 2^11 == 0): lane g reduces nodes
 // 8g..8g+7 to one in registers and stores the seven nodes it makes.  No lane idles
 // and nothing waits at a barrier, which matters on levels wide enough to keep every
